@@ -148,11 +148,6 @@ __device__ __forceinline__ u32x4 add_bf16x8(const u32x4& a, const u32x4& b) {
   return r;
 }
 
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, (int)bytes,
-                                           0x00020000);
-}
-
 constexpr uint32_t kOOB = 0x80000000u;  // offset that always reads as zero
 
 typedef __attribute__((address_space(3))) void lds_void_t;

@@ -1,12 +1,12 @@
-// fp32 grouped GEMMs of the expert layer on gfx950 MFMA (v_mfma_f32_32x32x2_f32).
+// fp32 grouped GEMMs of the expert layer on gfx950, on the bf16 matrix cores
+// with fp32 precision (three-term split, v_mfma_f32_32x32x16_bf16).
 //
 // The fp32 configurations of the reference (its CPU-runnable XS standard
 // layer) run the experts in fp32: F.grouped_mm on fp32 operands with fp32
 // accumulation and no intermediate rounding (transformers/integrations/
 // moe.py:439-459 forward, :226-242 backward formulas).  This file is that
 // path: the same six GEMMs as the bf16 kernels, unfused backward (the
-// combine backward and the gather backward run as their own kernels), every
-// product and sum in fp32.
+// combine backward and the gather backward run as their own kernels).
 //
 //   mode  C [rows x cols]          rows (operand)                 cols (operand)              k
 //   F1    gate_up -> act           routed rows (x gathered, kc)   [gate 64 | up 64] (W1, kc)  H
@@ -19,26 +19,51 @@
 // (kc: the operand's k index is contiguous in memory; km: its feature index
 // is, k strides by rows.)
 //
+// Products: the fp32 MFMA peaks at 157 TFLOP/s, the bf16 MFMA at 2500, so an
+// fp32 product made of six bf16 ones has 2.6 times the room.  Every operand
+// value is split into three bf16 terms x = hi + mid + lo (each the
+// round-to-nearest of what is left: 8 bits plus a sign per term, so the sum
+// is exact for every finite x whose terms do not underflow), and a product is
+// summed as hi*hi + hi*mid + mid*hi + hi*lo + lo*hi + mid*mid in the fp32
+// accumulators; the three products left out are at most 2^-25 of |x*y|
+// together, below the fp32 rounding of one addition.  The bf16 products are
+// exact, and one MFMA sums 16 of them per accumulator rounding where the fp32
+// MFMA sums 2: the XS layer's outputs are 0.9e-6 from the 64-bit ones
+// (2-norm) and its weight gradients 1.0e-6, against 1.0e-6 and 1.2e-6 with
+// the fp32 MFMA.  A value
+// that is not finite, or overflows as bf16, makes every element it touches
+// non-finite here; a workgroup that finds such an element in its tile
+// computes the tile again with the fp32 MFMA (v_mfma_f32_32x32x2_f32), whose
+// infinities and NaNs are the plain fp32 ones.
+//
 // Workgroup: 256 threads = 4 waves as 2 x 2, a 128 x 128 tile of C, each wave
 // a 64 x 64 block of 2 x 2 MFMA sub-tiles (64 fp32 accumulators per lane).
 // A k-stage is 32 deep: both operands are loaded global -> registers (16
-// bytes per load, coalesced along the contiguous index) and written to LDS
-// as [feature][k] rows of 36 floats (144 bytes: the 16-byte fragment reads of
-// eight consecutive features hit distinct banks); km operands are transposed
-// on the way in.  Two stage buffers: the loads of stage s+1 are in flight
-// while stage s is multiplied.  MFMA 32x32x2: lane L supplies feature L % 32
-// at k' = L / 32 of each operand; a lane reads 4 consecutive k of its
-// feature (k = 8kk + 4(L/32) + s, s = 0..3) with one ds_read_b128 and feeds
-// them to four MFMAs, so the k pairs (8kk + s, 8kk + 4 + s) of one call are
-// a permutation of the stage's k range.  Output: register 4q+c of a lane
+// bytes per load, coalesced along the contiguous index), split in registers
+// and written to LDS as three bf16 planes of [feature][32 k] (64-byte rows,
+// lds_at()'s swizzle makes the fragment reads and both operands' writes
+// bank-conflict free); the loads of stage s+1 are in flight while stage s is
+// multiplied.  One stage buffer of 48 KB, so that three workgroups share a
+// CU: one splits while the others multiply (two per CU: F1 662, FDX1 667 us).
+// Per stage a wave issues 48 MFMAs (1536 cycles) and about 250 VALU
+// instructions (1000 cycles, mostly the split); the matrix cores are busy 60%
+// of the cycles at 1.83 GHz.  Kernel times at S = 32768 rows, H = 1024, E =
+// 16, I = 768, with the fp32 MFMA -> with the split: F1 935 -> 626, F2 485 ->
+// 304, FDX2 658 -> 368, FDX1 1214 -> 573, FDW2 790 -> 290, FDW1 1453 -> 624 us
+// (84, 106, 78, 85, 65, 71 -> 165, 170, 140, 180, 178, 165 TFLOP/s).  Output: register 4q+c of a lane
 // holds (tile row L % 32, tile column 8q + 4(L/32) + c) of the sub-tile (the
-// column operand is MFMA's "A").  Epilogue: the tile is staged in LDS
-// (reusing the stage buffers) and written out row by row with 16-byte lanes,
-// applying the SwiGLU / dSwiGLU tail in fp32.
+// column operand is MFMA's "A").  Epilogue: 64 rows at a time are staged in
+// LDS (reusing the stage buffer) and written out row by row with 16-byte
+// lanes, applying the SwiGLU / dSwiGLU tail in fp32.
 //
 // Token-grouped tiles come from the permutation's row-tile table for 128-row
 // tiles ({expert, first row, end row} per tile, device-side); dW tiles are
-// (expert, row tile, column tile), their k range the expert's rows.
+// (expert, row tile, column tile), their k range the expert's rows.  Each XCD
+// takes a contiguous eighth of the tiles, so its L2 holds the rows and the
+// weights that neighbouring tiles share.
+#include <cmath>
+#include <type_traits>
+
 #include "common.h"
 #include "gemm_f32.h"
 
@@ -48,13 +73,15 @@ namespace {
 constexpr int FBM = 128;          // tile rows
 constexpr int FBN = 128;          // tile columns
 constexpr int FBK = 32;           // k per stage
-constexpr int FLD = FBK + 4;      // floats per feature row of a stage in LDS
+constexpr int FLD = FBK + 4;      // floats per feature row of an fp32 stage in LDS
 constexpr int FSTG = FBN + 4;     // floats per row of the epilogue staging tile
 constexpr int FNT = 256;          // threads per workgroup
 constexpr int FTILE_TABLE = 1;    // the permutation's 128-row tile table
-constexpr size_t kStageFloats = (size_t)(FBM + FBN) * FLD;
-constexpr size_t kLdsBytes =
-    (2 * kStageFloats > (size_t)FBM * FSTG ? 2 * kStageFloats : (size_t)FBM * FSTG) * sizeof(float);
+constexpr int kPlane = FBM * FBK * 2;          // bytes of one split plane of one operand
+constexpr int kOperand = 3 * kPlane;           // ... of the three planes of one operand
+constexpr size_t kLdsBytes = 2 * kOperand;
+static_assert((size_t)(FBM + FBN) * FLD * 4 <= kLdsBytes, "fp32 stage fits");
+static_assert((size_t)(FBM / 2) * FSTG * 4 <= kLdsBytes, "staging fits");
 
 enum FMode { F1 = 0, F2 = 1, FDX2 = 2, FDX1 = 3, FDW2 = 4, FDW1 = 5 };
 
@@ -72,16 +99,38 @@ struct FArgs {
   int64_t T, S;
   int E, H, I, topk;
   int n_ct, n_rt;         // column tiles; dW modes: row tiles per expert
+  int n_tiles;            // dW modes: E * n_rt * n_ct
+  uint32_t tok_mul;       // n / topk == (n * tok_mul) >> tok_shift for 0 <= n < 2^31
+  int tok_shift;
 };
 
 __device__ __forceinline__ f32x4 ld4(const float* p) { return *(const f32x4*)p; }
 
+// Byte offset of (feature f, 16-byte chunk c of its 32 k) in a split plane:
+// 64-byte rows, four to the 256 bytes that the LDS banks span.  The chunk is
+// XORed with the row's place among 16 so that 16 lanes reading one chunk of
+// 16 consecutive features cover all banks; the row's low bits are XORed with
+// f >> 4 so that the lanes writing features 4l + j (a k-major operand) do too.
+__device__ __forceinline__ uint32_t lds_at(int f, int c) {
+  return (uint32_t)((f ^ ((f >> 4) & 3)) * 64 + ((c ^ ((f >> 2) & 3)) << 4));
+}
+
+// Two fp32 values -> their three bf16 terms, packed in pairs.
+__device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& hi, uint32_t& mid,
+                                           uint32_t& lo) {
+  hi = pack_bf2(x0, x1);
+  const float r0 = x0 - bf_lo(hi), r1 = x1 - bf_hi(hi);
+  mid = pack_bf2(r0, r1);
+  lo = pack_bf2(r0 - bf_lo(mid), r1 - bf_hi(mid));
+}
+
 template <int MODE>
-__global__ __launch_bounds__(FNT) void f32_gemm_kernel(FArgs p) {
+__global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
   constexpr bool TOKEN = MODE == F1 || MODE == F2 || MODE == FDX2 || MODE == FDX1;
   constexpr bool COL_KM = MODE != F1 && MODE != F2;
   constexpr bool ROW_KM = MODE == FDW2 || MODE == FDW1;
   extern __shared__ __attribute__((aligned(16))) float fsm[];
+  char* const planes = (char*)fsm;  // row operand's hi, mid, lo planes, then the column operand's
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -90,19 +139,23 @@ __global__ __launch_bounds__(FNT) void f32_gemm_kernel(FArgs p) {
   const int H = p.H, I = p.I, I2 = 2 * p.I;
 
   // ------------------------------------------------------------ the tile
+  // XCD b % 8 (workgroups are dealt round-robin) walks a contiguous eighth.
   int e, row0 = 0, row_end = 0, ct, rt = 0, kbeg = 0, kend = 0;
+  const int n_tiles = TOKEN ? *p.tile_count * p.n_ct : p.n_tiles;
+  const int per_xcd = (n_tiles + 7) >> 3;
+  const int tile = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+  if ((int)(blockIdx.x >> 3) >= per_xcd || tile >= n_tiles) return;
   if constexpr (TOKEN) {
-    const int rtile = (int)(blockIdx.x / (unsigned)p.n_ct);
-    ct = (int)(blockIdx.x % (unsigned)p.n_ct);
-    if (rtile >= *p.tile_count) return;
+    const int rtile = tile / p.n_ct;
+    ct = tile % p.n_ct;
     const int4 ti = p.tile_info[rtile];
     e = ti.x;
     row0 = ti.y;
     row_end = ti.z;
   } else {
     const int per_e = p.n_rt * p.n_ct;
-    e = (int)(blockIdx.x / (unsigned)per_e);
-    const int rem = (int)(blockIdx.x % (unsigned)per_e);
+    e = tile / per_e;
+    const int rem = tile % per_e;
     rt = rem / p.n_ct;
     ct = rem % p.n_ct;
     kbeg = p.offsets[e];
@@ -117,248 +170,361 @@ __global__ __launch_bounds__(FNT) void f32_gemm_kernel(FArgs p) {
 
   // ------------------------------------------------------ operand loads
   // kc operand: thread t loads features t/8 + 32i (i = 0..3), k 4(t%8)..+3.
-  // km operand: thread t loads k rows t/32 + 8i, features 4(t%32)..+3.
+  // km operand: a thread loads four consecutive k rows (km_k + i) of four
+  // features, so that the four k of a feature are written as one 8-byte
+  // piece per plane; lanes l and l + 8 hold the two halves of a chunk, so
+  // 16 lanes write 128 bytes of distinct banks.
   const int kc_f = tid >> 3, kc_k = (tid & 7) * 4;
-  const int km_k = tid >> 5, km_f = (tid & 31) * 4;
+  const int km_k = (wid * 2 + ((lane >> 3) & 1)) * 4;
+  const int km_f = ((lane & 7) | ((lane >> 4) << 3)) * 4;
 
-  // Row operand, per load i: base pointer of the feature row (kc) or of
-  // feature column 0 of the k range (km), and a validity mask.
-  const float* rbase[4];
-  bool rok[4];
-  int64_t rld = 0;  // km: floats between k rows
+  auto div_topk = [&](int n) {  // row_src / topk by multiply-shift
+    return (int)(((uint64_t)(uint32_t)n * p.tok_mul) >> p.tok_shift);
+  };
+  // Operands are read through buffer descriptors rebased to each stage in
+  // scalar registers (64-bit base, extent capped at 4 GB), so that a lane
+  // keeps 32-bit offsets only and reads past an operand return zero: the
+  // ragged k range of the dW modes.  Rows past a token tile's end and weight
+  // rows past H repeat the last one, and features of a km operand past its
+  // width read what lies there: all of that only reaches elements of C that
+  // are not stored.  Gathered token rows (F1's rows, FDW1's columns) keep
+  // 64-bit addresses, since hidden_states may hold more than 4 GB.
+  const int l_end = TOKEN ? min(row_end - row0, FBM) - 1 : 0;  // last row of the tile
+  const char* rptr = nullptr;
+  const char* cptr = nullptr;
+  const char* cptr2 = nullptr;  // F1: the up rows
+  uint64_t rleft = 0, cleft = 0;
+  uint32_t rstep = FBK * 4, cstep = FBK * 4;
+  uint32_t roff[4], coff[4];
+  const float* xrow[4];
+  if constexpr (MODE == F1) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (MODE == F1) {
-      const int r = row0 + kc_f + 32 * i;
-      rok[i] = r < row_end;
-      const int tok = rok[i] ? p.row_src[r] / p.topk : 0;
-      rbase[i] = p.x + (int64_t)tok * H;
-    } else if constexpr (TOKEN) {
-      const int ld = MODE == F2 ? I : (MODE == FDX2 ? H : I2);
-      const int r = row0 + kc_f + 32 * i;
-      rok[i] = r < row_end;
-      rbase[i] = p.a0 + (int64_t)(rok[i] ? r : row0) * ld;
-    } else {
-      const int nf = MODE == FDW2 ? H : I2;  // features of the row operand
-      const int f = rt * FBM + km_f;
-      rok[i] = f < nf;
-      rld = nf;
-      rbase[i] = p.a0 + (int64_t)kbeg * nf + (rok[i] ? f : 0);
-    }
-  }
-  // Column operand.
-  const float* cbase[4];
-  bool cok[4];
-  int64_t cld = 0;
+    for (int i = 0; i < 4; ++i)
+      xrow[i] = p.x + (int64_t)div_topk(p.row_src[row0 + min(kc_f + 32 * i, l_end)]) * H + kc_k;
+  } else if constexpr (TOKEN) {
+    const int ld = MODE == F2 ? I : (MODE == FDX2 ? H : I2);
+    rptr = (const char*)(p.a0 + (int64_t)row0 * ld);
+    rleft = (uint64_t)(l_end + 1) * ld * 4;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if constexpr (MODE == F1) {
-      const int c = kc_f + 32 * i;  // tile column: gate features 0..63, up features 64..127
-      const int feat = ct * 64 + (c & 63);
-      cok[i] = feat < I;
-      const int wrow = (c < 64 ? 0 : I) + (cok[i] ? feat : 0);
-      cbase[i] = p.w + ((int64_t)e * I2 + wrow) * H;
-    } else if constexpr (MODE == F2) {
-      const int h = ct * FBN + kc_f + 32 * i;
-      cok[i] = h < H;
-      cbase[i] = p.w + ((int64_t)e * H + (cok[i] ? h : 0)) * I;
-    } else {
-      int nf;
-      const float* b;
-      if constexpr (MODE == FDX2) {  // down_proj[e] [H][I]: k = h, feature = i
-        nf = I;
-        b = p.w + (int64_t)e * H * I;
-        cld = I;
-      } else if constexpr (MODE == FDX1) {  // gate_up_proj[e] [2I][H]: k = j, feature = h
-        nf = H;
-        b = p.w + (int64_t)e * I2 * H;
-        cld = H;
-      } else if constexpr (MODE == FDW2) {  // act rows of e [rows][I]
-        nf = I;
-        b = p.a1 + (int64_t)kbeg * I;
-        cld = I;
-      } else {  // FDW1: hidden_states rows gathered through row_src (per stage)
-        nf = H;
-        b = p.x;
-        cld = H;
-      }
-      const int f = ct * FBN + km_f;
-      cok[i] = f < nf;
-      cbase[i] = b + (cok[i] ? f : 0);
-    }
+    for (int i = 0; i < 4; ++i)
+      roff[i] = (uint32_t)min(kc_f + 32 * i, l_end) * (uint32_t)(ld * 4) + kc_k * 4;
+  } else {
+    const int nf = MODE == FDW2 ? H : I2;  // features of the row operand
+    rptr = (const char*)(p.a0 + (int64_t)kbeg * nf + rt * FBM);
+    rleft = ((uint64_t)K_len * nf - rt * FBM) * 4;
+    rstep = (uint32_t)FBK * nf * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) roff[i] = (uint32_t)(km_k + i) * (uint32_t)(nf * 4) + km_f * 4;
   }
+  if constexpr (MODE == F1) {
+    // tile columns: gate features ct*64 .. +63, then their up features
+    cptr = (const char*)(p.w + ((int64_t)e * I2 + ct * 64) * H);
+    cptr2 = cptr + (int64_t)I * H * 4;
+    cleft = (uint64_t)64 * H * 4;  // I is a multiple of 64
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      coff[i] = (uint32_t)((kc_f + 32 * i) & 63) * (uint32_t)(H * 4) + kc_k * 4;
+  } else if constexpr (MODE == F2) {
+    cptr = (const char*)(p.w + ((int64_t)e * H + ct * FBN) * I);
+    const int last = min(H - ct * FBN, FBN) - 1;
+    cleft = (uint64_t)(last + 1) * I * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      coff[i] = (uint32_t)min(kc_f + 32 * i, last) * (uint32_t)(I * 4) + kc_k * 4;
+  } else if constexpr (MODE == FDW1) {
+    coff[0] = (uint32_t)(ct * FBN + km_f);  // hidden_states feature
+  } else {
+    // FDX2: down_proj[e] [H][I], k = h; FDX1: gate_up_proj[e] [2I][H], k = j;
+    // FDW2: act rows of e [rows][I]
+    const int nf = MODE == FDX1 ? H : I;
+    cptr = (const char*)((MODE == FDW2 ? p.a1 + (int64_t)kbeg * I
+                                       : p.w + (int64_t)e * (MODE == FDX1 ? I2 : H) * nf) +
+                         ct * FBN);
+    cleft = ((uint64_t)K_len * nf - ct * FBN) * 4;
+    cstep = (uint32_t)FBK * nf * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) coff[i] = (uint32_t)(km_k + i) * (uint32_t)(nf * 4) + km_f * 4;
+  }
+  auto stage_rsrc = [&](const char* ptr, uint64_t bytes, uint32_t step, int s) {
+    const uint64_t adv = (uint64_t)(uint32_t)s * step;
+    const uint64_t left = adv < bytes ? bytes - adv : 0ull;
+    return make_rsrc(ptr + adv, __builtin_amdgcn_readfirstlane(
+                                    (uint32_t)(left < 0xfffff000ull ? left : 0xfffff000ull)));
+  };
+  auto buf4 = [](__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0));
+  };
 
   f32x4 rv[4], cv[4];
   const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
-  auto load_stage = [&](int s) {
-    const int k0 = s * FBK;
+  // FDW1: row_src of the four k rows of the next stage to be loaded, read a
+  // stage ahead of the rows themselves.
+  int src[4];
+  auto load_src = [&](int s) {
+    if constexpr (MODE == FDW1) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      if constexpr (!ROW_KM) {
-        rv[i] = rok[i] ? ld4(rbase[i] + k0 + kc_k) : zero4;
-      } else {
-        const int k = k0 + km_k + 8 * i;
-        rv[i] = (rok[i] && k < K_len) ? ld4(rbase[i] + (int64_t)k * rld) : zero4;
-      }
-      if constexpr (!COL_KM) {
-        cv[i] = cok[i] ? ld4(cbase[i] + k0 + kc_k) : zero4;
-      } else if constexpr (MODE == FDW1) {
-        const int k = k0 + km_k + 8 * i;
-        const bool ok = cok[i] && k < K_len;
-        const int tok = ok ? p.row_src[kbeg + k] / p.topk : 0;
-        cv[i] = ok ? ld4(cbase[i] + (int64_t)tok * H) : zero4;
-      } else {
-        const int k = k0 + km_k + 8 * i;
-        cv[i] = (cok[i] && k < K_len) ? ld4(cbase[i] + (int64_t)k * cld) : zero4;
+      for (int i = 0; i < 4; ++i) {
+        const int k = s * FBK + km_k + i;
+        src[i] = k < K_len ? p.row_src[kbeg + k] : 0;
       }
     }
   };
-  // Stage buffer b: row operand [FBM][FLD] then column operand [FBN][FLD].
-  auto store_stage = [&](int b) {
-    float* R = fsm + (size_t)b * kStageFloats;
-    float* C = R + FBM * FLD;
+  auto load_stage = [&](int s) {
+    if constexpr (MODE == F1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rv[i] = ld4(xrow[i] + s * FBK);
+    } else {
+      const auto rr = stage_rsrc(rptr, rleft, rstep, s);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) rv[i] = buf4(rr, roff[i]);
+    }
+    if constexpr (MODE == FDW1) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const bool ok = (int)coff[0] < H && s * FBK + km_k + i < K_len;
+        cv[i] = ok ? ld4(p.x + (int64_t)div_topk(src[i]) * H + coff[0]) : zero4;
+      }
+      load_src(s + 1);
+    } else {
+      const auto rc = stage_rsrc(cptr, cleft, cstep, s);
+      const auto rc2 = MODE == F1 ? stage_rsrc(cptr2, cleft, cstep, s) : rc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) cv[i] = buf4(MODE == F1 && i >= 2 ? rc2 : rc, coff[i]);
+    }
+  };
+  // Splits a loaded operand into its three planes at `base`.
+  auto store_operand = [&](const f32x4 (&v)[4], char* base, auto km) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      if constexpr (!ROW_KM) {
-        *(f32x4*)(R + (kc_f + 32 * i) * FLD + kc_k) = rv[i];
-      } else {
+      float x[4];
+      uint32_t at;
+      if constexpr (decltype(km)::value) {  // k km_k..+3 of feature km_f + i
 #pragma unroll
-        for (int j = 0; j < 4; ++j) R[(km_f + j) * FLD + km_k + 8 * i] = rv[i][j];
-      }
-      if constexpr (!COL_KM) {
-        *(f32x4*)(C + (kc_f + 32 * i) * FLD + kc_k) = cv[i];
-      } else {
+        for (int j = 0; j < 4; ++j) x[j] = v[j][i];
+        at = lds_at(km_f + i, km_k >> 3) + ((km_k >> 2) & 1) * 8;
+      } else {  // k kc_k..+3 of feature kc_f + 32 i
 #pragma unroll
-        for (int j = 0; j < 4; ++j) C[(km_f + j) * FLD + km_k + 8 * i] = cv[i][j];
+        for (int j = 0; j < 4; ++j) x[j] = v[i][j];
+        at = lds_at(kc_f + 32 * i, kc_k >> 3) + ((kc_k >> 2) & 1) * 8;
       }
+      u32x2 hi, mid, lo;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint32_t a, b, c;
+        split_pair(x[2 * h], x[2 * h + 1], a, b, c);
+        hi[h] = a;
+        mid[h] = b;
+        lo[h] = c;
+      }
+      *(u32x2*)(base + at) = hi;
+      *(u32x2*)(base + kPlane + at) = mid;
+      *(u32x2*)(base + 2 * kPlane + at) = lo;
     }
   };
 
   f32x16 acc[2][2];
+  auto zero_acc = [&]() {
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+  };
+  zero_acc();
 
   if (nk > 0) {
+    // fragment addresses of k sub-step 0 (sub-step 1: chunk ^ 2)
+    uint32_t fa[2], fb[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      fa[i] = (uint32_t)kOperand + lds_at(wc * 64 + i * 32 + l32, hl);
+      fb[i] = lds_at(wr * 64 + i * 32 + l32, hl);
+    }
+    load_src(0);
     load_stage(0);
-    store_stage(0);
-    __syncthreads();
     for (int s = 0; s < nk; ++s) {
+      store_operand(rv, planes, std::integral_constant<bool, ROW_KM>{});
+      store_operand(cv, planes + kOperand, std::integral_constant<bool, COL_KM>{});
+      __syncthreads();
       if (s + 1 < nk) load_stage(s + 1);
-      const float* R = fsm + (size_t)(s & 1) * kStageFloats;
-      const float* C = R + FBM * FLD;
 #pragma unroll
-      for (int kk = 0; kk < FBK / 8; ++kk) {
-        f32x4 a[2], b[2];
+      for (int kk = 0; kk < 2; ++kk) {
+        bf16x8 a[3][2], b[3][2];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = ld4(C + (wc * 64 + i * 32 + l32) * FLD + kk * 8 + 4 * hl);
+        for (int t = 0; t < 3; ++t)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = ld4(R + (wr * 64 + j * 32 + l32) * FLD + kk * 8 + 4 * hl);
+          for (int i = 0; i < 2; ++i) {
+            a[t][i] = *(const bf16x8*)(planes + t * kPlane + (fa[i] ^ (kk * 32)));
+            b[t][i] = *(const bf16x8*)(planes + t * kPlane + (fb[i] ^ (kk * 32)));
+          }
+        // small products first
+        constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int q = 0; q < 4; ++q)
+        for (int t = 0; t < 6; ++t)
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][q], b[j][q], acc[i][j], 0, 0, 0);
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]][i], b[TB[t]][j],
+                                                                  acc[i][j], 0, 0, 0);
       }
-      // Stage s+1 goes to the other buffer, last read in step s-1 (every
-      // wave passed the barrier after that step).
-      if (s + 1 < nk) store_stage((s + 1) & 1);
-      __syncthreads();
+      __syncthreads();  // the stage is read: the next one may be written
+    }
+    // Non-finite elements: the whole tile again on the fp32 MFMA.
+    bool bad = false;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) < INFINITY);
+    if (__syncthreads_or(bad)) {
+      zero_acc();
+      float* const R = fsm;
+      float* const C = fsm + FBM * FLD;
+      load_src(0);
+      for (int s = 0; s < nk; ++s) {
+        load_stage(s);
+        __syncthreads();  // the previous stage is read
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if constexpr (!ROW_KM) {
+            *(f32x4*)(R + (kc_f + 32 * i) * FLD + kc_k) = rv[i];
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) R[(km_f + j) * FLD + km_k + i] = rv[i][j];
+          }
+          if constexpr (!COL_KM) {
+            *(f32x4*)(C + (kc_f + 32 * i) * FLD + kc_k) = cv[i];
+          } else {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) C[(km_f + j) * FLD + km_k + i] = cv[i][j];
+          }
+        }
+        __syncthreads();
+        // lane L supplies feature L % 32 at k 8kk + 4(L/32) + q, q = 0..3
+        for (int kk = 0; kk < FBK / 8; ++kk) {
+          f32x4 a[2], b[2];
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            a[i] = ld4(C + (wc * 64 + i * 32 + l32) * FLD + kk * 8 + 4 * hl);
+            b[i] = ld4(R + (wr * 64 + i * 32 + l32) * FLD + kk * 8 + 4 * hl);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+              for (int j = 0; j < 2; ++j)
+                acc[i][j] =
+                    __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][q], b[j][q], acc[i][j], 0, 0, 0);
+        }
+      }
     }
   }
 
   // ------------------------------------------------------------ epilogue
-  // The stage buffers are free (the loop ended with a barrier).
-  float* stg = fsm;  // [FBM][FSTG]
+  // Sub-tile j of both row halves at a time: staging row wr*32 + l32 is tile
+  // row wr*64 + j*32 + l32.
+  float* stg = fsm;  // [FBM / 2][FSTG]
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int j = 0; j < 2; ++j) {
+    __syncthreads();  // the stage buffer or the previous half is read
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int row = wr * 64 + j * 32 + l32;
         const int col = wc * 64 + i * 32 + 8 * q + 4 * hl;
         const f32x4 v = {acc[i][j][4 * q + 0], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
                          acc[i][j][4 * q + 3]};
-        *(f32x4*)(stg + row * FSTG + col) = v;
+        *(f32x4*)(stg + (wr * 32 + l32) * FSTG + col) = v;
       }
-  __syncthreads();
-
-  if constexpr (MODE == F1) {
-    // act = silu(gate) * up, silu(g) = g / (1 + exp(-g)) as torch evaluates it
-    const int f4 = (tid & 15) * 4;
-    const int feat = ct * 64 + f4;
-    for (int rr = tid >> 4; rr < FBM; rr += FNT / 16) {
-      const int r = row0 + rr;
-      if (r >= row_end || feat >= I) continue;
-      const f32x4 g = ld4(stg + rr * FSTG + f4);
-      const f32x4 u = ld4(stg + rr * FSTG + 64 + f4);
-      f32x4 a;
+    __syncthreads();
+    auto tile_row = [&](int sr) { return (sr >> 5) * 64 + j * 32 + (sr & 31); };
+    if constexpr (MODE == F1) {
+      // act = silu(gate) * up, silu(g) = g / (1 + exp(-g)) as torch evaluates it
+      const int f4 = (tid & 15) * 4;
+      const int feat = ct * 64 + f4;
+      for (int sr = tid >> 4; sr < FBM / 2; sr += FNT / 16) {
+        const int r = row0 + tile_row(sr);
+        if (r >= row_end || feat >= I) continue;
+        const f32x4 g = ld4(stg + sr * FSTG + f4);
+        const f32x4 u = ld4(stg + sr * FSTG + 64 + f4);
+        f32x4 a;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) a[c] = g[c] / (1.0f + expf(-g[c])) * u[c];
-      *(f32x4*)(p.out + (int64_t)r * I + feat) = a;
-      if (p.out2) {
-        *(f32x4*)(p.out2 + (int64_t)r * I2 + feat) = g;
-        *(f32x4*)(p.out2 + (int64_t)r * I2 + I + feat) = u;
+        for (int c = 0; c < 4; ++c) a[c] = g[c] / (1.0f + expf(-g[c])) * u[c];
+        *(f32x4*)(p.out + (int64_t)r * I + feat) = a;
+        if (p.out2) {
+          *(f32x4*)(p.out2 + (int64_t)r * I2 + feat) = g;
+          *(f32x4*)(p.out2 + (int64_t)r * I2 + I + feat) = u;
+        }
       }
-    }
-  } else if constexpr (MODE == FDX2) {
-    // d_act -> d_gate = d_act * up * sigmoid(g) * (1 + g * (1 - sigmoid(g))),
-    //          d_up = d_act * silu(g)   (autograd of silu(gate) * up)
-    const int c4 = (tid & 31) * 4;
-    const int i0 = ct * FBN + c4;
-    for (int rr = tid >> 5; rr < FBM; rr += FNT / 32) {
-      const int r = row0 + rr;
-      if (r >= row_end || i0 >= I) continue;
-      const f32x4 da = ld4(stg + rr * FSTG + c4);
-      const f32x4 g = ld4(p.a1 + (int64_t)r * I2 + i0);
-      const f32x4 u = ld4(p.a1 + (int64_t)r * I2 + I + i0);
-      f32x4 dg, du;
+    } else if constexpr (MODE == FDX2) {
+      // d_act -> d_gate = d_act * up * sigmoid(g) * (1 + g * (1 - sigmoid(g))),
+      //          d_up = d_act * silu(g)   (autograd of silu(gate) * up)
+      const int c4 = (tid & 31) * 4;
+      const int i0 = ct * FBN + c4;
+      for (int sr = tid >> 5; sr < FBM / 2; sr += FNT / 32) {
+        const int r = row0 + tile_row(sr);
+        if (r >= row_end || i0 >= I) continue;
+        const f32x4 da = ld4(stg + sr * FSTG + c4);
+        const f32x4 g = ld4(p.a1 + (int64_t)r * I2 + i0);
+        const f32x4 u = ld4(p.a1 + (int64_t)r * I2 + I + i0);
+        f32x4 dg, du;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const float sg = 1.0f / (1.0f + expf(-g[c]));
-        const float sl = g[c] / (1.0f + expf(-g[c]));
-        du[c] = da[c] * sl;
-        dg[c] = da[c] * u[c] * (sg * (1.0f + g[c] * (1.0f - sg)));
+        for (int c = 0; c < 4; ++c) {
+          const float sg = 1.0f / (1.0f + expf(-g[c]));
+          const float sl = g[c] / (1.0f + expf(-g[c]));
+          du[c] = da[c] * sl;
+          dg[c] = da[c] * u[c] * (sg * (1.0f + g[c] * (1.0f - sg)));
+        }
+        *(f32x4*)(p.out + (int64_t)r * I2 + i0) = dg;
+        *(f32x4*)(p.out + (int64_t)r * I2 + I + i0) = du;
       }
-      *(f32x4*)(p.out + (int64_t)r * I2 + i0) = dg;
-      *(f32x4*)(p.out + (int64_t)r * I2 + I + i0) = du;
-    }
-  } else {
-    // Plain tile: y (F2), d_xs (FDX1), d_down_proj[e] (FDW2), d_gate_up_proj[e] (FDW1).
-    const int c4 = (tid & 31) * 4;
-    int nrows, ncols, rbeg;
-    int64_t ld;
-    float* ob;
-    if constexpr (TOKEN) {
-      nrows = row_end;
-      rbeg = row0;
-      ncols = H;
-      ld = H;
-      ob = p.out;
     } else {
-      nrows = MODE == FDW2 ? H : I2;
-      rbeg = rt * FBM;
-      ncols = MODE == FDW2 ? I : H;
-      ld = ncols;
-      ob = p.out + (int64_t)e * nrows * ncols;
-    }
-    const int col = ct * FBN + c4;
-    for (int rr = tid >> 5; rr < FBM; rr += FNT / 32) {
-      const int r = rbeg + rr;
-      if (r < nrows && col < ncols) *(f32x4*)(ob + (int64_t)r * ld + col) = ld4(stg + rr * FSTG + c4);
+      // Plain tile: y (F2), d_xs (FDX1), d_down_proj[e] (FDW2), d_gate_up_proj[e] (FDW1).
+      const int c4 = (tid & 31) * 4;
+      int nrows, ncols, rbeg;
+      int64_t ld;
+      float* ob;
+      if constexpr (TOKEN) {
+        nrows = row_end;
+        rbeg = row0;
+        ncols = H;
+        ld = H;
+        ob = p.out;
+      } else {
+        nrows = MODE == FDW2 ? H : I2;
+        rbeg = rt * FBM;
+        ncols = MODE == FDW2 ? I : H;
+        ld = ncols;
+        ob = p.out + (int64_t)e * nrows * ncols;
+      }
+      const int col = ct * FBN + c4;
+      for (int sr = tid >> 5; sr < FBM / 2; sr += FNT / 32) {
+        const int r = rbeg + tile_row(sr);
+        if (r < nrows && col < ncols)
+          *(f32x4*)(ob + (int64_t)r * ld + col) = ld4(stg + sr * FSTG + c4);
+      }
     }
   }
+}
+
+// The multiply-shift of row_src / topk (Granlund and Montgomery, "Division by
+// invariant integers using multiplication", 1994).
+void set_topk_f32(FArgs& a, int top_k) {
+  a.topk = top_k;
+  int sh = 0;
+  while ((1 << sh) < top_k) ++sh;
+  a.tok_shift = 31 + sh;
+  a.tok_mul = (uint32_t)((((uint64_t)1 << (31 + sh)) + (uint64_t)top_k - 1) / (uint64_t)top_k);
 }
 
 template <int MODE>
 int launch_f32(const FArgs& a, int64_t blocks, hipStream_t st, const char* who) {
   if (blocks <= 0) return MOE_OK;
+  blocks = (blocks + 7) / 8 * 8;  // the XCDs' eighths are rounded up
   MOE_REQUIRE(blocks < ((int64_t)1 << 31), MOE_ERR_UNSUPPORTED, "%s: too many tiles", who);
   static std::atomic<int> lds_done[64];
   hipError_t err = set_dynamic_lds_once(lds_done, (const void*)f32_gemm_kernel<MODE>, (int)kLdsBytes);
@@ -414,7 +580,7 @@ int f32_gate_up_swiglu(const float* x, const int32_t* row_src, int top_k, const 
   if (S == 0) return MOE_OK;
   FArgs a{};
   a.x = x; a.w = w1; a.row_src = row_src; a.offsets = offsets; a.out = act; a.out2 = gate_up;
-  a.T = T; a.S = S; a.E = E; a.H = H; a.I = I; a.topk = top_k;
+  a.T = T; a.S = S; a.E = E; a.H = H; a.I = I; set_topk_f32(a, top_k);
   return launch_f32_token<F1>(a, tile_plan, 64, I, st, who);
 }
 
@@ -486,6 +652,7 @@ int f32_down_dw(const float* dy, const float* act, const int32_t* offsets, int64
   a.S = S; a.E = E; a.H = H; a.I = I;
   a.n_rt = (H + FBM - 1) / FBM;
   a.n_ct = (I + FBN - 1) / FBN;
+  a.n_tiles = E * a.n_rt * a.n_ct;
   // every expert's tiles are written (zeros for an expert without rows)
   return launch_f32<FDW2>(a, (int64_t)E * a.n_rt * a.n_ct, st, who);
 }
@@ -504,9 +671,10 @@ int f32_gate_up_dw(const float* dgu, const float* x, const int32_t* row_src, int
   F32_ALIGNED(d_w1, who);
   FArgs a{};
   a.x = x; a.a0 = dgu; a.row_src = row_src; a.offsets = offsets; a.out = d_w1;
-  a.T = T; a.S = S; a.E = E; a.H = H; a.I = I; a.topk = top_k;
+  a.T = T; a.S = S; a.E = E; a.H = H; a.I = I; set_topk_f32(a, top_k);
   a.n_rt = (2 * I + FBM - 1) / FBM;
   a.n_ct = (H + FBN - 1) / FBN;
+  a.n_tiles = E * a.n_rt * a.n_ct;
   return launch_f32<FDW1>(a, (int64_t)E * a.n_rt * a.n_ct, st, who);
 }
 

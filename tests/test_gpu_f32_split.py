@@ -1,0 +1,141 @@
+"""The fp32 grouped GEMMs (bf16 matrix cores, three-term split) against fp64.
+
+Bound per element: the kernel adds 6 * ceil(K/16) MFMA results of at most 16
+exact products into an fp32 accumulator, and leaves out products worth at
+most 2^-25 of |a||b|; with every MFMA adding its 16 products and the
+accumulator with at most 17 roundings, |error| <= (17 * 6 * ceil(K/16) + 2) *
+2^-24 * sum |a||b| (first order), K the contracted length."""
+import pytest
+import torch
+
+from moe_amd import experts_forward, ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _bound(K):
+    return (17 * 6 * ((K + 15) // 16) + 2) * 2.0 ** -24
+
+
+def _plan(T, E, K, seed):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    idx = torch.rand(T, E, generator=g, device=DEV).topk(K, dim=-1).indices
+    return ops.permute(idx, E), g
+
+
+def _wide(g, *shape):
+    """N(0,1) values over 2^-12 .. 2^12, so that all three terms matter."""
+    x = torch.randn(*shape, generator=g, device=DEV)
+    return x * torch.exp2(torch.randint(-12, 13, shape, generator=g, device=DEV).float())
+
+
+def _check(got, want, mags, K):
+    assert torch.isfinite(got).all()
+    err = (got.double() - want).abs()
+    assert bool((err <= _bound(K) * mags + 1e-300).all()), float((err / mags.clamp_min(1e-300)).max())
+
+
+CASES = [
+    (1, 64, 1, 1, 64),         # one row, smallest H and I
+    (128, 64, 1, 1, 128),      # one full tile
+    (129, 320, 3, 2, 64),      # tile remainders in rows and columns
+    (777, 256, 16, 4, 192),    # ragged experts
+    (2048, 1024, 16, 4, 768),  # the XS layer
+    (40, 128, 64, 6, 320),     # tiny groups, empty experts
+]
+
+
+@pytest.mark.parametrize("T,H,E,K,I", CASES)
+def test_f32_gemms_against_fp64(T, H, E, K, I):
+    print(f"f32 split T={T} H={H} E={E} K={K} I={I}", flush=True)
+    plan, g = _plan(T, E, K, T + E)
+    S = T * K
+    tok = plan.row_src.long() // K
+    off = plan.offsets.tolist()
+    x, w1, w2 = _wide(g, T, H), _wide(g, E, 2 * I, H), _wide(g, E, H, I)
+    act, dgu, dy = _wide(g, S, I), _wide(g, S, 2 * I), _wide(g, S, H)
+    gu, _ = ops.gemm_gate_up_swiglu(x, plan, w1)
+    y = ops.gemm_down(act, plan, w2)
+    dxs = ops.gemm_gate_up_backward_dx(dgu, plan, w1)
+    dw2 = ops.gemm_down_backward_dw(dy, act, plan, w2.shape)
+    dw1 = ops.gemm_gate_up_backward_dw(dgu, x, plan, w1.shape)
+    torch.cuda.synchronize()
+    for e in range(E):
+        r = slice(off[e], off[e + 1])
+        n = off[e + 1] - off[e]
+        if n == 0:
+            assert not dw1[e].any() and not dw2[e].any()
+            continue
+        xe = x[tok[r]].double()
+        a1, a2, ac, dg, d = (t.double() for t in (w1[e], w2[e], act[r], dgu[r], dy[r]))
+        _check(gu[r], xe @ a1.T, xe.abs() @ a1.abs().T, H)
+        _check(y[r], ac @ a2.T, ac.abs() @ a2.abs().T, I)
+        _check(dxs[r], dg @ a1, dg.abs() @ a1.abs(), 2 * I)
+        _check(dw2[e], d.T @ ac, d.abs().T @ ac.abs(), n)
+        _check(dw1[e], dg.T @ xe, dg.abs().T @ xe.abs(), n)
+
+
+def test_f32_gemms_small_magnitudes():
+    """Values near 2^-112, whose third term is below the smallest normal."""
+    T, H, I = 130, 64, 256
+    plan = ops.permute(torch.zeros(T, 1, dtype=torch.int64, device=DEV), 1)
+    g = torch.Generator(device=DEV).manual_seed(6)
+    act = torch.randn(T, I, generator=g, device=DEV) * 2.0 ** -112
+    w2 = torch.randn(1, H, I, generator=g, device=DEV)
+    y = ops.gemm_down(act, plan, w2)
+    a, w = act.double(), w2[0].double()
+    _check(y, a @ w.T, a.abs() @ w.abs().T, I)
+    assert float((y.double() - a @ w.T).norm() / (a @ w.T).norm()) < 1e-6
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan"), 3.4e38])
+def test_f32_gemms_nonfinite(bad):
+    """A value that is not finite (or overflows as bf16) reaches exactly the
+    elements that the plain fp32 product gives it, with their infinities and
+    NaNs, and the rest of its tile keeps the fp32 accuracy."""
+    print(f"f32 split non-finite {bad}", flush=True)
+    T, H, I = 200, 128, 192
+    plan = ops.permute(torch.zeros(T, 1, dtype=torch.int64, device=DEV), 1)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    act = torch.randn(T, I, generator=g, device=DEV)
+    w2 = torch.randn(1, H, I, generator=g, device=DEV) * 0.25
+    act[3, 17], act[150, 0] = bad, bad
+    w2[0, 70, 5] = bad
+    w2[0, 10, 17] = 0.0  # inf * 0 = NaN at (3, 10)
+    y = ops.gemm_down(act, plan, w2)
+    torch.cuda.synchronize()
+    want = act.double() @ w2[0].double().T
+    big = want.abs() > 3.4028235677973366e38  # beyond fp32
+    fin = torch.isfinite(want) & ~big
+    assert torch.equal(torch.isnan(y), torch.isnan(want))
+    assert torch.equal(torch.isinf(y), torch.isinf(want) | big)
+    assert torch.equal(y[torch.isinf(y)] > 0, want[torch.isinf(y)] > 0)
+    mags = act.double().abs() @ w2[0].double().abs().T
+    err = (y.double() - want).abs()[fin]
+    # the fp32 MFMA that recomputes these tiles: one rounding per two products
+    assert bool((err <= max(_bound(I), I * 2.0 ** -24) * mags[fin]).all())
+
+
+def test_f32_layer_gradients_against_fp64():
+    T, H, E, K, I = 513, 192, 8, 2, 128
+    g = torch.Generator(device=DEV).manual_seed(9)
+    x = torch.randn(T, H, generator=g, device=DEV)
+    w1 = torch.randn(E, 2 * I, H, generator=g, device=DEV) * 0.1
+    w2 = torch.randn(E, H, I, generator=g, device=DEV) * 0.1
+    p, idx = torch.softmax(torch.randn(T, E, generator=g, device=DEV), -1).topk(K, dim=-1)
+    dout = torch.randn(T, H, generator=g, device=DEV)
+    leaves = [t.clone().requires_grad_(True) for t in (x, p, w1, w2)]
+    out = experts_forward(leaves[0], idx, *leaves[1:])
+    out.backward(dout)
+    l64 = [t.double().requires_grad_(True) for t in (x, p, w1, w2)]
+    ref = torch.zeros(T, H, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        t, k = (idx == e).nonzero(as_tuple=True)
+        gate, up = (l64[0][t] @ l64[2][e].T).split(I, dim=1)
+        y = (torch.nn.functional.silu(gate) * up) @ l64[3][e].T
+        ref = ref.index_add(0, t, y * l64[1][t, k][:, None])
+    ref.backward(dout.double())
+    for got, want in [(out, ref)] + [(a.grad, b.grad) for a, b in zip(leaves, l64)]:
+        # fp32 rounding through three contractions of at most 256 terms
+        assert float((got.double() - want).norm() / want.norm()) < 5e-6
