@@ -92,3 +92,53 @@ def test_tile_plan_tables(T, E, K):
             exp += [(e, r, hi) for r in range(lo, hi, bm)]
         assert info.tolist() == [list(x) for x in exp]
         base += 16 * ((S + bm - 1) // bm + E)
+
+
+# (T, E, K): both forms of the permutation around their limits (S = 8192 rows
+# and, at 2400 rows, 2076 experts), remainders of 64 entries, of a wave's run and of a chunk
+FORMS = [(1, 1, 1), (4, 128, 8), (63, 7, 1), (65, 16, 4), (1024, 33, 1), (1025, 100, 3),
+         (4095, 128, 8), (4096, 128, 8), (4097, 128, 8), (8191, 60, 1), (8192, 60, 1), (8193, 60, 1),
+         (16384, 1, 1), (300, 2076, 8), (300, 2077, 8), (5000, 2288, 8), (70000, 3, 1)]
+
+
+@pytest.mark.parametrize("T,E,K", FORMS)
+def test_permute_forms(T, E, K):
+    print(f"permute form T={T} E={E} K={K}", flush=True)
+    idx = _routing(T, E, K, 11 * T + E, skew=1.0, sentinel_every=5 if E > 1 else 0)
+    S = T * K
+    plan = ops.permute(idx.to(DEV), E)
+    again = ops.permute(idx.to(DEV), E)
+    torch.cuda.synchronize()
+    ref = O.permute(idx, E)
+    for got, want in ((plan.counts, ref.counts), (plan.offsets, ref.offsets),
+                      (plan.row_src, ref.row_src), (plan.slot, ref.slot),
+                      (plan.tile_starts, ref.tile_starts)):
+        assert np.array_equal(got.cpu().numpy(), want)
+    assert torch.equal(plan.tile_plan, again.tile_plan)  # every byte is written
+    raw = plan.tile_plan.cpu().numpy()
+    base = (3 * (E + 1) * 4 + 4 + 15) // 16 * 16
+    for b, bm in enumerate(O.TILE_SIZES):
+        n = (S + bm - 1) // bm + E
+        info = raw[base: base + 16 * n].view(np.int32).reshape(n, 4)
+        exp = np.zeros((n, 4), np.int32)
+        t = 0
+        for e in range(E):
+            lo, hi = int(ref.offsets[e]), int(ref.offsets[e + 1])
+            for r in range(lo, hi, bm):
+                exp[t] = (e, r, hi, 0)
+                t += 1
+        assert np.array_equal(info, exp)
+        base += 16 * n
+    sched = raw[base:].view(np.int32)
+    assert not sched[:32].any()  # queue counters
+    xstart, xnz, xorder = sched[32:41], sched[48:56], sched[64:64 + E]
+    assert sorted(xorder.tolist()) == list(range(E))
+    assert xstart[0] == 0 and xstart[8] == E
+    counts = np.asarray(ref.counts)
+    assert int(xnz.sum()) == int((counts > 0).sum())
+    for x in range(8):
+        mine = counts[xorder[xstart[x]: xstart[x + 1]]]
+        assert (mine[:xnz[x]] > 0).all() and not mine[xnz[x]:].any()
+        # heaviest first, up to a bucket's width (an eighth of an octave)
+        cost = mine[:xnz[x]] + 192.0
+        assert (cost[1:] <= cost[:-1] * 2 ** 0.126).all()
