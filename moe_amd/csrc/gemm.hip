@@ -108,9 +108,10 @@ struct GemmArgs {
   const int* row_src;    // [S]
   const int* offsets;    // [E+1]
   const int* tile_count; // token modes: number of row tiles (tile_starts[E] for BR)
-  const int* row_tile;   // token modes: the plan's chosen row-tile index; a launch whose
-                         // BR is another one returns at once (null: no choice to honour)
   const int4* tile_info; // token modes: {expert, first row, end row, 0} per row tile
+  const int* row_tile;   // token_gemm_kernel: the plan's chosen row-tile index and the
+  const int* tile_counts[3];   // tile_count and tile_info of the three heights
+  const int4* tile_infos[3];
   bf16* out;
   bf16* out2;            // gate_up output of G1F (may be null); w * act [S,I] of G2DXF
   const void* rw;        // G2DXF: routing weights [T*K], fp32 or bf16 (rw_bf16)
@@ -213,15 +214,11 @@ __device__ __forceinline__ float fast_sigmoid(float x) {
 }
 
 template <int MODE, int BR>
-__global__ __launch_bounds__(kWaves<BR> * 64, 1) void grouped_gemm_kernel(GemmArgs p) {
+__device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
   constexpr int NW = kWaves<BR>;                          // waves, as NW/2 rows x 2 columns
   constexpr int NTHR = NW * 64;
   constexpr bool TOKEN = MODE <= G1DX || MODE == G2DXF;   // rows = routed rows of one expert
   constexpr bool TRL = MODE == RLT || MODE == RLTK || MODE == RLTS;  // transposed router linear
-  if constexpr (TOKEN) {
-    constexpr int my_tile = BR == 64 ? 0 : (BR == 128 ? 1 : 2);
-    if (p.row_tile && __builtin_amdgcn_readfirstlane(*p.row_tile) != my_tile) return;
-  }
   constexpr bool DENSE = MODE == RL || MODE == RDX || TRL;  // one "expert", dense rows
   constexpr bool COL_KM = !(MODE == G1F || MODE == G2F || MODE == RL || TRL);  // k-major cols
   constexpr bool ROW_KM = !TOKEN && !DENSE;               // row operand k-major (dW)
@@ -1737,6 +1734,32 @@ __global__ __launch_bounds__(kWaves<BR> * 64, 1) void grouped_gemm_kernel(GemmAr
   }
 }
 
+template <int MODE, int BR>
+__global__ __launch_bounds__(kWaves<BR> * 64, 1) void grouped_gemm_kernel(GemmArgs p) {
+  grouped_gemm<MODE, BR>(p);
+}
+
+// A token-grouped GEMM whose row-tile height the permutation chose: one
+// launch holds all three (a launch per height, of which two return at once,
+// cost 2-5 us for each of those two).
+template <int MODE>
+__global__ __launch_bounds__(kWaves<256> * 64, 1) void token_gemm_kernel(GemmArgs p) {
+  const int b = __builtin_amdgcn_readfirstlane(*p.row_tile);
+  if (b == 0) {
+    p.tile_count = p.tile_counts[0];
+    p.tile_info = p.tile_infos[0];
+    grouped_gemm<MODE, 64>(p);
+  } else if (b == 1) {
+    p.tile_count = p.tile_counts[1];
+    p.tile_info = p.tile_infos[1];
+    grouped_gemm<MODE, 128>(p);
+  } else {
+    p.tile_count = p.tile_counts[2];
+    p.tile_info = p.tile_infos[2];
+    grouped_gemm<MODE, 256>(p);
+  }
+}
+
 void set_topk(GemmArgs& a, int top_k) {
   a.topk = top_k;
   int sh = 0;
@@ -1761,69 +1784,72 @@ int num_cus() {
   return n;
 }
 
+// Launches `kernel` (of 256 threads, with `lds` bytes of dynamic LDS) as a
+// persistent grid: one workgroup per CU (a multiple of the 8 XCDs), never
+// more workgroups than tiles.
+int launch_persistent(void (*kernel)(GemmArgs), std::atomic<int> (&lds_done)[64], size_t lds,
+                      const GemmArgs& a, int max_tiles, hipStream_t st) {
+  if (max_tiles <= 0) return MOE_OK;
+  hipError_t err = set_dynamic_lds_once(lds_done, (const void*)kernel, (int)lds);
+  if (err != hipSuccess) {
+    set_error("grouped_gemm: hipFuncSetAttribute failed: %s", hipGetErrorString(err));
+    return MOE_ERR_HIP;
+  }
+  int grid = num_cus() / 8 * 8;
+  const int need = (max_tiles + 7) / 8 * 8;
+  if (grid > need) grid = need;
+  if (grid < 8) grid = 8;
+  kernel<<<grid, 256, lds, st>>>(a);
+  return check_launch("grouped_gemm");
+}
+
 template <int MODE, int BR>
 int launch(const GemmArgs& a, int max_tiles, hipStream_t st) {
+  static_assert(kWaves<BR> == 4, "256 threads");
   constexpr size_t stages = (size_t)NSLOT * SLOT;
   // staging tile of the non-PF epilogues ([BC][SROW] when transposed)
   constexpr size_t staging =
       MODE == RLTS ? (size_t)BC * (BR + 4) * sizeof(float)  // fp32 logits [token][expert]
                    : (size_t)((MODE == G2DWG || MODE == RLT || MODE == RLTK) ? BC : BR) * SROW *
                          sizeof(bf16);
-  const size_t lds = stages > staging ? stages : staging;
-  if (max_tiles <= 0) return MOE_OK;
   static std::atomic<int> lds_done[64];
-  hipError_t err =
-      set_dynamic_lds_once(lds_done, (const void*)grouped_gemm_kernel<MODE, BR>, (int)lds);
-  if (err != hipSuccess) {
-    set_error("grouped_gemm: hipFuncSetAttribute failed: %s", hipGetErrorString(err));
-    return MOE_ERR_HIP;
-  }
-  // Persistent grid: one workgroup per CU (a multiple of the 8 XCDs), never
-  // more workgroups than tiles.
-  int grid = num_cus() / 8 * 8;
-  const int need = (max_tiles + 7) / 8 * 8;
-  if (grid > need) grid = need;
-  if (grid < 8) grid = 8;
-  grouped_gemm_kernel<MODE, BR><<<grid, kWaves<BR> * 64, lds, st>>>(a);
-  return check_launch("grouped_gemm");
+  return launch_persistent(grouped_gemm_kernel<MODE, BR>, lds_done,
+                           stages > staging ? stages : staging, a, max_tiles, st);
 }
 
-// Row-tile height for the token-grouped GEMMs from the mean rows per expert.
-int pick_br(int64_t S, int E) {
-  const int64_t avg = S / (E > 0 ? E : 1);
-  if (avg >= 512) return 256;
-  if (avg >= 128) return 128;
-  return 64;
-}
+// Mean rows per expert from which the host picks 256-row tiles by itself.
+bool host_picks_256(int64_t S, int E) { return S / (E > 0 ? E : 1) >= 512; }
 
 // Launches a token-grouped GEMM.  With at least 512 routed rows per expert
 // on average every expert that has rows has enough for 256-row tiles, so the
 // host picks them.  Below that the rows per *routed-to* expert decide, which
 // only the device knows: the permutation wrote the height of least streamed
-// bytes into the plan, all three heights are launched, and the two others
-// return at once (one scalar load per workgroup).  Results do not depend on
-// the height: every output element is one k-ordered MFMA chain either way.
+// bytes into the plan and token_gemm_kernel takes it.  Results do not depend
+// on the height: every output element is one k-ordered MFMA chain either way.
 template <int MODE>
 int launch_token(GemmArgs a, int64_t S, int E, int ncols_per_tile_out, int ncols_total,
                  const void* tile_plan, hipStream_t st) {
   const char* pb = (const char*)tile_plan;
   a.n_ct = (ncols_total + ncols_per_tile_out - 1) / ncols_per_tile_out;
-  const bool device_choice = pick_br(S, E) != 256;
-  a.row_tile = device_choice ? (const int*)(pb + plan_row_tile_offset(E)) : nullptr;
-  for (int b = device_choice ? 0 : 2; b < 3; ++b) {
-    a.tile_count = (const int*)pb + (size_t)b * (E + 1) + E;
-    a.tile_info = (const int4*)(pb + plan_info_offset(S, E, b));
-    const int64_t max_tiles = plan_max_tiles(S, E, b) * a.n_ct;
-    if (max_tiles > (int64_t)1 << 30) {
+  for (int b = 0; b < 3; ++b) {
+    a.tile_counts[b] = (const int*)pb + (size_t)b * (E + 1) + E;
+    a.tile_infos[b] = (const int4*)(pb + plan_info_offset(S, E, b));
+    if (plan_max_tiles(S, E, b) * a.n_ct > (int64_t)1 << 30) {
       set_error("grouped_gemm: too many tiles");
       return MOE_ERR_UNSUPPORTED;
     }
-    const int rc = b == 2 ? launch<MODE, 256>(a, (int)max_tiles, st)
-                 : b == 1 ? launch<MODE, 128>(a, (int)max_tiles, st)
-                          : launch<MODE, 64>(a, (int)max_tiles, st);
-    if (rc != MOE_OK) return rc;
   }
-  return MOE_OK;
+  if (host_picks_256(S, E)) {
+    a.tile_count = a.tile_counts[2];
+    a.tile_info = a.tile_infos[2];
+    return launch<MODE, 256>(a, (int)(plan_max_tiles(S, E, 2) * a.n_ct), st);
+  }
+  a.row_tile = (const int*)(pb + plan_row_tile_offset(E));
+  constexpr size_t staging = (size_t)256 * SROW * sizeof(bf16);
+  constexpr size_t stages = (size_t)NSLOT * SLOT;
+  static std::atomic<int> lds_done[64];
+  return launch_persistent(token_gemm_kernel<MODE>, lds_done, stages > staging ? stages : staging,
+                           a, (int)(plan_max_tiles(S, E, 0) * a.n_ct), st);
 }
 int check_common(int64_t S, int E, int H, int I, int dtype, const char* who) {
   MOE_REQUIRE(dtype == MOE_DTYPE_BF16 || dtype == MOE_DTYPE_F32, MOE_ERR_DTYPE,
