@@ -251,7 +251,18 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
                       MODE == RDX || MODE == G2DXF;
   constexpr int NST = (MODE == G1F ? 12 : 8) * TJ;
   static_assert(!PF || FPW + NST <= 63, "vmcnt range");
-  static_assert(TOKEN || DENSE || BR == 256, "dW modes use 256-row tiles");
+  // VH: a tile multiplies and writes only the 64-row units it has (an
+  // expert's last tile is rarely full: a quarter of the rows multiplied are
+  // padding at 512 +- 22 rows per expert).  The waves' row sub-tiles
+  // interleave: sub-tile j of wave row w holds tile rows (2j + w)*32 .. +31,
+  // so that unit j is sub-tile j of both wave rows; the first nj are computed,
+  // by a main loop for each nj.  The row operand's rows past the end read
+  // zeros without memory access.  A second tile of few rows next to its
+  // expert's full one takes about 25 us where it took 29 (G1F at H = 2048, 257
+  // rows in each of 128 experts: 349 -> 305 us, G1DX 326 -> 299; 64-row tiles
+  // in a launch of their own would stream the weights from HBM again, as
+  // ordering the tiles by height did: 401 us).
+  constexpr bool VH = TOKEN && PF && TJ > 1;
 
   extern __shared__ __attribute__((aligned(16))) bf16 smem[];
 
@@ -319,6 +330,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
 
   struct Tile {
     int e, row0, row_end, ct, kbeg, kend, nk;
+    int nj;  // row sub-tiles per wave that have rows (VH), else TJ
   };
   // pre (token modes): the tile's {expert, first row, end row} loaded ahead
   auto decode = [&](int tt, const int4* pre = nullptr) {
@@ -367,6 +379,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     else if constexpr (MODE == G1DX) K_len = I2;
     else K_len = d.kend - d.kbeg;
     d.nk = (K_len + BK - 1) / BK;
+    d.nj = VH ? min(TJ, (d.row_end - d.row0 + 63) >> 6) : TJ;
     return d;
   };
 
@@ -535,7 +548,8 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         const int f = kc_feature(wid + NW * i);
         const int r = min(d.row0 + f, d.row_end - 1);
         const int tok = div_topk(rs ? rs[i] : p.row_src[r], p.tok_mul, p.tok_shift);
-        roff[i] = (uint32_t)tok * (uint32_t)(H * 2) + kc_chunk(f) * 16;
+        roff[i] = (!VH || d.row0 + f < d.row_end)
+                      ? (uint32_t)tok * (uint32_t)(H * 2) + kc_chunk(f) * 16 : kOOB;
       }
       rstep = BK * 2;
     } else if constexpr (TOKEN || DENSE) {
@@ -547,7 +561,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       for (int i = 0; i < RPW; ++i) {
         const int f = kc_feature(wid + NW * i);
         const int r = min(f, d.row_end - d.row0 - 1);
-        roff[i] = (uint32_t)r * (uint32_t)(ld * 2) + kc_chunk(f) * 16;
+        roff[i] = (!VH || r == f) ? (uint32_t)r * (uint32_t)(ld * 2) + kc_chunk(f) * 16 : kOOB;
       }
       rstep = BK * 2;
     } else {
@@ -567,7 +581,8 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     if constexpr (MODE == G2DXF) {
 #pragma unroll
       for (int j = 0; j < TJ; ++j)
-        nsrc[j] = p.row_src[min(d.row0 + wr * WR + j * 32 + l32, d.row_end - 1)];
+        nsrc[j] = p.row_src[min(d.row0 + (VH ? (2 * j + wr) * 32 : wr * WR + j * 32) + l32,
+                                d.row_end - 1)];
     }
   };
 
@@ -649,7 +664,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       a_off[q] = (uint32_t)tka * (BC * 2) +
                  ((uint32_t)((wc * 16 + q * 4 + tsub) ^ ((tka & 3) << 2)) << 4) + thalf;
     if constexpr (!ROW_KM)
-      b_off[q] = (uint32_t)(wr * WR + l32) * (BK * 2) + (uint32_t)(((2 * q + hl) ^ ((l32 >> 1) & 7)) * 16);
+      b_off[q] = (uint32_t)(wr * (VH ? 32 : WR) + l32) * (BK * 2) + (uint32_t)(((2 * q + hl) ^ ((l32 >> 1) & 7)) * 16);
     else
       b_off[q] = (uint32_t)tka * (BR * 2) +
                  ((uint32_t)((wr * (WR / 8) + q * 4 + tsub) ^ ((tka & 3) << 2)) << 4) + thalf;
@@ -683,7 +698,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
   };
   auto read_b = [&](int ks, int j) -> bf16x8 {
     if constexpr (!ROW_KM) {
-      return *(const __attribute__((address_space(3))) bf16x8*)lds_at(b_adr[ks] + j * 4096);
+      return *(const __attribute__((address_space(3))) bf16x8*)lds_at(b_adr[ks] + j * (VH ? 8192 : 4096));
     } else {
       const lds_char_t* q = lds_at(b_adr[j] + ks * (16 * BR * 2));
       return tr_frag(q, q + 4 * BR * 2);
@@ -721,10 +736,13 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       if constexpr (ROW_FIRST) issue_row(1);
       else issue_col(1, tk_b);
   };
-  // Main loop of tile `cur` (its prologue issued).  after_epi: the previous
-  // tile's epilogue stores were issued after this tile's prologue (PF modes).
-  auto mainloop = [&](const Tile& cur, bool after_epi) {
-    (void)after_epi;
+  // Main loop of tile `cur` (its prologue issued), over its first NJ row
+  // sub-tiles per wave.  epi_stores: how many stores of the previous tile's
+  // epilogue were issued after this tile's prologue (PF modes: 0, NST / 2 or
+  // NST).
+  auto mainloop = [&](const Tile& cur, int epi_stores, auto nj_t) {
+    constexpr int NJ = decltype(nj_t)::value;
+    (void)epi_stores;
       // Byte offsets of ring positions 2kt + c, c = 0..4, at stage kt.  The
       // positions advance by two per stage, so the five offsets rotate by
       // two at the end of each stage (register moves, not a modulo).
@@ -782,15 +800,16 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         }
       };
       constexpr int GQ = BK / 16 - 1;  // groups before the last sub-step: NGRP - TI
-      constexpr int NLR = TI + TJ;     // fragment reads of a sub-step
-      bf16x8 fa[2][TI], fb[2][TJ];
+      constexpr int NLR = TI + NJ;     // fragment reads of a sub-step
+      bf16x8 fa[2][TI], fb[2][NJ];
       if constexpr (PF) {
         // the previous tile's NST epilogue stores were issued after this
         // tile's first stages: they may still be in flight
         // (G2DXF: its epilogue waited for gate/up loads issued after this
         // tile's first stages, and loads complete in issue order, so those
         // stages have landed; only its trailing stores may be in flight.)
-        if (after_epi) WAIT_VMCNT_LGKM0(MODE == G2DXF ? 63 : FPW + NST);
+        if (epi_stores == NST) WAIT_VMCNT_LGKM0(MODE == G2DXF ? 63 : FPW + NST);
+        else if (epi_stores) WAIT_VMCNT_LGKM0(MODE == G2DXF ? 63 : FPW + NST / 2);
         else WAIT_VMCNT_LGKM0(FPW);
       } else {
         WAIT_VMCNT_LGKM0(FPW);
@@ -801,7 +820,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
 #pragma unroll
       for (int i = 0; i < TI; ++i) fa[0][i] = read_a(0, i);
 #pragma unroll
-      for (int j = 0; j < TJ; ++j) fb[0][j] = read_b(0, j);
+      for (int j = 0; j < NJ; ++j) fb[0][j] = read_b(0, j);
       // the part of W(0) that belongs to the (absent) last sub-step of stage -1
       __amdgpu_buffer_rsrc_t rs_second = second_rsrc(1);  // W(0)'s second half: stage 1
 #pragma unroll
@@ -822,7 +841,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
               win_op(kt, o, tk_a, rq[3], rq[4], rs_second, rs_first);  // positions 2kt+3, 2kt+4
             if (ks + 1 < GQ) {
               fa[(ks + 1) & 1][i] = read_a(ks + 1, i);
-              if (i < TJ) fb[(ks + 1) & 1][i] = read_b(ks + 1, i);
+              if (i < NJ) fb[(ks + 1) & 1][i] = read_b(ks + 1, i);
             } else {
               // The last sub-step's fragments, read in the groups before the
               // last one: the barrier's lgkmcnt(0) then finds them landed.
@@ -833,7 +852,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
               }
             }
 #pragma unroll
-            for (int j = 0; j < TJ; ++j)
+            for (int j = 0; j < NJ; ++j)
               acc[i][j] = mma(fa[ks & 1][i], fb[ks & 1][j], acc[i][j]);
             group_order();
             // Scalar instructions (slot offsets, descriptors, M0) may cross
@@ -866,9 +885,9 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
           for (int o = i * NOPS / NGRP; o < (i + 1) * NOPS / NGRP; ++o)
             win_op(kt + 1, o, tk_a, rq[0], rq[1], rs_second, rs_second);  // positions 2kt+5, 2kt+6
           fa[0][i] = read_a(0, i);
-          if (i < TJ) fb[0][i] = read_b(0, i);
+          if (i < NJ) fb[0][i] = read_b(0, i);
 #pragma unroll
-          for (int j = 0; j < TJ; ++j)
+          for (int j = 0; j < NJ; ++j)
             acc[i][j] = mma(fa[1][i], fb[1][j], acc[i][j]);
           group_order();
           __builtin_amdgcn_sched_barrier(0x4);
@@ -929,12 +948,19 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     }
   };
   u32x4 pre[ACCM ? 32 : 1];
-  auto epilogue_pf = [&](const Tile& c) {
+  // VH: only the pairs of sub-tiles with rows are written (returns the
+  // stores issued: half of NST where one of two pairs has rows).
+  auto epilogue_pf = [&](const Tile& c) -> int {
     // lane- and wave-derived addresses formed here (opaque to the
     // optimizer, which would otherwise hoist them out of the tile loop)
     int ln = lane, wd = wid;
     asm volatile("" : "+v"(ln), "+s"(wd));
     const int el32 = ln & 31, ehl = ln >> 5, ewr = wd >> 1, ewc = wd & 1;
+    // row rr (0..63) of the region holding sub-tiles j0, j0 + 1, relative to
+    // the first row of the store descriptor: the tile's (VH) or the wave's
+    auto erow = [&](int j0, int rr) {
+      return VH ? (2 * (j0 + (rr >> 5)) + ewr) * 32 + (rr & 31) : j0 * 32 + rr;
+    };
     lds_char_t* const reg = (lds_char_t*)smem + 3 * SLOT + wd * 16384;
     auto st16 = [&](__amdgpu_buffer_rsrc_t rs, uint32_t off, const u32x4& v) {
       __builtin_amdgcn_raw_buffer_store_b128(v, rs, off, 0, 2);  // non-temporal
@@ -992,21 +1018,23 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       // further adds a wave-uniform step.  lim: the lane's rows are valid
       // while that step's row count stays below it (never, for features
       // past I).
-      const int r0l = ewr * WR + rq;
+      const int r0l = ewr * (VH ? 32 : WR) + rq;
+      constexpr int JR = VH ? 64 : 32;  // rows from one sub-tile of the wave to the next
       const int lim = fok ? nr - r0l : INT32_MIN;
       const uint32_t bg = (uint32_t)r0l * (uint32_t)(I2 * 2) + (uint32_t)(fw + c8) * 2;
       const uint32_t ba = (uint32_t)r0l * (uint32_t)(I * 2) + (uint32_t)(fw + c8) * 2;
       auto og = [&](int j, int it) -> uint32_t {  // gate bytes of (row, lane's features)
-        const int d = j * 32 + it * 4;
+        const int d = j * JR + it * 4;
         return d < lim ? bg + (uint32_t)d * (uint32_t)(I2 * 2) : kOOB;
       };
       auto oa = [&](int j, int it) -> uint32_t {
-        const int d = j * 32 + it * 4;
+        const int d = j * JR + it * 4;
         return d < lim ? ba + (uint32_t)d * (uint32_t)(I * 2) : kOOB;
       };
       // gate/up of iteration n = j*NIT + it are loaded PD iterations ahead
       // (HBM latency: one iteration's arithmetic is ~1 k cycles)
-      constexpr int PD = 8, NN = TJ * NIT;
+      constexpr int PD = 8;
+      const int nn = (VH ? c.nj : TJ) * NIT;
       u32x4 gl[PD], ul[PD];
       auto load = [&](int n) {
         const uint32_t o = og(n / NIT, n % NIT);
@@ -1014,9 +1042,11 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         ul[n % PD] = __builtin_amdgcn_raw_buffer_load_b128(rgu, o + (uint32_t)I * 2, 0, 2);  // kOOB stays out
       };
 #pragma unroll
-      for (int n = 0; n < PD && n < NN; ++n) load(n);
+      for (int n = 0; n < PD; ++n) load(n);
+      static_assert(PD <= NIT, "the first loads are of sub-tile 0");
 #pragma unroll
       for (int j = 0; j < TJ; ++j) {
+        if (VH && j >= c.nj) break;
         // accumulator rows of sub-tile j -> region, fp32
 #pragma unroll
         for (int i = 0; i < TI; ++i)
@@ -1080,14 +1110,14 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
             dot = fmaf(gq[e0], a[e0], dot);
             dot = fmaf(gq[e1], a[e1], dot);
           }
-          if (n + PD < NN) load(n + PD);
+          if (n + PD < nn) load(n + PD);
           const uint32_t o = og(j, it), oaw = oa(j, it);
           __builtin_amdgcn_raw_buffer_store_b128(dgv, rdg, o, 0, 2);
           __builtin_amdgcn_raw_buffer_store_b128(duv, rdg, o + (uint32_t)I * 2, 0, 2);
           __builtin_amdgcn_raw_buffer_store_b128(awv, raw, oaw, 0, 2);
           // the row's partial over the wave's 128 features
           const float tot = group_sum<16>(fok ? dot : 0.f);
-          if ((ln & 15) == 0 && j * 32 + it * 4 < nr - r0l)
+          if ((ln & 15) == 0 && j * JR + it * 4 < nr - r0l)
             p.dw_part[(int64_t)sq[it] * n_part + c.ct * 2 + ewc] = tot;
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1095,14 +1125,15 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     } else if constexpr (MODE == G1F) {
       // tile columns of this wave: [gate 64 | up 64] of features fb..fb+63
       const int fb = c.ct * 128 + ewc * 64;
-      const int r0 = c.row0 + ewr * WR;
-      const int nr = min(WR, c.row_end - r0);
+      const int r0 = c.row0 + (VH ? 0 : ewr * WR);
+      const int nr = min(VH ? BR : WR, c.row_end - r0);
       const uint32_t rows = nr > 0 ? (uint32_t)nr : 0u;
       const auto ra = make_rsrc(p.out + (int64_t)r0 * I, rows * (uint32_t)I * 2);
       const auto rg = make_rsrc(p.out2 ? p.out2 + (int64_t)r0 * I2 : p.out,
                                 p.out2 ? rows * (uint32_t)I2 * 2 : 0u);
 #pragma unroll
       for (int j0 = 0; j0 < TJ; j0 += 2) {
+        if (VH && j0 >= c.nj) return NST / 2;
         const int nj = TJ - j0 >= 2 ? 2 : 1;
         write_rows(j0, nj);
 #pragma unroll
@@ -1119,7 +1150,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
             const float u0 = bf_lo(uv[w]), u1 = bf_hi(uv[w]);
             av[w] = pack_bf2(round_bf(g0 * fast_sigmoid(g0)) * u0, round_bf(g1 * fast_sigmoid(g1)) * u1);
           }
-          const int feat = fb + f8 * 8, gr = j0 * 32 + rr;
+          const int feat = fb + f8 * 8, gr = erow(j0, rr);
           const bool ok = feat < I;
           st16(ra, ok ? (uint32_t)gr * I * 2 + (uint32_t)feat * 2 : kOOB, av);
           st16(rg, ok ? (uint32_t)gr * I2 * 2 + (uint32_t)feat * 2 : kOOB, gv);
@@ -1175,7 +1206,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       int r0, nrows_all;
       const bf16* ob;
       if constexpr (TOKEN || MODE == RDX) {
-        r0 = c.row0 + ewr * WR;
+        r0 = c.row0 + (VH ? 0 : ewr * WR);
         nrows_all = c.row_end;
         ob = p.out;
       } else {
@@ -1183,7 +1214,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         nrows_all = I2;
         ob = p.out + (int64_t)c.e * I2 * H;
       }
-      const int nr = min(WR, nrows_all - r0);
+      const int nr = min(VH ? BR : WR, nrows_all - r0);
       const auto rs = make_rsrc(ob + (int64_t)r0 * H, nr > 0 ? (uint32_t)nr * (uint32_t)H * 2 : 0u);
       const int cb = c.ct * BC + ewc * 128;
       // G1DW accumulating: as G2DWG's above
@@ -1191,6 +1222,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         constexpr bool ACC = decltype(acc_t)::value;
 #pragma unroll
         for (int j0 = 0; j0 < TJ; j0 += 2) {
+          if (VH && j0 >= c.nj) break;
           const int nj = TJ - j0 >= 2 ? 2 : 1;
           if constexpr (ACC) {
             if (j0 == 0) {
@@ -1209,7 +1241,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
                 pre[kn] = __builtin_amdgcn_raw_buffer_load_b128(rs, dw_off(c, ln, wd, (kn >> 4) * 2, kn & 15), 0, 0);
             }
             u32x4 v = *(const __attribute__((address_space(3))) u32x4*)(reg + rr * 256 + P * 16);
-            const int col = cb + (P ^ (rr & 15)) * 8, gr = j0 * 32 + rr;
+            const int col = cb + (P ^ (rr & 15)) * 8, gr = erow(j0, rr);
             uint32_t off = col < H ? (uint32_t)gr * H * 2 + (uint32_t)col * 2 : kOOB;
             if constexpr (ACC) {
               v = add_bf16x8(pre[(j0 >> 1) * 16 + it], v);
@@ -1227,6 +1259,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         body(std::false_type{});
       }
     }
+    return VH && TJ > 2 && c.nj <= 2 ? NST / 2 : NST;
   };
   // RLTS: the selection counts of this lane's experts (entries e0 .. e0+SV-1
   // of its lane group of 8), summed over every token it routes and flushed
@@ -1274,7 +1307,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     }
     if ((dyn ? t >= 0 : t < t_end) && cur.nk > 0) prologue();
     if (dyn ? t >= 0 : t < t_end) take_rows();
-    bool first = true;
+    int stored = 0;
     while (dyn ? t >= 0 : t < t_end) {
 #pragma unroll
       for (int i = 0; i < TI; ++i)
@@ -1282,7 +1315,14 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         for (int j = 0; j < TJ; ++j)
 #pragma unroll
           for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-      if (cur.nk > 0) mainloop(cur, !first);
+      if (cur.nk > 0) {
+        if (!VH || cur.nj == TJ) mainloop(cur, stored, std::integral_constant<int, TJ>{});
+        else if (cur.nj == 1) mainloop(cur, stored, std::integral_constant<int, 1>{});
+        else if constexpr (TJ > 2) {
+          if (cur.nj == 2) mainloop(cur, stored, std::integral_constant<int, 2>{});
+          else mainloop(cur, stored, std::integral_constant<int, 3>{});
+        }
+      }
       // The ring is idle: the stages past the last one have landed (empty
       // descriptors) and every wave has finished its LDS reads.
       WAIT_VMCNT_LGKM0(0);
@@ -1303,12 +1343,11 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         }
       }
       if (more && nxt.nk > 0) prologue();
-      epilogue_pf(cur);
+      stored = epilogue_pf(cur);
       if (!more) break;
       take_rows();
       cur = nxt;
       t = tn_next;
-      first = false;
     }
   } else {
   for (; dyn ? t >= 0 : t < t_end; t = dyn ? claim() : t + nslot) {
@@ -1340,7 +1379,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
     // keep the wait counts exact.
     if (cur.nk > 0) {
       prologue();
-      mainloop(cur, false);
+      mainloop(cur, 0, std::integral_constant<int, TJ>{});
     }
 
     // --------------------------------------------------------- epilogue
