@@ -431,6 +431,43 @@ int moe_amd_seq_aux_backward(const void* scores, int scores_dtype, const double*
 int moe_amd_switch_aux_backward(const double* coef, const float* token_weights, int64_t T, int E,
                                 int grad_dtype, void* grad, void* stream);
 
+/* The sequence-wise loss of a whole model: L layers of one shape and dtype,
+ * scores[l] [T,E] and selected[l] [T,K] int64 (null: the top K of the
+ * normalised scores; `selected` itself may be null).  The arrays of pointers
+ * are host arrays, read during the call.  With c and P the counts and means of
+ * moe_amd_seq_stats and f = c * f_scale: coef[l,b,e] = f * coef_scale, and the
+ * loss = loss_scale * sum over l, b, e of f * P, in fp64 and rounded to fp32.
+ * src/models/load_balancing.py:93-169 has f_scale = E / (K S), coef_scale =
+ * 1 / (L B S) and loss_scale = 1 / (L B). */
+size_t moe_amd_seq_aux_loss_workspace_size(int L, int64_t T, int E, int B);
+int moe_amd_seq_aux_loss(const void* const* scores, const int64_t* const* selected, int L,
+                         int scores_dtype, int64_t T, int E, int K, int B, double f_scale,
+                         double coef_scale, double loss_scale, void* workspace,
+                         size_t workspace_bytes, double* coef, double* loss64, float* loss,
+                         void* stream);
+/* ... and its gradient: moe_amd_seq_aux_backward of every layer, with
+ * coef[l,b,e] * *d_loss in the place of coef (d_loss: device scalar). */
+int moe_amd_seq_aux_loss_backward(const void* const* scores, int L, int scores_dtype,
+                                  const double* coef, const float* d_loss, int64_t T, int E, int B,
+                                  void* const* d_scores, void* stream);
+
+/* The Switch loss of a whole model (src/models/load_balancing.py:19-90): L
+ * layers probs[l] [T,E] of one dtype (host array of pointers).  With the
+ * counts and sums of moe_amd_topk_stats added over the layers and d = denom,
+ * or denom * *denom_dev when denom_dev is given: loss = num_experts * sum_e
+ * (counts / d) (sums / d), coef[e] = counts / d * num_experts / d (fp64). */
+size_t moe_amd_switch_aux_loss_workspace_size(int L, int64_t T, int E);
+int moe_amd_switch_aux_loss(const void* const* probs, int L, int probs_dtype,
+                            const float* token_weights, int64_t T, int E, int K,
+                            double num_experts, double denom, const double* denom_dev,
+                            void* workspace, size_t workspace_bytes, double* coef, double* loss,
+                            void* stream);
+/* ... and its gradient: moe_amd_switch_aux_backward into every layer's
+ * grads[l], with coef * *d_loss in the place of coef. */
+int moe_amd_switch_aux_loss_backward(const double* coef, const float* d_loss,
+                                     const float* token_weights, int L, int64_t T, int E,
+                                     int grad_dtype, void* const* grads, void* stream);
+
 /* Aux-loss-free balancing step for L routers at once (train.py:79-139 without
  * the DDP all-reduce): counts[l] and biases[l] are device pointers to each
  * router's fp32 [E] local_tokens_per_expert and expert_bias (the two arrays

@@ -30,6 +30,7 @@ _p = ctypes.c_void_p
 _i = ctypes.c_int
 _i64 = ctypes.c_int64
 _f = ctypes.c_float
+_d = ctypes.c_double
 _sz = ctypes.c_size_t
 
 # name -> (restype, argtypes); mirrors include/moe_amd.h one to one.
@@ -88,7 +89,15 @@ SIGNATURES: dict[str, tuple] = {
     "moe_amd_seq_stats": (_i, [_p, _i, _p, _i64, _i, _i, _i, _p, _sz, _p, _p, _p]),
     "moe_amd_seq_aux_backward": (_i, [_p, _i, _p, _i64, _i, _i, _p, _p]),
     "moe_amd_switch_aux_backward": (_i, [_p, _p, _i64, _i, _i, _p, _p]),
-    "moe_amd_update_expert_biases": (_i, [_p, _p, _i, _i, _f, _i, ctypes.c_double, _p, _p]),
+    "moe_amd_seq_aux_loss_workspace_size": (_sz, [_i, _i64, _i, _i]),
+    "moe_amd_seq_aux_loss": (
+        _i, [_p, _p, _i, _i, _i64, _i, _i, _i, _d, _d, _d, _p, _sz, _p, _p, _p, _p]),
+    "moe_amd_seq_aux_loss_backward": (_i, [_p, _i, _i, _p, _p, _i64, _i, _i, _p, _p]),
+    "moe_amd_switch_aux_loss_workspace_size": (_sz, [_i, _i64, _i]),
+    "moe_amd_switch_aux_loss": (
+        _i, [_p, _i, _i, _p, _i64, _i, _i, _d, _d, _p, _p, _sz, _p, _p, _p]),
+    "moe_amd_switch_aux_loss_backward": (_i, [_p, _p, _p, _i, _i64, _i, _i, _p, _p]),
+    "moe_amd_update_expert_biases": (_i, [_p, _p, _i, _i, _f, _i, _d, _p, _p]),
 }
 
 _lock = threading.Lock()

@@ -21,6 +21,7 @@ implementation-defined); sums accumulate in fp64 in a fixed order.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Sequence
 
@@ -62,6 +63,12 @@ def topk_stats(probs: torch.Tensor, top_k: int, token_weights: torch.Tensor | No
     return out[:E], out[E:2 * E], out[2 * E:]
 
 
+def _ptr_array(tensors) -> ctypes.Array:
+    """Device addresses as a host array of pointers (None: null)."""
+    return (ctypes.c_void_p * len(tensors))(*[None if t is None else t.data_ptr()
+                                              for t in tensors])
+
+
 # ---------------------------------------------------------- Switch loss
 
 class SwitchAuxLoss(torch.autograd.Function):
@@ -72,39 +79,71 @@ class SwitchAuxLoss(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, num_experts, top_k, token_weights, *layers):
-        counts = sums = None
-        for g in layers:
-            c, s, _ = topk_stats(g, top_k, token_weights)
-            counts = c if counts is None else counts + c
-            sums = s if sums is None else sums + s
         # the number of (mask-weighted) tokens over all layers
+        denom_t = None
         if token_weights is not None:
-            denom_t = token_weights.to(torch.float64).sum() * len(layers)
-        else:
-            denom_t = torch.tensor(float(sum(g.shape[0] for g in layers)), dtype=torch.float64,
-                                   device=counts.device)
-        tpe = counts / denom_t
-        loss = (tpe * (sums / denom_t)).sum() * num_experts
-        ctx.coef = tpe * (num_experts / denom_t)
+            denom_t = token_weights.to(torch.float64).sum()
+        first = layers[0]
         ctx.token_weights = token_weights
         ctx.meta = [(g.shape, g.dtype) for g in layers]
-        return loss.to(layers[0].dtype if layers[0].is_floating_point() else torch.float32)
+        T, E = first.shape
+        if T > 0 and all(m == ctx.meta[0] for m in ctx.meta):
+            ctx.coef, loss = _switch_loss(num_experts, top_k, token_weights, denom_t, *layers)
+        else:
+            counts = sums = None
+            for g in layers:
+                c, s, _ = topk_stats(g, top_k, token_weights)
+                counts = c if counts is None else counts + c
+                sums = s if sums is None else sums + s
+            if denom_t is not None:
+                denom_t = denom_t * len(layers)
+            else:
+                denom_t = torch.tensor(float(sum(g.shape[0] for g in layers)), dtype=torch.float64,
+                                       device=counts.device)
+            tpe = counts / denom_t
+            loss = (tpe * (sums / denom_t)).sum() * num_experts
+            ctx.coef = tpe * (num_experts / denom_t)
+        return loss.to(first.dtype if first.is_floating_point() else torch.float32)
 
     @staticmethod
     @on_tensor_device
     def backward(ctx, g):
-        coef = _contig(ctx.coef * g.to(torch.float64))
-        w = ctx.token_weights
-        grads = []
-        for shape, dt in ctx.meta:
-            T, E = shape
+        w, coef = ctx.token_weights, ctx.coef
+        g = _contig(g.to(torch.float32))
+        grads: list = [None] * len(ctx.meta)
+        for meta in dict.fromkeys(ctx.meta):
+            (T, E), dt = meta
+            at = [i for i, m in enumerate(ctx.meta) if m == meta]
             gdt = dt if dt in (torch.float32, torch.bfloat16) else torch.float32
-            out = torch.empty(T, E, device=coef.device, dtype=gdt)
-            _call("moe_amd_switch_aux_backward", coef.data_ptr(),
-                  w.data_ptr() if w is not None else None, T, E, _dtype_code(gdt),
-                  out.data_ptr(), _stream(coef))
-            grads.append(out.to(dt))
+            outs = [torch.empty(T, E, device=coef.device, dtype=gdt) for _ in at]
+            _call("moe_amd_switch_aux_loss_backward", coef.data_ptr(), g.data_ptr(),
+                  w.data_ptr() if w is not None else None, len(at), T, E, _dtype_code(gdt),
+                  _ptr_array(outs), _stream(coef))
+            for i, out in zip(at, outs):
+                grads[i] = out if gdt == dt else out.to(dt)
         return (None, None, None, *grads)
+
+
+@on_tensor_device
+def _switch_loss(num_experts, top_k, token_weights, denom_t, *layers):
+    """(coef [E], loss) fp64 of layers of one shape and dtype, in three launches."""
+    _need_cuda(token_weights, *layers)
+    ps = [_as_probs(g) for g in layers]
+    L, (T, E), dev = len(ps), ps[0].shape, ps[0].device
+    w = token_weights
+    if w is not None:
+        w = _contig(w.reshape(-1).to(device=dev, dtype=torch.float32))
+        if w.numel() != T:
+            raise ValueError(f"token weights: {w.numel()} values for {T} tokens")
+    nbytes = int(_lib.load().moe_amd_switch_aux_loss_workspace_size(L, T, E))
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    out = torch.empty(E + 1, device=dev, dtype=torch.float64)
+    _call("moe_amd_switch_aux_loss", _ptr_array(ps), L, _dtype_code(ps[0].dtype),
+          w.data_ptr() if w is not None else None, T, E, top_k, float(num_experts),
+          float(L) if denom_t is not None else float(L * T),
+          denom_t.data_ptr() if denom_t is not None else None, ws.data_ptr(), nbytes,
+          out.data_ptr(), out[E:].data_ptr(), _stream(ps[0]))
+    return out[:E], out[E]
 
 
 def load_balancing_loss_func(gate_logits, num_experts: int | None = None, top_k: int = 2,
@@ -136,48 +175,58 @@ class SeqAuxLoss(torch.autograd.Function):
     @staticmethod
     @on_tensor_device
     def forward(ctx, num_experts, top_k, batch_size, selected, *layers):
-        total = None
-        ctx.saved = []
         L = len(layers)
-        for li, g in enumerate(layers):
-            _need_cuda(g)
-            s = _as_probs(g)
-            T, E = s.shape
+        _need_cuda(*layers)
+        ps = [_as_probs(g) for g in layers]
+        sels: list = [None] * L
+        for li in range(min(L, len(selected)) if selected is not None else 0):
+            cand, s = selected[li], ps[li]
+            if cand is not None and cand.shape == (s.shape[0], top_k):
+                if cand.dtype != torch.int64 or cand.device != s.device:
+                    cand = cand.to(device=s.device, dtype=torch.int64)
+                sels[li] = _contig(cand)
+        # layers of one shape and dtype (all of a model's) go through together
+        kinds = [(s.shape, s.dtype) for s in ps]
+        ctx.groups = []
+        total = None
+        for kind in dict.fromkeys(kinds):
+            at = [i for i, k in enumerate(kinds) if k == kind]
+            (T, E), dt = kind
+            dev, n = ps[at[0]].device, len(at)
             S = T // batch_size
-            sel = None
-            if selected is not None and li < len(selected):
-                cand = selected[li]
-                if cand is not None and tuple(cand.shape) == (T, top_k):
-                    sel = _contig(cand.to(device=s.device, dtype=torch.int64))
-            nbytes = int(_lib.load().moe_amd_seq_stats_workspace_size(T, E, batch_size))
+            nbytes = int(_lib.load().moe_amd_seq_aux_loss_workspace_size(n, T, E, batch_size))
             if nbytes == 0:
                 raise ValueError(f"seq load-balancing loss: {T} tokens do not split into "
                                  f"{batch_size} sequences")
-            ws = torch.empty(nbytes, device=s.device, dtype=torch.uint8)
-            cnt = torch.empty(batch_size, E, device=s.device, dtype=torch.float64)
-            P = torch.empty_like(cnt)
-            _call("moe_amd_seq_stats", s.data_ptr(), _dtype_code(s.dtype),
-                  sel.data_ptr() if sel is not None else None, T, E, top_k, batch_size,
-                  ws.data_ptr(), ws.numel(), cnt.data_ptr(), P.data_ptr(), _stream(s))
-            f = cnt * (num_experts / (top_k * S))
-            layer_loss = (f * P).sum(dim=-1).mean()
-            total = layer_loss if total is None else total + layer_loss
-            ctx.saved.append((s, f / (L * batch_size * S), g.dtype))
+            ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+            coef = torch.empty(n * batch_size * E + 1, device=dev, dtype=torch.float64)
+            loss = torch.empty((), device=dev, dtype=torch.float32)
+            loss64 = coef[-1]
+            _call("moe_amd_seq_aux_loss", _ptr_array([ps[i] for i in at]),
+                  _ptr_array([sels[i] for i in at]), n, _dtype_code(dt), T, E, top_k, batch_size,
+                  num_experts / (top_k * S), 1.0 / (L * batch_size * S), 1.0 / (L * batch_size),
+                  ws.data_ptr(), nbytes, coef.data_ptr(), loss64.data_ptr(), loss.data_ptr(),
+                  _stream(ps[at[0]]))
+            ctx.groups.append((at, [ps[i] for i in at], coef))
+            total = loss64 if total is None else total + loss64
         ctx.batch_size = batch_size
-        return (total / L).to(torch.float32)
+        ctx.dtypes = [g.dtype for g in layers]
+        return loss if len(ctx.groups) == 1 else total.to(torch.float32)
 
     @staticmethod
     @on_tensor_device
     def backward(ctx, g):
-        grads = []
-        for s, coef, dt in ctx.saved:
-            T, E = s.shape
-            c = _contig(coef * g.to(torch.float64))
-            out = torch.empty(T, E, device=s.device, dtype=s.dtype)
-            _call("moe_amd_seq_aux_backward", s.data_ptr(), _dtype_code(s.dtype), c.data_ptr(),
-                  T, E, ctx.batch_size, out.data_ptr(), _stream(s))
-            grads.append(out.to(dt))
-        ctx.saved = None
+        grads: list = [None] * len(ctx.dtypes)
+        g = _contig(g.to(torch.float32))
+        for at, ps, coef in ctx.groups:
+            T, E = ps[0].shape
+            outs = [torch.empty_like(s) for s in ps]
+            _call("moe_amd_seq_aux_loss_backward", _ptr_array(ps), len(ps),
+                  _dtype_code(ps[0].dtype), coef.data_ptr(), g.data_ptr(), T, E, ctx.batch_size,
+                  _ptr_array(outs), _stream(ps[0]))
+            for i, out in zip(at, outs):
+                grads[i] = out if out.dtype == ctx.dtypes[i] else out.to(ctx.dtypes[i])
+        ctx.groups = None
         return (None, None, None, None, *grads)
 
 

@@ -12,6 +12,14 @@
 //                   134-166), and its backward through the normalisation
 //   switch_aux_bwd  the Switch loss gradient, a per-expert coefficient times
 //                   a per-token weight
+//   seq_aux_loss, switch_aux_loss   either loss of a whole model: the same
+//                   passes over all layers at once, and the assembly of the
+//                   scalar.  A layer by itself is 8 MB (T = 16384, E = 128),
+//                   too little for the chip and less than its launches cost;
+//                   16 layers one by one, with ten small tensor operators
+//                   each, took 1.33 ms; together 0.27 ms, of it 90 us on the
+//                   GPU (statistics 34, gradients 46 us for 270 MB read and
+//                   134 MB written) and the rest the caller's host time
 //   update_biases   the aux-loss-free expert-bias update of every router in
 //                   one launch (train.py:79-139)
 //
@@ -26,7 +34,16 @@ namespace {
 
 constexpr int kWaves = 4;
 constexpr int kTokensPerWave = 8;  // topk_stats: tokens per wave (grid sizing)
-constexpr int kSeqChunk = 64;      // seq_stats: tokens per block
+constexpr int kSeqChunk = 64;      // seq_stats: tokens per block (one layer)
+constexpr int kMaxLayers = 32;     // layers per launch of the whole-model passes
+
+// The layers' tensors of one launch, by value in the kernel's arguments (no
+// pointer array to copy to the device).
+struct Layers {
+  const void* in[kMaxLayers];        // probabilities or scores [T,E]
+  const int64_t* sel[kMaxLayers];    // routed indices [T,K] (seq; may be null)
+  void* out[kMaxLayers];             // gradients
+};
 
 __device__ __forceinline__ float load_val(const void* p, int dtype, int64_t i) {
   return dtype == MOE_DTYPE_BF16 ? bf2f(((const bf16*)p)[i]) : ((const float*)p)[i];
@@ -65,9 +82,11 @@ __device__ void block_combine(const float (&acc)[NV], int E, float* buf, float* 
 // LDS ([groups][E] floats, dynamic shared memory).
 template <int G, int V>
 __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
-    const void* __restrict__ probs, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
+    Layers layers, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
     int K, float* __restrict__ part_cnt, float* __restrict__ part_sum,
     double* __restrict__ part_margin) {
+  const void* const __restrict__ probs = layers.in[blockIdx.y];
+  const size_t part = (size_t)blockIdx.y * gridDim.x + blockIdx.x;  // this block's partials
   constexpr int TPW = 64 / G, ROWS = kWaves * TPW;
   extern __shared__ float sbuf[];  // [ROWS][E]
   __shared__ double msh[ROWS], mmn[ROWS];
@@ -158,8 +177,9 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
       out[e] = s;
     }
   };
-  combine(cnt, part_cnt + (size_t)blockIdx.x * E);
-  combine(psum, part_sum + (size_t)blockIdx.x * E);
+  combine(cnt, part_cnt + part * E);
+  combine(psum, part_sum + part * E);
+  if (!part_margin) return;
   if (g == 0) {
     msh[row] = msum;
     mmn[row] = (double)mmin;
@@ -180,9 +200,11 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
 // counts [E], weighted probability sums [E], and the margin sum and minimum.
 template <int NV>
 __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
-    const void* __restrict__ probs, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
+    Layers layers, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
     int K, float* __restrict__ part_cnt, float* __restrict__ part_sum,
     double* __restrict__ part_margin) {
+  const void* const __restrict__ probs = layers.in[blockIdx.y];
+  const size_t part = (size_t)blockIdx.y * gridDim.x + blockIdx.x;  // this block's partials
   __shared__ float buf[kWaves * 64];
   __shared__ double mbuf[kWaves * 2];
   const int lane = threadIdx.x & 63;
@@ -231,8 +253,9 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
       mmin = fminf(mmin, m);
     }
   }
-  block_combine<NV>(cnt, E, buf, part_cnt + (size_t)blockIdx.x * E);
-  block_combine<NV>(psum, E, buf, part_sum + (size_t)blockIdx.x * E);
+  block_combine<NV>(cnt, E, buf, part_cnt + part * E);
+  block_combine<NV>(psum, E, buf, part_sum + part * E);
+  if (!part_margin) return;
   if (lane == 0) {
     mbuf[wid * 2] = msum;
     mbuf[wid * 2 + 1] = (double)mmin;
@@ -292,57 +315,76 @@ __global__ __launch_bounds__(64) void topk_stats_finalize_kernel(
   }
 }
 
-// Block (c, b): tokens [c*kSeqChunk, ...) of sequence b.  Normalised scores
+// Block (c, b, l): tokens [c*chunk, ...) of sequence b of layer l.  Normalised scores
 // s' = s / (sum s + 1e-20) per token; per block the selection counts of the
 // sequence's experts (the routed indices if given, else the top-k of s') and
 // the sums of s'.
 // seq_stats with G lanes per token (as topk_stats_group_kernel): block
-// (chunk c, sequence b) covers kSeqChunk tokens; the partial is the sum over
+// (chunk c, sequence b, layer l) covers chunk tokens; the partial is the sum over
 // the block's token groups in group order through LDS.
+// Lane g of a group holds experts (q*G + g)*4 + h in entry 4q + h, so that a
+// row moves as whole 128- or 256-byte pieces (with V consecutive experts per
+// lane the gradient's stores were 16 bytes in every 64: 218 us against 46).  Given indices are counted in
+// LDS (integers: any order), the top-k of s' in registers.
+template <int G>
+__device__ __forceinline__ int expert_of(int g, int j) { return ((j >> 2) * G + g) * 4 + (j & 3); }
+
+// Entries of one row (E == G*V, aligned) as 16-byte (fp32) or 8-byte vectors.
+template <int G, int V>
+__device__ __forceinline__ void load_row(const void* row0, int dtype, int64_t t, int g,
+                                         float (&v)[V]) {
+#pragma unroll
+  for (int q = 0; q < V / 4; ++q) {
+    const int64_t at = t * (G * V) + (q * G + g) * 4;
+    if (dtype == MOE_DTYPE_F32) {
+      const f32x4 a = *(const f32x4*)((const float*)row0 + at);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) v[4 * q + h] = a[h];
+    } else {
+      const u32x2 a = *(const u32x2*)((const bf16*)row0 + at);
+#pragma unroll
+      for (int h = 0; h < 4; ++h) v[4 * q + h] = (h & 1) ? bf_hi(a[h >> 1]) : bf_lo(a[h >> 1]);
+    }
+  }
+}
+
 template <int G, int V>
 __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
-    const void* __restrict__ scores, int dtype, const int64_t* __restrict__ selected, int64_t S,
-    int E, int K, float* __restrict__ part_cnt, float* __restrict__ part_sum) {
+    Layers layers, int dtype, int64_t S, int chunk, int E, int K, float* __restrict__ part_cnt,
+    float* __restrict__ part_sum) {
+  const void* const __restrict__ scores = layers.in[blockIdx.z];
+  const int64_t* const __restrict__ selected = layers.sel[blockIdx.z];
   constexpr int TPW = 64 / G, ROWS = kWaves * TPW;
-  extern __shared__ float sbuf[];  // [ROWS][E]
+  extern __shared__ float sbuf[];  // [ROWS][E], then int counts [E]
+  int* const hist = (int*)(sbuf + ROWS * E);
   const int lane = threadIdx.x & 63, g = lane & (G - 1), sub = lane / G;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row = wid * TPW + sub, e0 = g * V;
+  const int row = wid * TPW + sub;
   const int b = blockIdx.y, c = blockIdx.x;
-  const bool vec = E == G * V && (dtype == MOE_DTYPE_F32 ? V % 4 == 0 : V % 8 == 0) &&
-                   (((uintptr_t)scores & 15) == 0);
+  const bool vec = E == G * V && (((uintptr_t)scores & 15) == 0);
   float cnt[V], psum[V];
 #pragma unroll
   for (int j = 0; j < V; ++j) cnt[j] = psum[j] = 0.f;
-  const int64_t s0 = (int64_t)c * kSeqChunk;
-  const int64_t s1 = s0 + kSeqChunk < S ? s0 + kSeqChunk : S;
+  if (selected) {
+    for (int e = threadIdx.x; e < E; e += blockDim.x) hist[e] = 0;
+    __syncthreads();
+  }
+  const int64_t s0 = (int64_t)c * chunk;
+  const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
   for (int64_t sb = s0 + (int64_t)wid * TPW; sb < s1; sb += kWaves * TPW) {
     const int64_t st = sb + sub;
     const bool tok = st < s1;
     const int64_t t = (int64_t)b * S + (tok ? st : s1 - 1);
+    const int64_t ek = (selected && tok && g < K) ? selected[t * K + g] : -1;
     float v[V];
     if (vec) {
-      if (dtype == MOE_DTYPE_F32) {
-        const f32x4* src = (const f32x4*)((const float*)scores + t * E + e0);
-#pragma unroll
-        for (int q = 0; q < V / 4; ++q) {
-          const f32x4 a = src[q];
-#pragma unroll
-          for (int h = 0; h < 4; ++h) v[4 * q + h] = a[h];
-        }
-      } else {
-        const u32x4* src = (const u32x4*)((const bf16*)scores + t * E + e0);
-#pragma unroll
-        for (int q = 0; q < (V + 7) / 8; ++q) {
-          const u32x4 a = src[q];
-#pragma unroll
-          for (int h = 0; h < 8; ++h)
-            if (8 * q + h < V) v[8 * q + h] = (h & 1) ? bf_hi(a[h >> 1]) : bf_lo(a[h >> 1]);
-        }
-      }
+      load_row<G, V>(scores, dtype, t, g, v);
     } else {
 #pragma unroll
-      for (int j = 0; j < V; ++j) v[j] = e0 + j < E ? load_val(scores, dtype, t * E + e0 + j) : 0.f;
+      for (int j = 0; j < V; ++j) {
+        const int e = expert_of<G>(g, j);
+        v[j] = e < E ? load_val(scores, dtype, t * E + e) : 0.f;
+      }
     }
     float rs = 0.f;
 #pragma unroll
@@ -351,19 +393,17 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       v[j] = v[j] / rs;
-      if (tok && e0 + j < E) psum[j] += v[j];
+      if (tok) psum[j] += v[j];  // entries past E are zero
     }
     if (selected) {
-      for (int k = 0; k < K; ++k) {
-        const int64_t ek = selected[t * K + k];
-#pragma unroll
-        for (int j = 0; j < V; ++j)
-          if (tok && ek == e0 + j) cnt[j] += 1.f;
-      }
+      if (ek >= 0 && ek < E) atomicAdd(&hist[ek], 1);
     } else {
       uint64_t key[V];
 #pragma unroll
-      for (int j = 0; j < V; ++j) key[j] = e0 + j < E ? rank_key(v[j], e0 + j) : 0ull;
+      for (int j = 0; j < V; ++j) {
+        const int e = expert_of<G>(g, j);
+        key[j] = e < E ? rank_key(v[j], e) : 0ull;
+      }
       for (int k = 0; k < K; ++k) {
         uint64_t m = key[0];
 #pragma unroll
@@ -375,16 +415,16 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
       if (tok) {
 #pragma unroll
         for (int j = 0; j < V; ++j)
-          if (e0 + j < E && key[j] == 0ull) cnt[j] += 1.f;  // selected (real keys are never 0)
+          if (expert_of<G>(g, j) < E && key[j] == 0ull) cnt[j] += 1.f;  // selected (real keys are never 0)
       }
     }
   }
-  const size_t slot = ((size_t)b * gridDim.x + c) * E;
+  const size_t slot = (((size_t)blockIdx.z * gridDim.y + b) * gridDim.x + c) * E;
   auto combine = [&](const float (&acc)[V], float* out) {
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < V; ++j)
-      if (e0 + j < E) sbuf[row * E + e0 + j] = acc[j];
+      if (expert_of<G>(g, j) < E) sbuf[row * E + expert_of<G>(g, j)] = acc[j];
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
       float sm = 0.f;
@@ -392,14 +432,20 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
       out[e] = sm;
     }
   };
-  combine(cnt, part_cnt + slot);
-  combine(psum, part_sum + slot);
+  combine(psum, part_sum + slot);  // (its barriers come after every count)
+  if (selected) {
+    for (int e = threadIdx.x; e < E; e += blockDim.x) part_cnt[slot + e] = (float)hist[e];
+  } else {
+    combine(cnt, part_cnt + slot);
+  }
 }
 
 template <int NV>
 __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
-    const void* __restrict__ scores, int dtype, const int64_t* __restrict__ selected, int64_t S,
-    int E, int K, float* __restrict__ part_cnt, float* __restrict__ part_sum) {
+    Layers layers, int dtype, int64_t S, int chunk, int E, int K, float* __restrict__ part_cnt,
+    float* __restrict__ part_sum) {
+  const void* const __restrict__ scores = layers.in[blockIdx.z];
+  const int64_t* const __restrict__ selected = layers.sel[blockIdx.z];
   __shared__ float buf[kWaves * 64];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -407,8 +453,8 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
   float cnt[NV], psum[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.f;
-  const int64_t s0 = (int64_t)c * kSeqChunk;
-  const int64_t s1 = s0 + kSeqChunk < S ? s0 + kSeqChunk : S;
+  const int64_t s0 = (int64_t)c * chunk;
+  const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
   for (int64_t st = s0 + wid; st < s1; st += kWaves) {
     const int64_t t = (int64_t)b * S + st;
     float v[NV];
@@ -453,7 +499,7 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
         if (((taken & ~pad) >> j) & 1ull) cnt[j] += 1.f;
     }
   }
-  const size_t slot = ((size_t)b * gridDim.x + c) * E;
+  const size_t slot = (((size_t)blockIdx.z * gridDim.y + b) * gridDim.x + c) * E;
   block_combine<NV>(cnt, E, buf, part_cnt + slot);
   block_combine<NV>(psum, E, buf, part_sum + slot);
 }
@@ -480,12 +526,174 @@ __global__ __launch_bounds__(64) void seq_stats_finalize_kernel(
   }
 }
 
+// Sum of one fp64 value per thread over a block of 256 or 1024 threads, in a
+// fixed order; every thread gets it.  tmp: 17 doubles of LDS.
+__device__ double block_sum_f64(double v, double* tmp) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  v = wave_sum_f64(v);
+  __syncthreads();
+  if (lane == 0) tmp[wid] = v;
+  __syncthreads();
+  double s = 0.0;
+  for (int w = 0; w < nw; ++w) s += tmp[w];
+  return s;
+}
+
+// Sequence-wise loss, block (b, l): per expert, its selections c and the sum
+// of its normalised scores over the sequence's chunks (in chunk order, a
+// thread per expert: rows of partials are read whole), f = c * f_scale, the
+// gradient coefficient coef[l][b][e] = f * coef_scale, and the block's part
+// sum_e f * mean score of the loss.
+__global__ __launch_bounds__(256) void seq_loss_finalize_kernel(
+    const float* __restrict__ part_cnt, const float* __restrict__ part_sum, int nchunk, int E,
+    int64_t S, double f_scale, double coef_scale, double* __restrict__ coef,
+    double* __restrict__ part_loss) {
+  __shared__ double tmp[17];
+  const size_t lb = (size_t)blockIdx.y * gridDim.x + blockIdx.x;
+  double loss = 0.0;
+  for (int e = threadIdx.x; e < E; e += 256) {
+    double c = 0.0, s = 0.0;
+    const float* pc = part_cnt + lb * nchunk * E + e;
+    const float* ps = part_sum + lb * nchunk * E + e;
+#pragma unroll 8
+    for (int k = 0; k < nchunk; ++k) {
+      c += (double)pc[(size_t)k * E];
+      s += (double)ps[(size_t)k * E];
+    }
+    const double f = c * f_scale;
+    coef[lb * E + e] = f * coef_scale;
+    loss += f * (s / (double)S);
+  }
+  loss = block_sum_f64(loss, tmp);
+  if (threadIdx.x == 0) part_loss[lb] = loss;
+}
+
+// loss = scale * sum of n parts, in a fixed order.
+__global__ __launch_bounds__(256) void loss_sum_kernel(const double* __restrict__ part, int n,
+                                                       double scale, double* __restrict__ loss64,
+                                                       float* __restrict__ loss) {
+  __shared__ double tmp[17];
+  double s = 0.0;
+  for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+  s = block_sum_f64(s, tmp);
+  if (threadIdx.x == 0) {
+    *loss64 = s * scale;
+    *loss = (float)(s * scale);
+  }
+}
+
+// Switch loss, one block per layer: the layer's counts and sums from its
+// blocks' partials (sums64: [L][2][E]); 64 experts at a time, the 16 waves
+// take the partials in turn and are added in wave order.
+__global__ __launch_bounds__(1024) void switch_layer_sums_kernel(
+    const float* __restrict__ part_cnt, const float* __restrict__ part_sum, int nblk, int E,
+    double* __restrict__ sums64) {
+  __shared__ double red[2][16][64];
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const size_t base = (size_t)blockIdx.x * nblk * E;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane;
+    double c = 0.0, s = 0.0;
+    if (e < E)
+#pragma unroll 4
+      for (int k = wid; k < nblk; k += 16) {
+        c += (double)part_cnt[base + (size_t)k * E + e];
+        s += (double)part_sum[base + (size_t)k * E + e];
+      }
+    __syncthreads();
+    red[0][wid][lane] = c;
+    red[1][wid][lane] = s;
+    __syncthreads();
+    if (wid < 2 && e < E) {
+      double v = 0.0;
+      for (int w = 0; w < 16; ++w) v += red[wid][w][lane];
+      sums64[((size_t)blockIdx.x * 2 + wid) * E + e] = v;
+    }
+  }
+}
+
+// ... and the loss E * sum_e (counts / d) (sums / d) with the gradient
+// coefficients coef[e] = counts / d * num_experts / d; d = denom, or
+// denom * *denom_dev.
+__global__ __launch_bounds__(1024) void switch_loss_kernel(
+    const double* __restrict__ sums64, int L, int E, double num_experts, double denom,
+    const double* __restrict__ denom_dev, double* __restrict__ coef, double* __restrict__ loss) {
+  __shared__ double tmp[17];
+  const double d = denom_dev ? denom * *denom_dev : denom;
+  double acc = 0.0;
+  for (int e = threadIdx.x; e < E; e += 1024) {
+    double c = 0.0, s = 0.0;
+    for (int l = 0; l < L; ++l) {
+      c += sums64[((size_t)l * 2) * E + e];
+      s += sums64[((size_t)l * 2 + 1) * E + e];
+    }
+    const double tpe = c / d;
+    coef[e] = tpe * (num_experts / d);
+    acc += tpe * (s / d);
+  }
+  acc = block_sum_f64(acc, tmp);
+  if (threadIdx.x == 0) *loss = acc * num_experts;
+}
+
+// Gradient of the sequence-wise loss with G lanes per token (E == G*V), all
+// layers in one launch: block (c, b, l) holds its lanes' coefficients of
+// sequence b in registers and streams tokens [c*chunk, ...) through 16-byte
+// vectors.  The arithmetic of seq_aux_bwd_kernel, sums over the G lanes in
+// the group's butterfly order.
+template <int G, int V>
+__global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_group_kernel(
+    Layers layers, int dtype, const double* __restrict__ coef, const float* __restrict__ grad,
+    int64_t S, int chunk) {
+  constexpr int TPW = 64 / G, E = G * V;
+  const int lane = threadIdx.x & 63, g = lane & (G - 1), sub = lane / G;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int b = blockIdx.y;
+  const void* const __restrict__ scores = layers.in[blockIdx.z];
+  void* const __restrict__ out = layers.out[blockIdx.z];
+  const double up = grad ? (double)*grad : 1.0;
+  float gc[V];
+#pragma unroll
+  for (int j = 0; j < V; ++j)
+    gc[j] = (float)(coef[((size_t)blockIdx.z * gridDim.y + b) * E + expert_of<G>(g, j)] * up);
+  const int64_t s0 = (int64_t)blockIdx.x * chunk;
+  const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
+  for (int64_t sb = s0 + (int64_t)wid * TPW; sb < s1; sb += kWaves * TPW) {
+    const int64_t st = sb + sub;
+    const bool tok = st < s1;
+    const int64_t t = (int64_t)b * S + (tok ? st : s1 - 1);
+    float v[V];
+    load_row<G, V>(scores, dtype, t, g, v);
+    float rs = 0.f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) rs += v[j];
+    rs = group_sum<G>(rs) + 1e-20f;
+    float dot = 0.f;
+#pragma unroll
+    for (int j = 0; j < V; ++j) dot += gc[j] * (v[j] / rs);
+    dot = group_sum<G>(dot);
+    if (!tok) continue;
+#pragma unroll
+    for (int q = 0; q < V / 4; ++q) {
+      float d[4];
+#pragma unroll
+      for (int h = 0; h < 4; ++h) d[h] = (gc[4 * q + h] - dot) / rs;
+      const int64_t at = t * E + (q * G + g) * 4;
+      if (dtype == MOE_DTYPE_F32) *(f32x4*)((float*)out + at) = f32x4{d[0], d[1], d[2], d[3]};
+      else *(u32x2*)((bf16*)out + at) = u32x2{pack_bf2(d[0], d[1]), pack_bf2(d[2], d[3])};
+    }
+  }
+}
+
 // d s from d s' through s' = s / (sum s + eps): (g - <g, s'>) / (sum s + eps),
-// with g[t][e] = coef[b(t)][e].
+// with g[t][e] = coef[l][b(t)][e] (times *grad when given), layer l = blockIdx.y.
 template <int NV>
 __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_kernel(
-    const void* __restrict__ scores, int dtype, const double* __restrict__ coef, int64_t T,
-    int64_t S, int E, void* __restrict__ d_scores) {
+    Layers layers, int dtype, const double* __restrict__ coef_all, const float* __restrict__ grad,
+    int64_t T, int64_t S, int E) {
+  const void* const __restrict__ scores = layers.in[blockIdx.y];
+  void* const __restrict__ d_scores = layers.out[blockIdx.y];
+  const double* const __restrict__ coef = coef_all + (size_t)blockIdx.y * (T / S) * E;
+  const double up = grad ? (double)*grad : 1.0;
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t nwaves = (int64_t)gridDim.x * kWaves;
@@ -497,7 +705,7 @@ __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_kernel(
     for (int j = 0; j < NV; ++j) {
       const int e = j * 64 + lane;
       v[j] = e < E ? load_val(scores, dtype, t * E + e) : 0.f;
-      g[j] = e < E ? (float)coef[b * E + e] : 0.f;
+      g[j] = e < E ? (float)(coef[b * E + e] * up) : 0.f;
       rs += v[j];
     }
     rs = wave_sum(rs) + 1e-20f;
@@ -517,17 +725,44 @@ __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_kernel(
   }
 }
 
-// grad[t][e] = coef[e] * (w ? w[t] : 1).
+// grad[t][e] = coef[e] * *up * (w ? w[t] : 1), four experts at a time (E % 4
+// == 0), all layers in one launch.
+__global__ __launch_bounds__(256) void switch_aux_bwd_vec_kernel(Layers layers,
+                                                                 const double* __restrict__ coef,
+                                                                 const float* __restrict__ up,
+                                                                 const float* __restrict__ tok_w,
+                                                                 int64_t T, int E, int dtype) {
+  void* const __restrict__ grad = layers.out[blockIdx.y];
+  const int q = E / 4;
+  const double u = (double)*up;
+  const int64_t stride = (int64_t)gridDim.x * 256;
+  const int64_t n = T * (int64_t)q;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) {
+    const int64_t t = i / q;
+    const int e = (int)(i - t * q) * 4;
+    const float w = tok_w ? tok_w[t] : 1.f;
+    float g[4];
+#pragma unroll
+    for (int h = 0; h < 4; ++h) g[h] = (float)(coef[e + h] * u) * w;
+    if (dtype == MOE_DTYPE_BF16)
+      ((u32x2*)grad)[i] = u32x2{pack_bf2(g[0], g[1]), pack_bf2(g[2], g[3])};
+    else __builtin_nontemporal_store(f32x4{g[0], g[1], g[2], g[3]}, (f32x4*)grad + i);
+  }
+}
+
+// The same of one layer, any E.
 __global__ __launch_bounds__(256) void switch_aux_bwd_kernel(const double* __restrict__ coef,
+                                                             const float* __restrict__ up,
                                                              const float* __restrict__ tok_w,
                                                              int64_t T, int E, int dtype,
                                                              void* __restrict__ grad) {
+  const double u = up ? (double)*up : 1.0;
   const int64_t n = T * (int64_t)E;
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int64_t t = i / E;
     const int e = (int)(i - t * E);
-    const float g = (float)coef[e] * (tok_w ? tok_w[t] : 1.f);
+    const float g = (float)(coef[e] * u) * (tok_w ? tok_w[t] : 1.f);
     if (dtype == MOE_DTYPE_BF16) ((bf16*)grad)[i] = f2bf(g);
     else ((float*)grad)[i] = g;
   }
@@ -650,6 +885,92 @@ int check_stats_shape(int64_t T, int E, int K, int dtype, const char* who) {
 
 size_t seq_chunks(int64_t S) { return (size_t)((S + kSeqChunk - 1) / kSeqChunk); }
 
+// topk_stats of layers, nb blocks each (partials [layer][block][E]).
+void launch_topk_stats(const Layers& layers, int nl, int dtype, const float* token_weights,
+                       int64_t T, int E, int K, int nb, float* pc, float* ps, double* pm,
+                       hipStream_t st) {
+  int G, V;
+  group_shape(E, K, G, V);
+  const dim3 grid(nb, nl);
+  if (G) {
+    const size_t shm = (size_t)kWaves * (64 / G) * E * sizeof(float);
+#define MOE_STATS_GROUP(G_, V_)                                                               \
+  topk_stats_group_kernel<G_, V_><<<grid, 64 * kWaves, shm, st>>>(layers, dtype, token_weights, \
+                                                                  T, E, K, pc, ps, pm)
+    if (G == 8 && V == 4) MOE_STATS_GROUP(8, 4);
+    else if (G == 8 && V == 8) MOE_STATS_GROUP(8, 8);
+    else if (G == 8) MOE_STATS_GROUP(8, 16);
+    else if (V == 4) MOE_STATS_GROUP(16, 4);
+    else if (V == 8) MOE_STATS_GROUP(16, 8);
+    else MOE_STATS_GROUP(16, 16);
+#undef MOE_STATS_GROUP
+  } else {
+    MOE_DISPATCH_NV_B(E, topk_stats_kernel, grid, 64 * kWaves, 0, st>>>(
+        layers, dtype, token_weights, T, E, K, pc, ps, pm));
+  }
+}
+
+// seq_stats of nl layers, nc chunks of `chunk` tokens per sequence (partials
+// [layer][sequence][chunk][E]).
+void launch_seq_stats(const Layers& layers, int nl, int dtype, int64_t S, int B, int nc, int chunk,
+                      int E, int K, float* pc, float* ps, hipStream_t st) {
+  int G, V;
+  group_shape(E, K, G, V);
+  const dim3 grid(nc, B, nl);
+  if (G) {
+    const size_t shm = ((size_t)kWaves * (64 / G) + 1) * E * sizeof(float);
+#define MOE_SEQ_GROUP(G_, V_)                                                               \
+  seq_stats_group_kernel<G_, V_><<<grid, 64 * kWaves, shm, st>>>(layers, dtype, S, chunk, E, K, \
+                                                                 pc, ps)
+    if (G == 8 && V == 4) MOE_SEQ_GROUP(8, 4);
+    else if (G == 8 && V == 8) MOE_SEQ_GROUP(8, 8);
+    else if (G == 8) MOE_SEQ_GROUP(8, 16);
+    else if (V == 4) MOE_SEQ_GROUP(16, 4);
+    else if (V == 8) MOE_SEQ_GROUP(16, 8);
+    else MOE_SEQ_GROUP(16, 16);
+#undef MOE_SEQ_GROUP
+  } else {
+    MOE_DISPATCH_NV_B(E, seq_stats_kernel, grid, 64 * kWaves, 0, st>>>(layers, dtype, S, chunk, E,
+                                                                      K, pc, ps));
+  }
+}
+
+// Gradient of the sequence-wise loss of nl layers; every tensor 16-byte
+// aligned (vec) takes the group kernel where E fills the lanes.
+void launch_seq_bwd(const Layers& layers, int nl, bool vec, int dtype, const double* coef,
+                    const float* grad, int64_t T, int E, int B, hipStream_t st) {
+  const int64_t S = T / B;
+  // 256 tokens per block; 64 while that leaves the chip short of blocks
+  const int chunk = (S + 255) / 256 * B * nl >= 1024 ? 256 : 64;
+  const dim3 grid((unsigned)((S + chunk - 1) / chunk), B, nl);
+#define MOE_SEQ_BWD(G_, V_)                                                                     \
+  seq_aux_bwd_group_kernel<G_, V_><<<grid, 64 * kWaves, 0, st>>>(layers, dtype, coef, grad, S, \
+                                                                 chunk)
+  if (vec && B < 65536 && E == 128) MOE_SEQ_BWD(8, 16);
+  else if (vec && B < 65536 && E == 64) MOE_SEQ_BWD(8, 8);
+  else if (vec && B < 65536 && E == 32) MOE_SEQ_BWD(8, 4);
+  else if (vec && B < 65536 && E == 256) MOE_SEQ_BWD(16, 16);
+  else {
+    int64_t nb = (T + kWaves * 8 - 1) / (kWaves * 8);
+    if (nb > 4096) nb = 4096;
+    MOE_DISPATCH_NV_B(E, seq_aux_bwd_kernel, dim3((unsigned)nb, nl), 64 * kWaves, 0,
+                      st>>>(layers, dtype, coef, grad, T, S, E));
+  }
+#undef MOE_SEQ_BWD
+}
+
+// Tokens per block of the whole-model sequence statistics: 256 (a block's
+// combine costs as much as 100 tokens), 64 while that leaves the chip short of
+// blocks.
+int seq_loss_chunk(int L, int64_t S, int B) {
+  return (S + 255) / 256 * B * L >= 1024 ? 256 : kSeqChunk;
+}
+// Blocks per layer of the whole-model top-k statistics.
+int switch_blocks(int L, int64_t T) {
+  const int nb = stats_blocks(T), most = 2048 / L > 16 ? 2048 / L : 16;
+  return nb < most ? nb : most;
+}
+
 }  // namespace
 }  // namespace moe
 
@@ -683,25 +1004,9 @@ extern "C" int moe_amd_topk_stats(const void* probs, int probs_dtype, const floa
     topk_stats_finalize_kernel<<<E + 1, 64, 0, st>>>(pc, ps, pm, 0, E, counts, prob_sums, margin);
     return check_launch(who);
   }
-  int G, V;
-  group_shape(E, K, G, V);
-  if (G) {
-    const size_t shm = (size_t)kWaves * (64 / G) * E * sizeof(float);
-#define MOE_STATS_GROUP(G_, V_)                                                        \
-  topk_stats_group_kernel<G_, V_><<<nb, 64 * kWaves, shm, st>>>(probs, probs_dtype,     \
-                                                                token_weights, T, E, K, \
-                                                                pc, ps, pm)
-    if (G == 8 && V == 4) MOE_STATS_GROUP(8, 4);
-    else if (G == 8 && V == 8) MOE_STATS_GROUP(8, 8);
-    else if (G == 8) MOE_STATS_GROUP(8, 16);
-    else if (V == 4) MOE_STATS_GROUP(16, 4);
-    else if (V == 8) MOE_STATS_GROUP(16, 8);
-    else MOE_STATS_GROUP(16, 16);
-#undef MOE_STATS_GROUP
-  } else {
-    MOE_DISPATCH_NV_B(E, topk_stats_kernel, nb, 64 * kWaves, 0, st>>>(
-        probs, probs_dtype, token_weights, T, E, K, pc, ps, pm));
-  }
+  Layers layers{};
+  layers.in[0] = probs;
+  launch_topk_stats(layers, 1, probs_dtype, token_weights, T, E, K, nb, pc, ps, pm, st);
   topk_stats_finalize_kernel<<<E + 1, 64, 0, st>>>(pc, ps, pm, nb, E, counts, prob_sums, margin);
   return check_launch(who);
 }
@@ -732,24 +1037,10 @@ extern "C" int moe_amd_seq_stats(const void* scores, int scores_dtype,
   hipStream_t st = (hipStream_t)stream;
   float* pc = (float*)workspace;
   float* ps = pc + (size_t)B * nc * E;
-  int G, V;
-  group_shape(E, K, G, V);
-  if (G) {
-    const size_t shm = (size_t)kWaves * (64 / G) * E * sizeof(float);
-#define MOE_SEQ_GROUP(G_, V_)                                                                 \
-  seq_stats_group_kernel<G_, V_><<<dim3(nc, B), 64 * kWaves, shm, st>>>(scores, scores_dtype, \
-                                                                        selected, S, E, K, pc, ps)
-    if (G == 8 && V == 4) MOE_SEQ_GROUP(8, 4);
-    else if (G == 8 && V == 8) MOE_SEQ_GROUP(8, 8);
-    else if (G == 8) MOE_SEQ_GROUP(8, 16);
-    else if (V == 4) MOE_SEQ_GROUP(16, 4);
-    else if (V == 8) MOE_SEQ_GROUP(16, 8);
-    else MOE_SEQ_GROUP(16, 16);
-#undef MOE_SEQ_GROUP
-  } else {
-    MOE_DISPATCH_NV_B(E, seq_stats_kernel, dim3(nc, B), 64 * kWaves, 0, st>>>(
-        scores, scores_dtype, selected, S, E, K, pc, ps));
-  }
+  Layers layers{};
+  layers.in[0] = scores;
+  layers.sel[0] = selected;
+  launch_seq_stats(layers, 1, scores_dtype, S, B, nc, kSeqChunk, E, K, pc, ps, st);
   seq_stats_finalize_kernel<<<(unsigned)((int64_t)B * E), 64, 0, st>>>(pc, ps, nc, B, E, S,
                                                                         counts, mean_scores);
   return check_launch(who);
@@ -764,11 +1055,11 @@ extern "C" int moe_amd_seq_aux_backward(const void* scores, int scores_dtype,
   MOE_REQUIRE(B >= 1 && T % B == 0, MOE_ERR_ARG, "%s: T must be a multiple of B", who);
   MOE_REQUIRE(T == 0 || (scores && coef && d_scores), MOE_ERR_ARG, "%s: null pointer", who);
   if (T == 0) return MOE_OK;
-  const int64_t S = T / B;
-  int64_t nb = (T + kWaves * 8 - 1) / (kWaves * 8);
-  if (nb > 4096) nb = 4096;
-  MOE_DISPATCH_NV_B(E, seq_aux_bwd_kernel, (unsigned)nb, 64 * kWaves, 0,
-                    (hipStream_t)stream>>>(scores, scores_dtype, coef, T, S, E, d_scores));
+  Layers layers{};
+  layers.in[0] = scores;
+  layers.out[0] = d_scores;
+  launch_seq_bwd(layers, 1, al16(scores) && al16(d_scores), scores_dtype, coef, nullptr, T, E, B,
+                 (hipStream_t)stream);
   return check_launch(who);
 }
 
@@ -783,8 +1074,162 @@ extern "C" int moe_amd_switch_aux_backward(const double* coef, const float* toke
   if (T == 0) return MOE_OK;
   int64_t nb = (T * (int64_t)E + 255) / 256;
   if (nb > 8192) nb = 8192;
-  switch_aux_bwd_kernel<<<(unsigned)nb, 256, 0, (hipStream_t)stream>>>(coef, token_weights, T, E,
-                                                                      grad_dtype, grad);
+  switch_aux_bwd_kernel<<<(unsigned)nb, 256, 0, (hipStream_t)stream>>>(coef, nullptr, token_weights,
+                                                                      T, E, grad_dtype, grad);
+  return check_launch(who);
+}
+
+extern "C" size_t moe_amd_seq_aux_loss_workspace_size(int L, int64_t T, int E, int B) {
+  if (L < 1 || T < 1 || E < 1 || B < 1 || T % B) return 0;
+  const int64_t S = T / B;
+  const int chunk = seq_loss_chunk(L, S, B);
+  const size_t parts = (size_t)L * B * (size_t)((S + chunk - 1) / chunk) * E;
+  return align_up(parts * 2 * sizeof(float), 16) + ((size_t)L * B + 1) * sizeof(double);
+}
+
+extern "C" int moe_amd_seq_aux_loss(const void* const* scores, const int64_t* const* selected,
+                                    int L, int scores_dtype, int64_t T, int E, int K, int B,
+                                    double f_scale, double coef_scale, double loss_scale,
+                                    void* workspace, size_t workspace_bytes, double* coef,
+                                    double* loss64, float* loss, void* stream) {
+  const char* who = "seq_aux_loss";
+  int rc = check_stats_shape(T, E, K, scores_dtype, who);
+  if (rc) return rc;
+  MOE_REQUIRE(L >= 1 && B >= 1 && T > 0 && T % B == 0, MOE_ERR_ARG,
+              "%s: L=%d layers, T=%lld must be a positive multiple of the batch size %d", who, L,
+              (long long)T, B);
+  MOE_REQUIRE(scores && coef && loss64 && loss, MOE_ERR_ARG, "%s: null pointer", who);
+  for (int l = 0; l < L; ++l) MOE_REQUIRE(scores[l], MOE_ERR_ARG, "%s: layer %d is null", who, l);
+  const size_t need = moe_amd_seq_aux_loss_workspace_size(L, T, E, B);
+  MOE_REQUIRE(workspace && workspace_bytes >= need, MOE_ERR_WORKSPACE,
+              "%s: workspace of %zu bytes needed", who, need);
+  MOE_REQUIRE(((uintptr_t)workspace & 15) == 0, MOE_ERR_ALIGN, "%s: workspace alignment", who);
+  const int64_t S = T / B;
+  const int chunk = seq_loss_chunk(L, S, B);
+  const int64_t nc64 = (S + chunk - 1) / chunk;
+  MOE_REQUIRE(nc64 < 65536 && B < 65536 && L < 65536, MOE_ERR_UNSUPPORTED, "%s: grid too large",
+              who);
+  const int nc = (int)nc64;
+  hipStream_t st = (hipStream_t)stream;
+  const size_t per_layer = (size_t)B * nc * E;
+  float* pc = (float*)workspace;
+  float* ps = pc + (size_t)L * per_layer;
+  double* parts = (double*)((char*)workspace + align_up((size_t)L * per_layer * 2 * sizeof(float), 16));
+  for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
+    const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
+    Layers layers{};
+    for (int l = 0; l < nl; ++l) {
+      layers.in[l] = scores[l0 + l];
+      layers.sel[l] = selected ? selected[l0 + l] : nullptr;
+    }
+    launch_seq_stats(layers, nl, scores_dtype, S, B, nc, chunk, E, K, pc + l0 * per_layer,
+                     ps + l0 * per_layer, st);
+  }
+  seq_loss_finalize_kernel<<<dim3(B, L), 256, 0, st>>>(pc, ps, nc, E, S, f_scale, coef_scale, coef,
+                                                       parts);
+  loss_sum_kernel<<<1, 256, 0, st>>>(parts, L * B, loss_scale, loss64, loss);
+  return check_launch(who);
+}
+
+extern "C" int moe_amd_seq_aux_loss_backward(const void* const* scores, int L, int scores_dtype,
+                                             const double* coef, const float* d_loss, int64_t T,
+                                             int E, int B, void* const* d_scores, void* stream) {
+  const char* who = "seq_aux_loss_backward";
+  int rc = check_stats_shape(T, E, 1, scores_dtype, who);
+  if (rc) return rc;
+  MOE_REQUIRE(L >= 1 && B >= 1 && T % B == 0, MOE_ERR_ARG, "%s: T must be a multiple of B", who);
+  if (T == 0) return MOE_OK;
+  MOE_REQUIRE(scores && coef && d_loss && d_scores, MOE_ERR_ARG, "%s: null pointer", who);
+  for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
+    const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
+    Layers layers{};
+    bool vec = true;
+    for (int l = 0; l < nl; ++l) {
+      MOE_REQUIRE(scores[l0 + l] && d_scores[l0 + l], MOE_ERR_ARG, "%s: layer %d is null", who,
+                  l0 + l);
+      layers.in[l] = scores[l0 + l];
+      layers.out[l] = d_scores[l0 + l];
+      vec = vec && al16(layers.in[l]) && al16(layers.out[l]);
+    }
+    launch_seq_bwd(layers, nl, vec, scores_dtype, coef + (size_t)l0 * B * E, d_loss, T, E, B,
+                   (hipStream_t)stream);
+  }
+  return check_launch(who);
+}
+
+extern "C" size_t moe_amd_switch_aux_loss_workspace_size(int L, int64_t T, int E) {
+  if (L < 1 || T < 1 || E < 1) return 0;
+  return align_up((size_t)L * switch_blocks(L, T) * E * 2 * sizeof(float), 16) +
+         (size_t)L * 2 * E * sizeof(double);
+}
+
+extern "C" int moe_amd_switch_aux_loss(const void* const* probs, int L, int probs_dtype,
+                                       const float* token_weights, int64_t T, int E, int K,
+                                       double num_experts, double denom, const double* denom_dev,
+                                       void* workspace, size_t workspace_bytes, double* coef,
+                                       double* loss, void* stream) {
+  const char* who = "switch_aux_loss";
+  int rc = check_stats_shape(T, E, K, probs_dtype, who);
+  if (rc) return rc;
+  MOE_REQUIRE(L >= 1 && L < 65536 && T > 0, MOE_ERR_ARG, "%s: L=%d layers of T=%lld tokens", who, L,
+              (long long)T);
+  MOE_REQUIRE(probs && coef && loss, MOE_ERR_ARG, "%s: null pointer", who);
+  for (int l = 0; l < L; ++l) MOE_REQUIRE(probs[l], MOE_ERR_ARG, "%s: layer %d is null", who, l);
+  const size_t need = moe_amd_switch_aux_loss_workspace_size(L, T, E);
+  MOE_REQUIRE(workspace && workspace_bytes >= need, MOE_ERR_WORKSPACE,
+              "%s: workspace of %zu bytes needed", who, need);
+  MOE_REQUIRE(((uintptr_t)workspace & 15) == 0, MOE_ERR_ALIGN, "%s: workspace alignment", who);
+  hipStream_t st = (hipStream_t)stream;
+  const int nb = switch_blocks(L, T);
+  const size_t per_layer = (size_t)nb * E;
+  float* pc = (float*)workspace;
+  float* ps = pc + L * per_layer;
+  double* sums = (double*)((char*)workspace + align_up(L * per_layer * 2 * sizeof(float), 16));
+  for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
+    const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
+    Layers layers{};
+    for (int l = 0; l < nl; ++l) layers.in[l] = probs[l0 + l];
+    launch_topk_stats(layers, nl, probs_dtype, token_weights, T, E, K, nb, pc + l0 * per_layer,
+                      ps + l0 * per_layer, nullptr, st);
+  }
+  switch_layer_sums_kernel<<<L, 1024, 0, st>>>(pc, ps, nb, E, sums);
+  switch_loss_kernel<<<1, 1024, 0, st>>>(sums, L, E, num_experts, denom, denom_dev, coef, loss);
+  return check_launch(who);
+}
+
+extern "C" int moe_amd_switch_aux_loss_backward(const double* coef, const float* d_loss,
+                                                const float* token_weights, int L, int64_t T,
+                                                int E, int grad_dtype, void* const* grads,
+                                                void* stream) {
+  const char* who = "switch_aux_loss_backward";
+  MOE_REQUIRE(T >= 0 && E >= 1 && L >= 1, MOE_ERR_ARG, "%s: bad sizes", who);
+  MOE_REQUIRE(grad_dtype == MOE_DTYPE_F32 || grad_dtype == MOE_DTYPE_BF16, MOE_ERR_DTYPE,
+              "%s: dtype %d", who, grad_dtype);
+  if (T == 0) return MOE_OK;
+  MOE_REQUIRE(coef && d_loss && grads, MOE_ERR_ARG, "%s: null pointer", who);
+  hipStream_t st = (hipStream_t)stream;
+  for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
+    const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
+    Layers layers{};
+    bool vec = E % 4 == 0;
+    for (int l = 0; l < nl; ++l) {
+      MOE_REQUIRE(grads[l0 + l], MOE_ERR_ARG, "%s: layer %d is null", who, l0 + l);
+      layers.out[l] = grads[l0 + l];
+      vec = vec && al16(layers.out[l]);
+    }
+    int64_t nb = (T * (int64_t)E + 1023) / 1024;
+    const int64_t most = 8192 / nl;
+    if (nb > most) nb = most;
+    if (vec) {
+      switch_aux_bwd_vec_kernel<<<dim3((unsigned)nb, nl), 256, 0, st>>>(layers, coef, d_loss,
+                                                                       token_weights, T, E,
+                                                                       grad_dtype);
+    } else {
+      for (int l = 0; l < nl; ++l)
+        switch_aux_bwd_kernel<<<(unsigned)nb, 256, 0, st>>>(coef, d_loss, token_weights, T, E,
+                                                            grad_dtype, layers.out[l]);
+    }
+  }
   return check_launch(who);
 }
 

@@ -1,0 +1,99 @@
+"""The load-balancing losses over a model's layers at once: layer counts past
+one launch's 32, layers of two shapes, every gradient kernel (lanes filled or
+not), chunks of 64 and of 256 tokens, ragged sequences, misaligned inputs.
+fp32 data with fp64 sums: loss within 1e-6 of the fp64 oracle, gradients
+within 1e-5 of the largest (the fp32 arithmetic of a token's 16 to 256
+terms); bf16 gradients within their rounding, 2^-8."""
+import pytest
+import torch
+
+from moe_amd import balancing as Bal
+from oracle import balancing_oracle as B
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _layers(shapes, E, dtype, seed, softmax=False):
+    g = torch.Generator().manual_seed(seed)
+    out = []
+    for T in shapes:
+        z = torch.randn(T, E, generator=g)
+        out.append((torch.softmax(z, -1) if softmax else torch.sigmoid(z)).to(dtype))
+    return out, g
+
+
+def _compare(loss, ref, gin, ref_in, dtype):
+    loss.backward()
+    ref_g = torch.autograd.grad(ref, ref_in)
+    torch.cuda.synchronize()
+    assert abs(loss.item() - ref.item()) <= (1e-6 if dtype == torch.float32 else 1e-2) * ref.item()
+    for x, rg in zip(gin, ref_g):
+        lim = (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5) * rg.abs().max()
+        assert (x.grad.double().cpu() - rg).abs().max() <= lim
+
+
+SEQ = [
+    # layers' tokens, sequences, E, K, selected given, dtype
+    ((96,) * 33, 2, 64, 6, True, torch.float32),          # two launches
+    ((520, 520, 260), 2, 128, 8, True, torch.float32),    # layers of two shapes
+    ((2060,) * 3, 4, 128, 4, False, torch.float32),       # 64-token chunks, a ragged last one
+    ((16384,) * 16, 1, 128, 4, True, torch.float32),      # 256-token chunks
+    ((65,) * 2, 1, 32, 2, False, torch.float32),
+    ((300,) * 2, 1, 256, 8, True, torch.bfloat16),
+    ((130,) * 2, 2, 100, 4, False, torch.float32),        # lanes partly empty
+    ((50,) * 2, 1, 1792, 8, False, torch.float32),
+]
+
+
+@pytest.mark.parametrize("shapes,bsz,E,K,given,dtype", SEQ)
+def test_seq_loss_layers(shapes, bsz, E, K, given, dtype):
+    print(f"seq loss {len(shapes)} x {shapes[0]} B={bsz} E={E} {dtype}", flush=True)
+    layers, g = _layers(shapes, E, dtype, sum(shapes) + E)
+    sel = tuple(torch.rand(T, E, generator=g).topk(K, dim=-1).indices for T in shapes)
+    ref_in = [x.double().requires_grad_(True) for x in layers]
+    ref = B.seq_aux_loss(tuple(ref_in), E, K, bsz, sel if given else None)
+    gin = [x.to(DEV).requires_grad_(True) for x in layers]
+    loss = Bal.seq_load_balancing_loss_func(
+        tuple(gin), E, K, batch_size=bsz,
+        selected_experts=tuple(s.to(DEV) for s in sel) if given else None)
+    _compare(loss, ref, gin, ref_in, dtype)
+
+
+SWITCH = [
+    ((96,) * 33, 64, 6, torch.float32, False),
+    ((520, 260), 128, 8, torch.float32, False),
+    ((4096,) * 4, 128, 8, torch.float32, True),
+    ((777,) * 2, 100, 3, torch.float32, True),
+    ((130,) * 2, 63, 4, torch.float32, False),   # E not a multiple of 4
+    ((300,) * 3, 256, 8, torch.bfloat16, False),
+    ((40,) * 2, 1792, 8, torch.float32, False),
+]
+
+
+@pytest.mark.parametrize("shapes,E,K,dtype,masked", SWITCH)
+def test_switch_loss_layers(shapes, E, K, dtype, masked):
+    print(f"switch loss {len(shapes)} x {shapes[0]} E={E} {dtype} masked={masked}", flush=True)
+    layers, g = _layers(shapes, E, dtype, sum(shapes) + E, softmax=True)
+    mask = (torch.rand(1, shapes[0], generator=g) > 0.3).float() if masked else None
+    ref_in = [x.double().requires_grad_(True) for x in layers]
+    ref = B.switch_aux_loss(tuple(ref_in), E, K, attention_mask=mask)
+    gin = [x.to(DEV).requires_grad_(True) for x in layers]
+    loss = Bal.load_balancing_loss_func(tuple(gin), E, K,
+                                        attention_mask=mask.to(DEV) if masked else None)
+    _compare(loss, ref, gin, ref_in, dtype)
+
+
+def test_layers_of_odd_alignment():
+    """Contiguous [T,E] views that start 4 bytes into their storage."""
+    T, E, K = 200, 64, 4
+    layers, _ = _layers((T, T), E, torch.float32, 7)
+    ref_in = [x.double().requires_grad_(True) for x in layers]
+    ref = B.seq_aux_loss(tuple(ref_in), E, K, 1)
+    gin = []
+    for x in layers:
+        v = torch.empty(T * E + 1, device=DEV)[1:].view(T, E)
+        v.copy_(x)
+        gin.append(v.requires_grad_(True))
+    loss = Bal.seq_load_balancing_loss_func(tuple(gin), E, K)
+    _compare(loss, ref, gin, ref_in, torch.float32)
