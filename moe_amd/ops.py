@@ -47,11 +47,13 @@ def _timed(name: str, fn, *args):
 
 
 def _device_of(args, kwargs):
-    for a in (*args, *kwargs.values()):
+    """Index of the device of the first GPU tensor (or plan) among the
+    arguments, or None."""
+    for a in (*args, *kwargs.values()) if kwargs else args:
         if isinstance(a, RoutingPlan):
-            return a.counts.device
+            return a.counts.device.index
         if getattr(a, "is_cuda", False):
-            return a.device
+            return a.device.index
     return None
 
 
@@ -62,9 +64,9 @@ def on_tensor_device(fn):
     @functools.wraps(fn)
     def run(*args, **kwargs):
         dev = _device_of(args, kwargs)
-        if dev is None or dev.index is None or dev.index == torch.cuda.current_device():
+        if dev is None or dev == torch.cuda.current_device():
             return fn(*args, **kwargs)
-        with torch.cuda.device(dev.index):
+        with torch.cuda.device(dev):
             return fn(*args, **kwargs)
     return run
 
@@ -76,7 +78,10 @@ def _call(name: str, *args) -> None:
         # capture (no GPU fault); until that is understood, refuse capture.
         raise RuntimeError(f"moe_amd.{name}: HIP graph capture of the moe_amd kernels is not "
                            "supported; run them eagerly")
-    _timed(name, _lib.call, name, *args)
+    if _events is None:
+        _lib.call(name, *args)
+    else:
+        _timed(name, _lib.call, name, *args)
 
 
 def _ptr(t: torch.Tensor | None) -> int | None:
@@ -84,7 +89,10 @@ def _ptr(t: torch.Tensor | None) -> int | None:
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current stream's handle on t's device.  A launch costs the host
+    about as much as the arguments it is given: torch.cuda.current_stream
+    builds a Stream object for 4 us, this reads the handle."""
+    return torch._C._cuda_getCurrentRawStream(t.device.index)
 
 
 def _dtype_code(dt: torch.dtype) -> int:
