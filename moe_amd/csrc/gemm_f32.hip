@@ -50,7 +50,12 @@
 // of the cycles at 1.83 GHz.  Kernel times at S = 32768 rows, H = 1024, E =
 // 16, I = 768, with the fp32 MFMA -> with the split: F1 935 -> 626, F2 485 ->
 // 304, FDX2 658 -> 368, FDX1 1214 -> 573, FDW2 790 -> 290, FDW1 1453 -> 624 us
-// (84, 106, 78, 85, 65, 71 -> 165, 170, 140, 180, 178, 165 TFLOP/s).  Output: register 4q+c of a lane
+// (84, 106, 78, 85, 65, 71 -> 165, 170, 140, 180, 178, 165 TFLOP/s); the
+// loads of an operand issued as soon as its registers are free, no wait for
+// them at the barriers and the priority of multiplying waves take another 2%
+// (2493 -> 2451 us over the six).  That is 1.1
+// PFLOP/s of bf16 products, what the board's power leaves the bf16 grouped
+// GEMMs too.  Output: register 4q+c of a lane
 // holds (tile row L % 32, tile column 8q + 4(L/32) + c) of the sub-tile (the
 // column operand is MFMA's "A").  Epilogue: 64 rows at a time are staged in
 // LDS (reusing the stage buffer) and written out row by row with 16-byte
@@ -269,15 +274,17 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
       }
     }
   };
-  auto load_stage = [&](int s) {
+  auto load_rows = [&](int s) {
     if constexpr (MODE == F1) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rv[i] = ld4(xrow[i] + s * FBK);
+      for (int i = 0; i < 4; ++i) rv[i] = ld4(xrow[i] + min(s, nk - 1) * FBK);
     } else {
       const auto rr = stage_rsrc(rptr, rleft, rstep, s);
 #pragma unroll
       for (int i = 0; i < 4; ++i) rv[i] = buf4(rr, roff[i]);
     }
+  };
+  auto load_cols = [&](int s) {
     if constexpr (MODE == FDW1) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -322,6 +329,13 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
     }
   };
 
+  // Workgroup barrier over LDS accesses only: __syncthreads would also wait
+  // for the next stage's global loads.
+  auto sync_lds = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
   f32x16 acc[2][2];
   auto zero_acc = [&]() {
 #pragma unroll
@@ -342,12 +356,24 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
       fb[i] = lds_at(wr * 64 + i * 32 + l32, hl);
     }
     load_src(0);
-    load_stage(0);
+    load_rows(0);
+    load_cols(0);
     for (int s = 0; s < nk; ++s) {
+      // An operand's next loads go out as soon as its registers are free, so
+      // they have a barrier, the MFMAs and the other operand's split to land.
+      // (Unconditionally: past the last stage the descriptors are empty, F1
+      // reads its last rows again.  A branch would make every wait a full one.)
+      __builtin_amdgcn_s_setprio(0);
       store_operand(rv, planes, std::integral_constant<bool, ROW_KM>{});
+      __builtin_amdgcn_sched_barrier(0);
+      load_rows(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
       store_operand(cv, planes + kOperand, std::integral_constant<bool, COL_KM>{});
-      __syncthreads();
-      if (s + 1 < nk) load_stage(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      load_cols(s + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_setprio(1);  // multiplying waves issue first (1%)
+      sync_lds();
 #pragma unroll
       for (int kk = 0; kk < 2; ++kk) {
         bf16x8 a[3][2], b[3][2];
@@ -369,7 +395,7 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
               acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]][i], b[TB[t]][j],
                                                                   acc[i][j], 0, 0, 0);
       }
-      __syncthreads();  // the stage is read: the next one may be written
+      sync_lds();  // the stage is read: the next one may be written
     }
     // Non-finite elements: the whole tile again on the fp32 MFMA.
     bool bad = false;
@@ -385,7 +411,8 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
       float* const C = fsm + FBM * FLD;
       load_src(0);
       for (int s = 0; s < nk; ++s) {
-        load_stage(s);
+        load_rows(s);
+        load_cols(s);
         __syncthreads();  // the previous stage is read
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
