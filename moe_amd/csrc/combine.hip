@@ -83,23 +83,24 @@ __global__ __launch_bounds__(64 * kWaves) void combine_kernel(
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int nvalid = offsets[E];
   const int64_t nw = (int64_t)gridDim.x * kWaves;
+  const int hbeg = ((int)blockIdx.y * 64 + lane) * N, hstep = (int)gridDim.y * 64 * N;
   for (int64_t t = (int64_t)blockIdx.x * kWaves + wid; t < ntok; t += nw) {
     if constexpr (KM > 0) {
       int sk[KM];
       float wk[KM];
       token_rows<KM>(slot, w, wdt, t, lane, sk, wk);
       const bool rp = wdt == MOE_DTYPE_BF16 && sizeof(T) == 2;
-      for (int h0 = lane * N; h0 < H; h0 += 64 * N * kChunks) {
+      for (int h0 = hbeg; h0 < H; h0 += hstep * kChunks) {
         typename Vec<T>::Raw v[kChunks][KM];
 #pragma unroll
         for (int c = 0; c < kChunks; ++c)
 #pragma unroll
           for (int k = 0; k < KM; ++k)
-            if (sk[k] < nvalid && h0 + c * 64 * N < H)
-              v[c][k] = Vec<T>::load_raw(y + (int64_t)sk[k] * H + h0 + c * 64 * N);
+            if (sk[k] < nvalid && h0 + c * hstep < H)
+              v[c][k] = Vec<T>::load_raw(y + (int64_t)sk[k] * H + h0 + c * hstep);
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
-          if (h0 + c * 64 * N >= H) break;
+          if (h0 + c * hstep >= H) break;
           float acc[N];
 #pragma unroll
           for (int i = 0; i < N; ++i) acc[i] = 0.f;
@@ -113,11 +114,11 @@ __global__ __launch_bounds__(64 * kWaves) void combine_kernel(
               acc[i] += prod;
             }
           }
-          Vec<T>::store(out + t * H + h0 + c * 64 * N, acc);
+          Vec<T>::store(out + t * H + h0 + c * hstep, acc);
         }
       }
     } else {
-      for (int h0 = lane * N; h0 < H; h0 += 64 * N) {
+      for (int h0 = hbeg; h0 < H; h0 += hstep) {
         float acc[N];
 #pragma unroll
         for (int i = 0; i < N; ++i) acc[i] = 0.f;
@@ -228,24 +229,25 @@ __global__ __launch_bounds__(64 * kWaves) void gather_bwd_kernel(
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int nvalid = offsets[E];
   const int64_t nw = (int64_t)gridDim.x * kWaves;
+  const int hbeg = ((int)blockIdx.y * 64 + lane) * N, hstep = (int)gridDim.y * 64 * N;
   for (int64_t t = (int64_t)blockIdx.x * kWaves + wid; t < ntok; t += nw) {
     int sk[KM > 0 ? KM : 1];
     float wk[KM > 0 ? KM : 1];
     if constexpr (KM > 0) token_rows<KM>(slot, nullptr, 0, t, lane, sk, wk);
     if constexpr (KM > 0) {
-      for (int h0 = lane * N; h0 < H; h0 += 64 * N * kChunks) {
+      for (int h0 = hbeg; h0 < H; h0 += hstep * kChunks) {
         typename Vec<T>::Raw v[kChunks][KM], a[kChunks];
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
-          if (h0 + c * 64 * N >= H) break;
+          if (h0 + c * hstep >= H) break;
 #pragma unroll
           for (int k = 0; k < KM; ++k)
-            if (sk[k] < nvalid) v[c][k] = Vec<T>::load_raw(dxs + (int64_t)sk[k] * H + h0 + c * 64 * N);
-          if (addend) a[c] = Vec<T>::load_raw(addend + t * H + h0 + c * 64 * N);
+            if (sk[k] < nvalid) v[c][k] = Vec<T>::load_raw(dxs + (int64_t)sk[k] * H + h0 + c * hstep);
+          if (addend) a[c] = Vec<T>::load_raw(addend + t * H + h0 + c * hstep);
         }
 #pragma unroll
         for (int c = 0; c < kChunks; ++c) {
-          if (h0 + c * 64 * N >= H) break;
+          if (h0 + c * hstep >= H) break;
           float acc[N];
 #pragma unroll
           for (int i = 0; i < N; ++i) acc[i] = 0.f;
@@ -261,12 +263,12 @@ __global__ __launch_bounds__(64 * kWaves) void gather_bwd_kernel(
 #pragma unroll
             for (int i = 0; i < N; ++i) acc[i] = Vec<T>::round(acc[i]) + Vec<T>::get(a[c], i);
           }
-          Vec<T>::store(dx + t * H + h0 + c * 64 * N, acc);
+          Vec<T>::store(dx + t * H + h0 + c * hstep, acc);
         }
       }
       continue;
     }
-    for (int h0 = lane * N; h0 < H; h0 += 64 * N) {
+    for (int h0 = hbeg; h0 < H; h0 += hstep) {
       float acc[N];
 #pragma unroll
       for (int i = 0; i < N; ++i) acc[i] = 0.f;
@@ -297,6 +299,18 @@ int grid_tokens(int64_t ntok) {
   int64_t b = (ntok + kWaves - 1) / kWaves;
   if (b > 32768) b = 32768;
   return (int)(b < 1 ? 1 : b);
+}
+
+// Combine and gather backward: one wave per token walks the row in pieces of
+// 1 KB, a memory round trip each; while the tokens leave the chip short of
+// waves (256 CUs x 4 SIMDs x 8 = 8192 at once) the pieces go to waves of
+// their own (blockIdx.y).
+template <typename T>
+dim3 grid_rows(int64_t ntok, int H) {
+  const int pieces = (H + 64 * Vec<T>::N - 1) / (64 * Vec<T>::N);
+  const int64_t ny = ntok > 0 ? 16384 / ntok : 1;
+  return dim3((unsigned)grid_tokens(ntok),
+              (unsigned)(ny < 1 ? 1 : (ny < pieces ? ny : pieces)));
 }
 
 int check_rows(int64_t T, int K, int E, int H, int dtype, const char* who) {
@@ -361,10 +375,10 @@ extern "C" int moe_amd_combine(const void* y, const int32_t* slot, const int32_t
   if (T == 0) return MOE_OK;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MOE_DTYPE_BF16)
-    MOE_DISPATCH_K(K, combine_kernel, bf16, grid_tokens(T), 64 * kWaves, 0, st>>>(
+    MOE_DISPATCH_K(K, combine_kernel, bf16, grid_rows<bf16>(T, H), 64 * kWaves, 0, st>>>(
         (const bf16*)y, slot, offsets, topk_weights, weights_dtype, T, K, E, H, (bf16*)out));
   else
-    MOE_DISPATCH_K(K, combine_kernel, float, grid_tokens(T), 64 * kWaves, 0, st>>>(
+    MOE_DISPATCH_K(K, combine_kernel, float, grid_rows<float>(T, H), 64 * kWaves, 0, st>>>(
         (const float*)y, slot, offsets, topk_weights, weights_dtype, T, K, E, H, (float*)out));
   return check_launch(who);
 }
@@ -408,10 +422,10 @@ int gather_backward_impl(const void* d_xs, const int32_t* slot, const int32_t* o
   if (T == 0) return MOE_OK;
   hipStream_t st = (hipStream_t)stream;
   if (dtype == MOE_DTYPE_BF16)
-    MOE_DISPATCH_K(K, gather_bwd_kernel, bf16, grid_tokens(T), 64 * kWaves, 0, st>>>(
+    MOE_DISPATCH_K(K, gather_bwd_kernel, bf16, grid_rows<bf16>(T, H), 64 * kWaves, 0, st>>>(
         (const bf16*)d_xs, slot, offsets, (const bf16*)addend, T, K, E, H, (bf16*)d_x));
   else
-    MOE_DISPATCH_K(K, gather_bwd_kernel, float, grid_tokens(T), 64 * kWaves, 0, st>>>(
+    MOE_DISPATCH_K(K, gather_bwd_kernel, float, grid_rows<float>(T, H), 64 * kWaves, 0, st>>>(
         (const float*)d_xs, slot, offsets, (const float*)addend, T, K, E, H, (float*)d_x));
   return check_launch(who);
 }
