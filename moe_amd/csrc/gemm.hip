@@ -1438,7 +1438,8 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
         }
         float my_w;
         int my_e;
-        group_sigmoid_topk<G, V>(sc, key, grp, g, K, p.ngroups, p.gtopk, p.renorm, p.scaling, 0,
+        group_sigmoid_topk<G, V>([&](int e) { return dsk_score(stf[rr * FROW + e], 0); }, key, grp,
+                                 g, K, p.ngroups, eg, p.gtopk, p.renorm, p.scaling, 0,
                                  tok && p.tpe != nullptr, scnt, my_w, my_e);
         if (tok) {
 #pragma unroll

@@ -106,9 +106,12 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void softmax_topk_kernel(
 // ngroups > 0, each group on one lane; rank keys of the biased scores, the
 // winner's unbiased score taken from its owner lane, weights renormalised by
 // their sum in rank order (+1e-20), scaled), cast.  VEC: E == G*V, fp32 rows
-// moved as 16-byte vectors.
+// moved as 16-byte vectors.  Eight waves per block: every block adds its
+// counts to the same E addresses, about 18 ns each, and four-wave blocks spent
+// 9 to 19 us of 36 to 41 on that (T = 32768, E = 128 and T = 65536, E = 64).
+constexpr int kSigmoidWaves = 8;
 template <int G, int V, bool VEC>
-__global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_group_kernel(
+__global__ __launch_bounds__(64 * kSigmoidWaves) void sigmoid_topk_group_kernel(
     const float* __restrict__ logits, const float* __restrict__ bias, int64_t T, int E, int K,
     int renorm, float scaling, int ngroups, int gtopk, float* __restrict__ scores,
     void* __restrict__ topk_w, int w_dtype, int64_t* __restrict__ topk_idx,
@@ -130,8 +133,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_group_kernel
     grp[j] = e0 + j < E ? (e0 + j) / eg : -1;
     cnt[j] = 0;
   }
-  const int64_t stride = (int64_t)gridDim.x * kWavesPerBlock * TPW;
-  for (int64_t tb = ((int64_t)blockIdx.x * kWavesPerBlock + wid) * TPW; tb < T; tb += stride) {
+  const int64_t stride = (int64_t)gridDim.x * kSigmoidWaves * TPW;
+  for (int64_t tb = ((int64_t)blockIdx.x * kSigmoidWaves + wid) * TPW; tb < T; tb += stride) {
     const int64_t t = tb + sub;
     const bool tok = t < T;
     const int64_t tt = tok ? t : T - 1;
@@ -166,8 +169,9 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_group_kernel
     }
     float my_w;
     int my_e;
-    group_sigmoid_topk<G, V>(sc, key, grp, g, K, ngroups, gtopk, renorm, scaling, scores_in,
-                             false, cnt, my_w, my_e);
+    group_sigmoid_topk<G, V>(
+        [&](int e) { return dsk_score(logits[tt * E + e], scores_in); }, key, grp, g, K, ngroups,
+        eg, gtopk, renorm, scaling, scores_in, false, cnt, my_w, my_e);
     if (tok && g < K) {
       if (w_dtype == MOE_DTYPE_BF16)
         ((bf16*)topk_w)[t * K + g] = f2bf(my_w);
@@ -305,6 +309,16 @@ void launch_softmax_group(bool key16, int grid, size_t shm, hipStream_t st, cons
 int grid_group(int64_t T, int G) {
   const int64_t per_block = (int64_t)kWavesPerBlock * (64 / G) * 2;  // two token batches per wave
   int64_t blocks = (T + per_block - 1) / per_block;
+  if (blocks > 8192) blocks = 8192;
+  return (int)(blocks < 1 ? 1 : blocks);
+}
+
+// The DeepSeek group kernel's blocks: two token batches per wave where that
+// still gives every CU a block, else one (T = 512: 18 us with two).
+int grid_sigmoid(int64_t T, int G) {
+  const int64_t per_batch = (int64_t)kSigmoidWaves * (64 / G);
+  int64_t blocks = (T + 2 * per_batch - 1) / (2 * per_batch);
+  if (blocks < 256) blocks = (T + per_batch - 1) / per_batch;
   if (blocks > 8192) blocks = 8192;
   return (int)(blocks < 1 ? 1 : blocks);
 }
@@ -896,7 +910,7 @@ int sigmoid_topk_run(const float* logits, const float* expert_bias, int64_t T, i
     const bool vec = E == G * V && al16(logits) && al16(scores);
     const int ng = num_groups > 0 ? num_groups : 0, gk = num_groups > 0 ? group_topk : 0;
 #define MOE_SIGMOID_GROUP(G_, V_, VEC_)                                                       \
-  sigmoid_topk_group_kernel<G_, V_, VEC_><<<grid_group(T, G_), 64 * kWavesPerBlock, shm, st>>>( \
+  sigmoid_topk_group_kernel<G_, V_, VEC_><<<grid_sigmoid(T, G_), 64 * kSigmoidWaves, shm, st>>>( \
       logits, expert_bias, T, E, K, renormalize, scaling_factor, ng, gk, scores, topk_weights, \
       weights_dtype, topk_index, tokens_per_expert, scores_in)
 #define MOE_SIGMOID_GROUP_V(G_, V_)            \

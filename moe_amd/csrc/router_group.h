@@ -95,46 +95,78 @@ __device__ __forceinline__ float dsk_weight(float v, float ssum, int renorm, flo
   return v;
 }
 
+// The largest key below thr of this lane's V keys, or 0: the minimum of
+// thr-1-key (keys at or above thr wrap past thr-1 and lose), so that no key
+// has to be marked as taken.
+template <int V>
+__device__ __forceinline__ uint64_t lane_next_key(const uint64_t (&key)[V], uint64_t thr) {
+  const uint64_t lim = thr - 1;
+  uint64_t d = lim - key[0];
+#pragma unroll
+  for (int j = 1; j < V; ++j) {
+    const uint64_t dj = lim - key[j];
+    d = dj < d ? dj : d;
+  }
+  return d <= lim ? lim - d : 0ull;
+}
+
 // DeepSeek-V3 selection of one token on a group of G lanes (the router
 // kernel, router.hip, and the gating linear's fused epilogue, gemm.hip, so
-// that both produce the same bits): lane g holds the token's entries
-// e0 = g*V .. e0+V-1 as unbiased sigmoid scores sc and rank keys of the
-// biased scores (0 past E).  With ngroups > 0 the experts form ngroups equal
-// groups of eg = E/ngroups (ngroups <= G); each group is scored by the sum of
-// its (K / gtopk) best biased scores, added best first, the gtopk best groups
-// (higher score first, lower group id on equal scores) are kept and the
-// other groups' entries drop out (router.py:22-70).  Then K rounds of a group
-// max over the keys; the winner's owner lane hands its unbiased score to the
-// group (router.py:130) and counts the selection in cnt (when count), the
-// scores are summed in rank order for the renormalisation (+1e-20) and
-// lane g < K receives the g-th weight and expert (router.py:133-138), in
-// torch's bf16 arithmetic when scores_in (dsk_weight).  The order of every
-// step is that of the wave-per-token router kernel as well, so the
-// selection and the weights are its bit for bit on the same scores.
-template <int G, int V>
-__device__ __forceinline__ void group_sigmoid_topk(const float (&sc)[V], uint64_t (&key)[V],
+// that both produce the same bits): lane g holds the rank keys of the biased
+// scores of entries e0 = g*V .. e0+V-1 (0 past E); score_of(e) gives the
+// unbiased sigmoid score of entry e.  With ngroups > 0 the experts form
+// ngroups equal groups of eg = E/ngroups (ngroups <= G); each group is scored
+// by the sum of its (K / gtopk) best biased scores, added best first, the
+// gtopk best groups (higher score first, lower group id on equal scores) are
+// kept and the other groups' entries drop out (router.py:22-70).  Where a
+// group is 1, 2 or 4 whole lanes those score it by themselves; else all lanes
+// score the groups one after the other.  Then K rounds of a group max over the keys;
+// lane g < K takes the g-th winner's unbiased score (router.py:130), the
+// scores are summed in rank order for the renormalisation (+1e-20) and lane g
+// receives the g-th weight and expert (router.py:133-138), in torch's bf16
+// arithmetic when scores_in (dsk_weight); cnt counts this lane's selected
+// entries (when count).  The order of every step is that of the wave-per-token
+// router kernel as well, so the selection and the weights are its bit for bit
+// on the same scores.
+// VALU-bound.  T = 32768, E = 128, 8 groups keep 4, K = 8 in the router
+// kernel: 51 us with eight group scores of two rounds each over all lanes,
+// marks on taken keys and the winner's score carried through every round, 27
+// us so (32 with the counts).  E = 256 (two lanes per group): 96 -> 62 us.
+template <int G, int V, typename F>
+__device__ __forceinline__ void group_sigmoid_topk(F&& score_of, uint64_t (&key)[V],
                                                    const int (&grp)[V], int g, int K,
-                                                   int ngroups, int gtopk, int renorm,
+                                                   int ngroups, int eg, int gtopk, int renorm,
                                                    float scaling, int scores_in, bool count,
                                                    int (&cnt)[V], float& my_w, int& my_e) {
   if (ngroups > 0) {
     const int per = K / gtopk;
     float gv = -INFINITY;  // lane g < ngroups: group g's score
-    for (int gi = 0; gi < ngroups; ++gi) {
-      uint64_t gk[V];
-#pragma unroll
-      for (int j = 0; j < V; ++j) gk[j] = grp[j] == gi ? key[j] : 0ull;
+    const int base = (int)(threadIdx.x & 63) - g;
+    if (eg == V || eg == 2 * V || eg == 4 * V) {
+      const int m = eg / V;  // lanes per group
       float acc = 0.f;
+      uint64_t thr = ~0ull;
       for (int q = 0; q < per; ++q) {
-        uint64_t b = gk[0];
-#pragma unroll
-        for (int j = 1; j < V; ++j) b = gk[j] > b ? gk[j] : b;
-        b = group_max_key<G>(b);
+        uint64_t b = lane_next_key<V>(key, thr);
+        if (m == 2) b = group_max_key<2>(b);
+        else if (m == 4) b = group_max_key<4>(b);
+        thr = b;
         acc += key_value(b);
-#pragma unroll
-        for (int j = 0; j < V; ++j) gk[j] = gk[j] == b ? 0ull : gk[j];
       }
-      gv = g == gi ? acc : gv;
+      gv = m == 1 ? acc : __shfl(acc, base + (g * m & (G - 1)), 64);
+    } else {
+      for (int gi = 0; gi < ngroups; ++gi) {
+        uint64_t gk[V];
+#pragma unroll
+        for (int j = 0; j < V; ++j) gk[j] = grp[j] == gi ? key[j] : 0ull;
+        float acc = 0.f;
+        uint64_t thr = ~0ull;
+        for (int q = 0; q < per; ++q) {
+          thr = group_max_key<G>(lane_next_key<V>(gk, thr));
+          acc += key_value(thr);
+        }
+        gv = g == gi ? acc : gv;
+      }
     }
     uint64_t gkey = g < ngroups ? rank_key(gv, g) : 0ull;
     uint32_t keep = 0;
@@ -147,28 +179,21 @@ __device__ __forceinline__ void group_sigmoid_topk(const float (&sc)[V], uint64_
     for (int j = 0; j < V; ++j)
       if (grp[j] < 0 || !((keep >> grp[j]) & 1u)) key[j] = 0ull;
   }
-  float ssum = 0.f;
-  my_w = 0.f;
-  my_e = 0;
+  uint64_t thr = ~0ull, mine = 0;
   for (int k = 0; k < K; ++k) {
-    uint64_t b = key[0];
+    thr = group_max_key<G>(lane_next_key<V>(key, thr));
+    mine = g == k ? thr : mine;
+  }
+  my_e = g < K ? key_index(mine) : 0;
+  my_w = g < K ? score_of(my_e) : 0.f;
+  if (count) {
 #pragma unroll
-    for (int j = 1; j < V; ++j) b = key[j] > b ? key[j] : b;
-    b = group_max_key<G>(b);
-    float own = -INFINITY;  // the winner's unbiased score, on its owner lane
-#pragma unroll
-    for (int j = 0; j < V; ++j) {
-      const bool hit = key[j] == b;
-      own = hit ? sc[j] : own;
-      key[j] = hit ? 0ull : key[j];
-      cnt[j] += (hit && count) ? 1 : 0;
-    }
-    const float sk = group_max<G>(own);
-    ssum += sk;
-    if (g == k) {
-      my_w = sk;
-      my_e = key_index(b);
-    }
+    for (int j = 0; j < V; ++j) cnt[j] += key[j] >= thr ? 1 : 0;  // thr: the K-th key, not 0
+  }
+  float ssum = 0.f;
+  if (renorm) {
+    const int base = (int)(threadIdx.x & 63) - g;
+    for (int k = 0; k < K; ++k) ssum += __shfl(my_w, base + k, 64);
   }
   my_w = dsk_weight(my_w, ssum, renorm, scaling, scores_in);
 }
