@@ -177,6 +177,10 @@ class SeqAuxLoss(torch.autograd.Function):
     def forward(ctx, num_experts, top_k, batch_size, selected, *layers):
         L = len(layers)
         _need_cuda(*layers)
+        if any(g.device != layers[0].device for g in layers):
+            # one launch reads them all
+            raise RuntimeError("seq load-balancing loss: expected all layers on the same device, "
+                               f"got {sorted({str(g.device) for g in layers})}")
         ps = [_as_probs(g) for g in layers]
         sels: list = [None] * L
         for li in range(min(L, len(selected)) if selected is not None else 0):
