@@ -34,7 +34,7 @@ import torch
 
 METRIC = ("MoE layer fwd+bwd tokens/sec and grouped-GEMM TFLOP/s (% bf16 MFMA peak), 1 GPU")
 PEAK_BF16_TFLOPS = 2500.0
-PEAK_FP32_TFLOPS = 157.3  # dense fp32 MFMA (the fp32 XS-standard layer's GEMMs)
+PEAK_FP32_TFLOPS = PEAK_BF16_TFLOPS / 6  # six bf16 MFMA products per fp32 one (gemm_f32.hip)
 PEAK_HBM_GBS = 8000.0
 
 
