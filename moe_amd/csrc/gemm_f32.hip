@@ -24,42 +24,45 @@
 // value is split into three bf16 terms x = hi + mid + lo (each the
 // round-to-nearest of what is left: 8 bits plus a sign per term, so the sum
 // is exact for every finite x whose terms do not underflow), and a product is
-// summed as hi*hi + hi*mid + mid*hi + hi*lo + lo*hi + mid*mid in the fp32
-// accumulators; the three products left out are at most 2^-25 of |x*y|
-// together, below the fp32 rounding of one addition.  The bf16 products are
-// exact, and one MFMA sums 16 of them per accumulator rounding where the fp32
-// MFMA sums 2: the XS layer's outputs are 0.9e-6 from the 64-bit ones
-// (2-norm) and its weight gradients 1.0e-6, against 1.0e-6 and 1.2e-6 with
-// the fp32 MFMA.  A value
-// that is not finite, or overflows as bf16, makes every element it touches
-// non-finite here; a workgroup that finds such an element in its tile
+// summed as hi*hi + hi*mid + mid*hi + hi*lo + lo*hi + mid*mid; the three
+// products left out are at most 2^-24 of |x*y| together.  hi*hi has its own
+// fp32 accumulators and the five small products share others, added once at
+// the end: in one accumulator all six MFMAs of 16 k would round at the sum's
+// scale, where the fp32 MFMA rounds once for 2 k, and a row with few terms
+// other than zero came out up to twice as far from 64 bits as there.  2-norm
+// errors, fp32 MFMA / one accumulator / two: 1 nonzero term 2.5e-8 / 3.4e-8 /
+// 2.6e-8, 4 terms 4.1e-8 / 7.6e-8 / 2.7e-8, 64 terms 1.4e-7 / 2.7e-7 / 5.6e-8,
+// 768 terms 4.9e-7 / 4.2e-7 / 1.6e-7.  A weight gradient over at most 32 rows
+// (one stage) also sums mid*lo and lo*mid, so that the one product of a single
+// row is rounded as the fp32 MFMA's: 2.53e-8 both, 3.46e-8 before.
+// A value that is not finite, or overflows as bf16, makes every element it
+// touches non-finite here; a workgroup that finds such an element in its tile
 // computes the tile again with the fp32 MFMA (v_mfma_f32_32x32x2_f32), whose
 // infinities and NaNs are the plain fp32 ones.
 //
 // Workgroup: 256 threads = 4 waves as 2 x 2, a 128 x 128 tile of C, each wave
-// a 64 x 64 block of 2 x 2 MFMA sub-tiles (64 fp32 accumulators per lane).
+// a 64 x 64 block of 2 x 2 MFMA sub-tiles (64 fp32 accumulators per lane for
+// hi*hi, 64 for the small products).
 // A k-stage is 32 deep: both operands are loaded global -> registers (16
 // bytes per load, coalesced along the contiguous index), split in registers
 // and written to LDS as three bf16 planes of [feature][32 k] (64-byte rows,
 // lds_at()'s swizzle makes the fragment reads and both operands' writes
 // bank-conflict free); the loads of stage s+1 are in flight while stage s is
-// multiplied.  One stage buffer of 48 KB, so that three workgroups share a
-// CU: one splits while the others multiply (two per CU: F1 662, FDX1 667 us).
+// multiplied.  One stage buffer of 48 KB and 128 accumulators: two workgroups
+// share a CU, one splits while the other multiplies.  (With one accumulator
+// per element three workgroups fit: the six GEMMs below took 2436 us, now 2582.)
 // Per stage a wave issues 48 MFMAs (1536 cycles) and about 250 VALU
-// instructions (1000 cycles, mostly the split); the matrix cores are busy 60%
-// of the cycles at 1.83 GHz.  Kernel times at S = 32768 rows, H = 1024, E =
-// 16, I = 768, with the fp32 MFMA -> with the split: F1 935 -> 626, F2 485 ->
-// 304, FDX2 658 -> 368, FDX1 1214 -> 573, FDW2 790 -> 290, FDW1 1453 -> 624 us
-// (84, 106, 78, 85, 65, 71 -> 165, 170, 140, 180, 178, 165 TFLOP/s); the
-// loads of an operand issued as soon as its registers are free, no wait for
-// them at the barriers and the priority of multiplying waves take another 2%
-// (2493 -> 2451 us over the six).  That is 1.1
-// PFLOP/s of bf16 products, what the board's power leaves the bf16 grouped
-// GEMMs too.  Output: register 4q+c of a lane
-// holds (tile row L % 32, tile column 8q + 4(L/32) + c) of the sub-tile (the
-// column operand is MFMA's "A").  Epilogue: 64 rows at a time are staged in
-// LDS (reusing the stage buffer) and written out row by row with 16-byte
-// lanes, applying the SwiGLU / dSwiGLU tail in fp32.
+// instructions (1000 cycles, mostly the split).  Kernel times at S = 32768
+// rows, H = 1024, E = 16, I = 768, with the fp32 MFMA -> with the split: F1 899 ->
+// 571, F2 467 -> 282, FDX2 645 -> 358, FDX1 1195 -> 545, FDW2 792 -> 279, FDW1
+// 1448 -> 548 us (180, 183, 144, 189, 185, 188 TFLOP/s).  That is 1.1 PFLOP/s of
+// bf16 products, what the board's power leaves the bf16 grouped GEMMs too.
+// An operand's loads go out as soon as its registers are free, no barrier
+// waits for them and multiplying waves have priority (2% over the six).
+// Output: register 4q+c of a lane holds (tile row L % 32, tile column 8q + 4(L/32) + c)
+// of the sub-tile (the column operand is MFMA's "A").  Epilogue: 64 rows at a
+// time are staged in LDS (reusing the stage buffer) and written out row by row
+// with 16-byte lanes, applying the SwiGLU / dSwiGLU tail in fp32.
 //
 // Token-grouped tiles come from the permutation's row-tile table for 128-row
 // tiles ({expert, first row, end row} per tile, device-side); dW tiles are
@@ -130,7 +133,7 @@ __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& hi, uin
 }
 
 template <int MODE>
-__global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
+__global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
   constexpr bool TOKEN = MODE == F1 || MODE == F2 || MODE == FDX2 || MODE == FDX1;
   constexpr bool COL_KM = MODE != F1 && MODE != F2;
   constexpr bool ROW_KM = MODE == FDW2 || MODE == FDW1;
@@ -336,16 +339,17 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
-  f32x16 acc[2][2];
-  auto zero_acc = [&]() {
+  f32x16 acc[2][2], low[2][2];  // hi*hi; the small products
+  auto zero = [](f32x16 (&v)[2][2]) {
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+        for (int r = 0; r < 16; ++r) v[i][j][r] = 0.f;
   };
-  zero_acc();
+  zero(acc);
+  zero(low);
 
   if (nk > 0) {
     // fragment addresses of k sub-step 0 (sub-step 1: chunk ^ 2)
@@ -358,11 +362,16 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
     load_src(0);
     load_rows(0);
     load_cols(0);
-    for (int s = 0; s < nk; ++s) {
+    // One stage, with the last NP of the eight products (small ones first).
+    auto stage = [&](int s, auto np) {
+      constexpr int NP = decltype(np)::value;
+      constexpr int TA[8] = {2, 1, 2, 0, 1, 1, 0, 0}, TB[8] = {1, 2, 0, 2, 1, 0, 1, 0};
       // An operand's next loads go out as soon as its registers are free, so
       // they have a barrier, the MFMAs and the other operand's split to land.
-      // (Unconditionally: past the last stage the descriptors are empty, F1
-      // reads its last rows again.  A branch would make every wait a full one.)
+      // (Unconditionally, since a branch would make every wait a full one: what
+      // lies past the last stage is not used.  A k-major operand's descriptor
+      // is empty there, a k-contiguous one reads on within the tile's rows, or
+      // zeros past them, and F1 reads its last rows again.)
       __builtin_amdgcn_s_setprio(0);
       store_operand(rv, planes, std::integral_constant<bool, ROW_KM>{});
       __builtin_amdgcn_sched_barrier(0);
@@ -384,18 +393,23 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
             a[t][i] = *(const bf16x8*)(planes + t * kPlane + (fa[i] ^ (kk * 32)));
             b[t][i] = *(const bf16x8*)(planes + t * kPlane + (fb[i] ^ (kk * 32)));
           }
-        // small products first
-        constexpr int TA[6] = {2, 0, 1, 1, 0, 0}, TB[6] = {0, 2, 1, 0, 1, 0};
 #pragma unroll
-        for (int t = 0; t < 6; ++t)
+        for (int t = 8 - NP; t < 8; ++t)
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int j = 0; j < 2; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]][i], b[TB[t]][j],
-                                                                  acc[i][j], 0, 0, 0);
+            for (int j = 0; j < 2; ++j) {
+              f32x16& c = t < 7 ? low[i][j] : acc[i][j];
+              c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]][i], b[TB[t]][j], c, 0, 0, 0);
+            }
       }
       sync_lds();  // the stage is read: the next one may be written
+    };
+    // dW of an expert with few rows: see the head of the file
+    if (ROW_KM && nk == 1) {
+      stage(0, std::integral_constant<int, 8>{});
+    } else {
+      for (int s = 0; s < nk; ++s) stage(s, std::integral_constant<int, 6>{});
     }
     // Non-finite elements: the whole tile again on the fp32 MFMA.
     bool bad = false;
@@ -404,9 +418,12 @@ __global__ __launch_bounds__(FNT, 3) void f32_gemm_kernel(FArgs p) {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) bad |= !(fabsf(acc[i][j][r]) < INFINITY);
+        for (int r = 0; r < 16; ++r) {
+          acc[i][j][r] += low[i][j][r];
+          bad |= !(fabsf(acc[i][j][r]) < INFINITY);
+        }
     if (__syncthreads_or(bad)) {
-      zero_acc();
+      zero(acc);
       float* const R = fsm;
       float* const C = fsm + FBM * FLD;
       load_src(0);

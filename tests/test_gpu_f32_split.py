@@ -1,10 +1,15 @@
 """The fp32 grouped GEMMs (bf16 matrix cores, three-term split) against fp64.
 
-Bound per element: the kernel adds 6 * ceil(K/16) MFMA results of at most 16
-exact products into an fp32 accumulator, and leaves out products worth at
-most 2^-25 of |a||b|; with every MFMA adding its 16 products and the
-accumulator with at most 17 roundings, |error| <= (17 * 6 * ceil(K/16) + 2) *
-2^-24 * sum |a||b| (first order), K the contracted length."""
+Bound per element: with K the contracted length and u = 2^-24, the kernel adds
+ceil(K/16) MFMA results of at most 16 exact products hi*hi into one fp32
+accumulator and five times as many small ones, worth at most 2^-7 of |a||b|,
+into another, every MFMA with at most 17 roundings; it leaves out products of
+at most 2^-24 of |a||b| and adds the two accumulators.  To first order |error|
+<= (18 * ceil(K/16) + 3) * u * sum |a||b|.
+
+That bound grows with K and does not see a lost third term, so the 2-norm
+errors are also held against a chain of fp32 fused multiply-adds over the same
+terms (test_f32_gemms_no_further_than_fp32_chain)."""
 import pytest
 import torch
 
@@ -15,7 +20,7 @@ DEV = "cuda"
 
 
 def _bound(K):
-    return (17 * 6 * ((K + 15) // 16) + 2) * 2.0 ** -24
+    return (18 * ((K + 15) // 16) + 3) * 2.0 ** -24
 
 
 def _plan(T, E, K, seed):
@@ -74,6 +79,103 @@ def test_f32_gemms_against_fp64(T, H, E, K, I):
         _check(dxs[r], dg @ a1, dg.abs() @ a1.abs(), 2 * I)
         _check(dw2[e], d.T @ ac, d.abs().T @ ac.abs(), n)
         _check(dw1[e], dg.T @ xe, dg.abs().T @ xe.abs(), n)
+
+
+MODES = ["gate_up", "down", "down_dx", "gate_up_dx", "down_dw", "gate_up_dw"]
+
+
+def _operands(mode, K, seed, nonzero=0):
+    """Operands a [M,K], b [N,K] of one expert, N(0,1); with `nonzero`, a keeps
+    that many terms per row.  M, N have tile remainders."""
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    M, N = {"down_dw": (192, 64), "gate_up_dw": (384, 64), "gate_up": (130, 384)}.get(mode, (130, 192))
+    a, b = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    if nonzero and nonzero < K:
+        at = torch.rand(M, K, generator=g, device=DEV).topk(nonzero, dim=-1).indices
+        a = torch.zeros_like(a).scatter_(1, at, a.gather(1, at))
+    return a, b
+
+
+def _product(mode, a, b):
+    """a b^T by one of the six GEMMs, for one expert."""
+    rows = a.shape[1] if mode.endswith("_dw") else a.shape[0]
+    plan = ops.permute(torch.zeros(rows, 1, dtype=torch.int64, device=DEV), 1)
+    if mode == "gate_up":
+        return ops.gemm_gate_up_swiglu(a, plan, b[None].contiguous())[0]
+    if mode == "down":
+        return ops.gemm_down(a, plan, b[None].contiguous())
+    if mode == "gate_up_dx":
+        return ops.gemm_gate_up_backward_dx(a, plan, b.T[None].contiguous())
+    if mode == "down_dx":  # at gate = 64 and up = 1 the tail gives d_gate = d_act, d_up = 64 d_act
+        gu = torch.ones(rows, 2 * b.shape[0], device=DEV)
+        gu[:, :b.shape[0]] = 64.0
+        d = ops.gemm_down_backward_dx_dswiglu(a, plan, b.T[None].contiguous(), gu)
+        assert torch.equal(d[:, :b.shape[0]] * 64, d[:, b.shape[0]:])
+        return d[:, :b.shape[0]]
+    at, bt = a.T.contiguous(), b.T.contiguous()
+    if mode == "down_dw":
+        return ops.gemm_down_backward_dw(at, bt, plan, (1, a.shape[0], b.shape[0]))[0]
+    return ops.gemm_gate_up_backward_dw(at, bt, plan, (1, a.shape[0], b.shape[0]))[0]
+
+
+def _chain32(a, b):
+    """a b^T as a chain of fp32 fused multiply-adds in k order."""
+    acc = torch.zeros(a.shape[0], b.shape[0], device=DEV)
+    for k in range(a.shape[1]):
+        acc = (acc.double() + a[:, k, None].double() * b[None, :, k].double()).float()
+    return acc
+
+
+def _terms(x):
+    hi = x.bfloat16().float()
+    mid = (x - hi).bfloat16().float()
+    return mid.double(), (x - hi - mid).double()
+
+
+def _left_out(a, b, eight):
+    """The part of a b^T that the kernel leaves out (eight of nine products, or six)."""
+    (am, al), (bm, bl) = _terms(a), _terms(b)
+    d = al @ bl.T
+    return d if eight else d + am @ bl.T + al @ bm.T
+
+
+CHAIN = ([(m, K, nz) for m in MODES[:4] for K, nz in [(128, 1), (128, 2), (128, 4), (256, 16),
+                                                      (768, 64), (128, 128), (768, 768)]]
+         + [(m, K, nz) for m in MODES[4:] for K, nz in [(1, 1), (2, 2), (3, 3), (32, 32), (33, 33),
+                                                        (200, 4), (200, 200)]])
+
+
+@pytest.mark.parametrize("mode,K,nonzero", CHAIN)
+def test_f32_gemms_no_further_than_fp32_chain(mode, K, nonzero):
+    """2-norm distance from 64 bits: that of a chain of fp32 fused multiply-adds
+    over the same terms, with what the kernel leaves out added in quadrature
+    (and 1% for what rounds below that)."""
+    print(f"f32 split {mode} K={K} nonzero={nonzero}", flush=True)
+    a, b = _operands(mode, K, 7 * K + nonzero, nonzero)
+    want = a.double() @ b.double().T
+    err = (_product(mode, a, b).double() - want).norm()
+    chain = (_chain32(a, b).double() - want).norm()
+    left = _left_out(a, b, mode.endswith("_dw") and K <= 32).norm()
+    assert float(err) <= 1.01 * float((chain ** 2 + left ** 2).sqrt()), float(err / want.norm())
+
+
+def test_f32_down_dx_dswiglu_tail():
+    """dX + dSwiGLU on ordinary gates, no further from 64 bits than the same
+    formulas in fp32 on the fp32 chain's d_act."""
+    T, H, I = 200, 192, 128
+    g = torch.Generator(device=DEV).manual_seed(4)
+    dy, w2 = torch.randn(T, H, generator=g, device=DEV), torch.randn(H, I, generator=g, device=DEV)
+    gu = torch.randn(T, 2 * I, generator=g, device=DEV) * 3
+    plan = ops.permute(torch.zeros(T, 1, dtype=torch.int64, device=DEV), 1)
+
+    def tail(da, gu):
+        gate, up = gu.split(I, dim=1)
+        s = torch.sigmoid(gate)
+        return torch.cat([da * up * s * (1 + gate * (1 - s)), da * gate * s], dim=1)
+
+    want = tail(dy.double() @ w2.double(), gu.double())
+    err = (ops.gemm_down_backward_dx_dswiglu(dy, plan, w2[None], gu).double() - want).norm()
+    assert float(err) <= float((tail(_chain32(dy, w2.T), gu).double() - want).norm())
 
 
 def test_f32_gemms_small_magnitudes():
@@ -137,5 +239,6 @@ def test_f32_layer_gradients_against_fp64():
         ref = ref.index_add(0, t, y * l64[1][t, k][:, None])
     ref.backward(dout.double())
     for got, want in [(out, ref)] + [(a.grad, b.grad) for a, b in zip(leaves, l64)]:
-        # fp32 rounding through three contractions of at most 256 terms
-        assert float((got.double() - want).norm() / want.norm()) < 5e-6
+        # three contractions of at most 256 terms, each no further than a chain of fp32
+        # multiply-adds (2.9e-7 at 256 terms), in quadrature, and the fp32 tail's roundings
+        assert float((got.detach().double() - want.detach()).norm() / want.detach().norm()) < 6e-7
