@@ -38,7 +38,9 @@
 // A value that is not finite, or overflows as bf16, makes every element it
 // touches non-finite here; a workgroup that finds such an element in its tile
 // computes the tile again with the fp32 MFMA (v_mfma_f32_32x32x2_f32), whose
-// infinities and NaNs are the plain fp32 ones.
+// infinities and NaNs are the plain fp32 ones, and takes those elements from
+// it.  The others keep their bits: an element depends on its own row and
+// column only, whatever else is in the tile.
 //
 // Workgroup: 256 threads = 4 waves as 2 x 2, a 128 x 128 tile of C, each wave
 // a 64 x 64 block of 2 x 2 MFMA sub-tiles (64 fp32 accumulators per lane for
@@ -411,7 +413,8 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
     } else {
       for (int s = 0; s < nk; ++s) stage(s, std::integral_constant<int, 6>{});
     }
-    // Non-finite elements: the whole tile again on the fp32 MFMA.
+    // Non-finite elements: the tile again on the fp32 MFMA (into `low`, which is
+    // free by now), from which only they are taken.
     bool bad = false;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
@@ -423,7 +426,7 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
           bad |= !(fabsf(acc[i][j][r]) < INFINITY);
         }
     if (__syncthreads_or(bad)) {
-      zero(acc);
+      zero(low);
       float* const R = fsm;
       float* const C = fsm + FBM * FLD;
       load_src(0);
@@ -461,10 +464,17 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
             for (int i = 0; i < 2; ++i)
 #pragma unroll
               for (int j = 0; j < 2; ++j)
-                acc[i][j] =
-                    __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][q], b[j][q], acc[i][j], 0, 0, 0);
+                low[i][j] =
+                    __builtin_amdgcn_mfma_f32_32x32x2f32(a[i][q], b[j][q], low[i][j], 0, 0, 0);
         }
       }
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r)
+            acc[i][j][r] = fabsf(acc[i][j][r]) < INFINITY ? acc[i][j][r] : low[i][j][r];
     }
   }
 

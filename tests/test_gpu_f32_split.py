@@ -110,7 +110,7 @@ def _product(mode, a, b):
         gu = torch.ones(rows, 2 * b.shape[0], device=DEV)
         gu[:, :b.shape[0]] = 64.0
         d = ops.gemm_down_backward_dx_dswiglu(a, plan, b.T[None].contiguous(), gu)
-        assert torch.equal(d[:, :b.shape[0]] * 64, d[:, b.shape[0]:])
+        assert torch.equal((d[:, :b.shape[0]] * 64).nan_to_num(), d[:, b.shape[0]:].nan_to_num())
         return d[:, :b.shape[0]]
     at, bt = a.T.contiguous(), b.T.contiguous()
     if mode == "down_dw":
@@ -217,6 +217,32 @@ def test_f32_gemms_nonfinite(bad):
     err = (y.double() - want).abs()[fin]
     # the fp32 MFMA that recomputes these tiles: one rounding per two products
     assert bool((err <= max(_bound(I), I * 2.0 ** -24) * mags[fin]).all())
+
+
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("bad", [float("inf"), float("nan"), -3.4e38])
+def test_f32_gemms_nonfinite_stays_in_its_rows(mode, bad):
+    """In every GEMM: the elements of a non-finite (or bf16-overflowing) value's
+    row and column are the fp32 product's, all others of the tile keep the bits
+    that they have without it."""
+    print(f"f32 split {mode} non-finite {bad}", flush=True)
+    a, b = _operands(mode, 256, 17)
+    clean = _product(mode, a, b)
+    a[3, 17], a[125, 255] = bad, bad
+    b[40, 5] = bad
+    b[10, 17] = 0.0  # inf * 0 = NaN at (3, 10)
+    got = _product(mode, a, b)
+    want = a.double() @ b.double().T
+    big = want.abs() > 3.4028235677973366e38  # beyond fp32
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(torch.isinf(got), torch.isinf(want) | big)
+    assert torch.equal(got[torch.isinf(got)] > 0, want[torch.isinf(got)] > 0)
+    fin = torch.isfinite(got)
+    mags = a.double().abs() @ b.double().abs().T
+    assert bool(((got.double() - want).abs()[fin] <= 256 * 2.0 ** -24 * mags[fin]).all())
+    rows = [i for i in range(a.shape[0]) if i not in (3, 125)]
+    cols = [i for i in range(b.shape[0]) if i not in (10, 40)]
+    assert torch.equal(got[rows][:, cols], clean[rows][:, cols])
 
 
 def test_f32_layer_gradients_against_fp64():
