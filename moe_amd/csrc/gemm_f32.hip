@@ -23,7 +23,7 @@
 // fp32 product made of six bf16 ones has 2.6 times the room.  Every operand
 // value is split into three bf16 terms x = hi + mid + lo (each the
 // round-to-nearest of what is left: 8 bits plus a sign per term, so the sum
-// is exact for every finite x whose terms do not underflow), and a product is
+// is exact), and a product is
 // summed as hi*hi + hi*mid + mid*hi + hi*lo + lo*hi + mid*mid; the three
 // products left out are at most 2^-24 of |x*y| together.  hi*hi has its own
 // fp32 accumulators and the five small products share others, added once at
@@ -35,7 +35,12 @@
 // 768 terms 4.9e-7 / 4.2e-7 / 1.6e-7.  A weight gradient over at most 32 rows
 // (one stage) also sums mid*lo and lo*mid, so that the one product of a single
 // row is rounded as the fp32 MFMA's: 2.53e-8 both, 3.46e-8 before.
-// A value that is not finite, or overflows as bf16, makes every element it
+// Both operands are multiplied by 2^16 on their way, and the sums by
+// 2^-32 at the end (exact in normal range): the last bit of the smallest fp32
+// subnormal then lies at the smallest bf16 one, so that no term underflows
+// (without it a value below 2^-110 lost its third term, then its second: 2.2e-6
+// at 2^-116, 5.6e-4 at 2^-124; now 9e-8 down to 2^-128, as at 1).
+// A value that is not finite, or overflows (from 2^112 on, sums from 2^96 on), makes every element it
 // touches non-finite here; a workgroup that finds such an element in its tile
 // computes the tile again with the fp32 MFMA (v_mfma_f32_32x32x2_f32), whose
 // infinities and NaNs are the plain fp32 ones, and takes those elements from
@@ -52,12 +57,13 @@
 // bank-conflict free); the loads of stage s+1 are in flight while stage s is
 // multiplied.  One stage buffer of 48 KB and 128 accumulators: two workgroups
 // share a CU, one splits while the other multiplies.  (With one accumulator
-// per element three workgroups fit: the six GEMMs below took 2436 us, now 2582.)
-// Per stage a wave issues 48 MFMAs (1536 cycles) and about 250 VALU
-// instructions (1000 cycles, mostly the split).  Kernel times at S = 32768
+// per element three workgroups fit: the six GEMMs below took 2436 us, with two
+// 2585, with the operands' scaling 2673.)
+// Per stage a wave issues 48 MFMAs (1536 cycles) and about 280 VALU
+// instructions (1100 cycles, mostly the split).  Kernel times at S = 32768
 // rows, H = 1024, E = 16, I = 768, with the fp32 MFMA -> with the split: F1 899 ->
-// 571, F2 467 -> 282, FDX2 645 -> 358, FDX1 1195 -> 545, FDW2 792 -> 279, FDW1
-// 1448 -> 548 us (180, 183, 144, 189, 185, 188 TFLOP/s).  That is 1.1 PFLOP/s of
+// 596, F2 467 -> 298, FDX2 645 -> 361, FDX1 1195 -> 577, FDW2 792 -> 287, FDW1
+// 1448 -> 556 us (173, 173, 143, 179, 180, 185 TFLOP/s).  That is 1.1 PFLOP/s of
 // bf16 products, what the board's power leaves the bf16 grouped GEMMs too.
 // An operand's loads go out as soon as its registers are free, no barrier
 // waits for them and multiplying waves have priority (2% over the six).
@@ -125,9 +131,13 @@ __device__ __forceinline__ uint32_t lds_at(int f, int c) {
   return (uint32_t)((f ^ ((f >> 4) & 3)) * 64 + ((c ^ ((f >> 2) & 3)) << 4));
 }
 
-// Two fp32 values -> their three bf16 terms, packed in pairs.
+constexpr float kScale = 65536.f;  // on both operands: see the head of the file
+
+// Two fp32 values -> the three bf16 terms of kScale times each, packed in pairs.
 __device__ __forceinline__ void split_pair(float x0, float x1, uint32_t& hi, uint32_t& mid,
                                            uint32_t& lo) {
+  x0 *= kScale;
+  x1 *= kScale;
   hi = pack_bf2(x0, x1);
   const float r0 = x0 - bf_lo(hi), r1 = x1 - bf_hi(hi);
   mid = pack_bf2(r0, r1);
@@ -422,7 +432,7 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          acc[i][j][r] += low[i][j][r];
+          acc[i][j][r] = (acc[i][j][r] + low[i][j][r]) * (1.f / kScale / kScale);
           bad |= !(fabsf(acc[i][j][r]) < INFINITY);
         }
     if (__syncthreads_or(bad)) {

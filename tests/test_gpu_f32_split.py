@@ -178,17 +178,19 @@ def test_f32_down_dx_dswiglu_tail():
     assert float(err) <= float((tail(_chain32(dy, w2.T), gu).double() - want).norm())
 
 
-def test_f32_gemms_small_magnitudes():
-    """Values near 2^-112, whose third term is below the smallest normal."""
-    T, H, I = 130, 64, 256
-    plan = ops.permute(torch.zeros(T, 1, dtype=torch.int64, device=DEV), 1)
-    g = torch.Generator(device=DEV).manual_seed(6)
-    act = torch.randn(T, I, generator=g, device=DEV) * 2.0 ** -112
-    w2 = torch.randn(1, H, I, generator=g, device=DEV)
-    y = ops.gemm_down(act, plan, w2)
-    a, w = act.double(), w2[0].double()
-    _check(y, a @ w.T, a.abs() @ w.abs().T, I)
-    assert float((y.double() - a @ w.T).norm() / (a @ w.T).norm()) < 1e-6
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("ea,eb", [(-112, 0), (-120, 0), (-128, 20), (-140, 40), (50, -140),
+                                   (-62, -62), (100, -100), (110, -90), (60, 60)])
+def test_f32_gemms_magnitudes(mode, ea, eb):
+    """Operands near 2^ea and 2^eb, subnormal ones among them: as far from 64
+    bits as at 1."""
+    print(f"f32 split {mode} 2^{ea} x 2^{eb}", flush=True)
+    a, b = _operands(mode, 256, 3)
+    a = torch.ldexp(a.double(), torch.tensor(ea, device=DEV)).float()
+    b = torch.ldexp(b.double(), torch.tensor(eb, device=DEV)).float()
+    want = a.double() @ b.double().T
+    err = (_product(mode, a, b).double() - want).norm()
+    assert float(err / want.norm()) <= float((_chain32(a, b).double() - want).norm() / want.norm())
 
 
 @pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan"), 3.4e38])
