@@ -57,17 +57,17 @@ int stats_blocks(int64_t T) {
 }
 
 // Combines the four waves' per-lane accumulators of one [E] vector in wave
-// order and writes the block's partial.  `buf` holds kWaves * 64 floats.
-template <int NV>
-__device__ void block_combine(const float (&acc)[NV], int E, float* buf, float* out) {
+// order and writes the block's partial.  `buf` holds kWaves * 64 values.
+template <int NV, typename T>
+__device__ void block_combine(const T (&acc)[NV], int E, double* buf, double* out) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     __syncthreads();
-    buf[wid * 64 + lane] = acc[j];
+    buf[wid * 64 + lane] = (double)acc[j];
     __syncthreads();
     if (wid == 0) {
-      float s = buf[lane];
+      double s = buf[lane];
       for (int w = 1; w < kWaves; ++w) s += buf[w * 64 + lane];
       const int e = j * 64 + lane;
       if (e < E) out[e] = s;
@@ -78,12 +78,13 @@ __device__ void block_combine(const float (&acc)[NV], int E, float* buf, float* 
 // The same statistics with G lanes per token (E <= 16*G, K <= G): lane g of
 // a group owns experts g*V .. g*V+V-1, ranks through rank_key with G-lane DPP
 // butterflies (as the softmax router's group kernel).  The block partial is
-// the sum over the block's kWaves*64/G token groups in group order, through
-// LDS ([groups][E] floats, dynamic shared memory).
+// the fp64 sum over the block's kWaves*64/G token groups in group order, through
+// LDS ([groups][E] floats, dynamic shared memory): only a group's own tokens
+// (up to 16, stats_blocks' limit apart) are added in fp32.
 template <int G, int V>
 __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
     Layers layers, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
-    int K, float* __restrict__ part_cnt, float* __restrict__ part_sum,
+    int K, double* __restrict__ part_cnt, double* __restrict__ part_sum,
     double* __restrict__ part_margin) {
   const void* const __restrict__ probs = layers.in[blockIdx.y];
   const size_t part = (size_t)blockIdx.y * gridDim.x + blockIdx.x;  // this block's partials
@@ -165,15 +166,15 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
     }
   }
   // Block partials: rows in group order, per expert.
-  auto combine = [&](const float (&acc)[V], float* out) {
+  auto combine = [&](const float (&acc)[V], double* out) {
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < V; ++j)
       if (e0 + j < E) sbuf[row * E + e0 + j] = acc[j];
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      float s = 0.f;
-      for (int r = 0; r < ROWS; ++r) s += sbuf[r * E + e];
+      double s = 0.0;
+      for (int r = 0; r < ROWS; ++r) s += (double)sbuf[r * E + e];
       out[e] = s;
     }
   };
@@ -201,17 +202,17 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_group_kernel(
 template <int NV>
 __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
     Layers layers, int dtype, const float* __restrict__ tok_w, int64_t T, int E,
-    int K, float* __restrict__ part_cnt, float* __restrict__ part_sum,
+    int K, double* __restrict__ part_cnt, double* __restrict__ part_sum,
     double* __restrict__ part_margin) {
   const void* const __restrict__ probs = layers.in[blockIdx.y];
   const size_t part = (size_t)blockIdx.y * gridDim.x + blockIdx.x;  // this block's partials
-  __shared__ float buf[kWaves * 64];
+  __shared__ double buf[kWaves * 64];
   __shared__ double mbuf[kWaves * 2];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  float cnt[NV], psum[NV];
+  double cnt[NV], psum[NV];
 #pragma unroll
-  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.f;
+  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.0;
   double msum = 0.0;
   float mmin = INFINITY;
   const int64_t nwaves = (int64_t)gridDim.x * kWaves;
@@ -224,7 +225,7 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
       const int e = j * 64 + lane;
       if (e < E) {
         v[j] = load_val(probs, dtype, t * E + e);
-        psum[j] += w * v[j];
+        psum[j] += (double)w * (double)v[j];
       } else {
         v[j] = -INFINITY;
         taken |= 1ull << j;
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j)
-      if (((taken & ~pad) >> j) & 1ull) cnt[j] += w;
+      if (((taken & ~pad) >> j) & 1ull) cnt[j] += (double)w;
     if (K < E) {  // margin between the k-th and (k+1)-th largest value
       float bv;
       int be;
@@ -283,15 +284,15 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 // l+64, ... in order, then the lanes are combined by a fixed butterfly.
 // Block E reduces the margin partials the same way.
 __global__ __launch_bounds__(64) void topk_stats_finalize_kernel(
-    const float* __restrict__ part_cnt, const float* __restrict__ part_sum,
+    const double* __restrict__ part_cnt, const double* __restrict__ part_sum,
     const double* __restrict__ part_margin, int nblk, int E, double* __restrict__ counts,
     double* __restrict__ sums, double* __restrict__ margin) {
   const int lane = threadIdx.x, e = blockIdx.x;
   if (e < E) {
     double c = 0.0, s = 0.0;
     for (int b = lane; b < nblk; b += 64) {
-      c += (double)part_cnt[(size_t)b * E + e];
-      s += (double)part_sum[(size_t)b * E + e];
+      c += part_cnt[(size_t)b * E + e];
+      s += part_sum[(size_t)b * E + e];
     }
     c = wave_sum_f64(c);
     s = wave_sum_f64(s);
@@ -360,8 +361,8 @@ __device__ __forceinline__ void load_row(const void* row0, int dtype, int64_t t,
 
 template <int G, int V>
 __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
-    Layers layers, int dtype, int64_t S, int chunk, int E, int K, float* __restrict__ part_cnt,
-    float* __restrict__ part_sum) {
+    Layers layers, int dtype, int64_t S, int chunk, int E, int K, double* __restrict__ part_cnt,
+    double* __restrict__ part_sum) {
   const void* const __restrict__ scores = layers.in[blockIdx.z];
   const int64_t* const __restrict__ selected = layers.sel[blockIdx.z];
   constexpr int TPW = 64 / G, ROWS = kWaves * TPW;
@@ -427,21 +428,21 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
     }
   }
   const size_t slot = (((size_t)blockIdx.z * gridDim.y + b) * gridDim.x + c) * E;
-  auto combine = [&](const float (&acc)[V], float* out) {
+  auto combine = [&](const float (&acc)[V], double* out) {
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < V; ++j)
       if (expert_of<G>(g, j) < E) sbuf[row * E + expert_of<G>(g, j)] = acc[j];
     __syncthreads();
     for (int e = threadIdx.x; e < E; e += blockDim.x) {
-      float sm = 0.f;
-      for (int r = 0; r < ROWS; ++r) sm += sbuf[r * E + e];
+      double sm = 0.0;
+      for (int r = 0; r < ROWS; ++r) sm += (double)sbuf[r * E + e];
       out[e] = sm;
     }
   };
   combine(psum, part_sum + slot);  // (its barriers come after every count)
   if (selected) {
-    for (int e = threadIdx.x; e < E; e += blockDim.x) part_cnt[slot + e] = (float)hist[e];
+    for (int e = threadIdx.x; e < E; e += blockDim.x) part_cnt[slot + e] = (double)hist[e];
   } else {
     combine(cnt, part_cnt + slot);
   }
@@ -449,17 +450,21 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_group_kernel(
 
 template <int NV>
 __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
-    Layers layers, int dtype, int64_t S, int chunk, int E, int K, float* __restrict__ part_cnt,
-    float* __restrict__ part_sum) {
+    Layers layers, int dtype, int64_t S, int chunk, int E, int K, double* __restrict__ part_cnt,
+    double* __restrict__ part_sum) {
   const void* const __restrict__ scores = layers.in[blockIdx.z];
   const int64_t* const __restrict__ selected = layers.sel[blockIdx.z];
-  __shared__ float buf[kWaves * 64];
+  __shared__ double buf[kWaves * 64];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.y, c = blockIdx.x;
-  float cnt[NV], psum[NV];
+  float cnt[NV];  // whole numbers up to chunk
+  double psum[NV];
 #pragma unroll
-  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.f;
+  for (int j = 0; j < NV; ++j) {
+    cnt[j] = 0.f;
+    psum[j] = 0.0;
+  }
   const int64_t s0 = (int64_t)c * chunk;
   const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
   for (int64_t st = s0 + wid; st < s1; st += kWaves) {
@@ -478,7 +483,7 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       v[j] = v[j] / rs;
-      psum[j] += v[j];
+      psum[j] += (double)v[j];
     }
     if (selected) {
       for (int k = 0; k < K; ++k) {
@@ -514,7 +519,7 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
 // One wave per (b, e): counts[b][e] = sum over chunks, mean[b][e] = sum over
 // chunks / S, in the fixed order of wave_sum_f64.
 __global__ __launch_bounds__(64) void seq_stats_finalize_kernel(
-    const float* __restrict__ part_cnt, const float* __restrict__ part_sum, int nchunk, int B,
+    const double* __restrict__ part_cnt, const double* __restrict__ part_sum, int nchunk, int B,
     int E, int64_t S, double* __restrict__ counts, double* __restrict__ mean) {
   const int lane = threadIdx.x;
   const int64_t i = blockIdx.x;
@@ -522,8 +527,8 @@ __global__ __launch_bounds__(64) void seq_stats_finalize_kernel(
   double c = 0.0, s = 0.0;
   for (int k = lane; k < nchunk; k += 64) {
     const size_t o = ((size_t)b * nchunk + k) * E + e;
-    c += (double)part_cnt[o];
-    s += (double)part_sum[o];
+    c += part_cnt[o];
+    s += part_sum[o];
   }
   c = wave_sum_f64(c);
   s = wave_sum_f64(s);
@@ -552,7 +557,7 @@ __device__ double block_sum_f64(double v, double* tmp) {
 // gradient coefficient coef[l][b][e] = f * coef_scale, and the block's part
 // sum_e f * mean score of the loss.
 __global__ __launch_bounds__(256) void seq_loss_finalize_kernel(
-    const float* __restrict__ part_cnt, const float* __restrict__ part_sum, int nchunk, int E,
+    const double* __restrict__ part_cnt, const double* __restrict__ part_sum, int nchunk, int E,
     int64_t S, double f_scale, double coef_scale, double* __restrict__ coef,
     double* __restrict__ part_loss) {
   __shared__ double tmp[17];
@@ -560,12 +565,12 @@ __global__ __launch_bounds__(256) void seq_loss_finalize_kernel(
   double loss = 0.0;
   for (int e = threadIdx.x; e < E; e += 256) {
     double c = 0.0, s = 0.0;
-    const float* pc = part_cnt + lb * nchunk * E + e;
-    const float* ps = part_sum + lb * nchunk * E + e;
+    const double* pc = part_cnt + lb * nchunk * E + e;
+    const double* ps = part_sum + lb * nchunk * E + e;
 #pragma unroll 8
     for (int k = 0; k < nchunk; ++k) {
-      c += (double)pc[(size_t)k * E];
-      s += (double)ps[(size_t)k * E];
+      c += pc[(size_t)k * E];
+      s += ps[(size_t)k * E];
     }
     const double f = c * f_scale;
     coef[lb * E + e] = f * coef_scale;
@@ -593,7 +598,7 @@ __global__ __launch_bounds__(256) void loss_sum_kernel(const double* __restrict_
 // blocks' partials (sums64: [L][2][E]); 64 experts at a time, the 16 waves
 // take the partials in turn and are added in wave order.
 __global__ __launch_bounds__(1024) void switch_layer_sums_kernel(
-    const float* __restrict__ part_cnt, const float* __restrict__ part_sum, int nblk, int E,
+    const double* __restrict__ part_cnt, const double* __restrict__ part_sum, int nblk, int E,
     double* __restrict__ sums64) {
   __shared__ double red[2][16][64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -604,8 +609,8 @@ __global__ __launch_bounds__(1024) void switch_layer_sums_kernel(
     if (e < E)
 #pragma unroll 4
       for (int k = wid; k < nblk; k += 16) {
-        c += (double)part_cnt[base + (size_t)k * E + e];
-        s += (double)part_sum[base + (size_t)k * E + e];
+        c += part_cnt[base + (size_t)k * E + e];
+        s += part_sum[base + (size_t)k * E + e];
       }
     __syncthreads();
     red[0][wid][lane] = c;
@@ -891,7 +896,7 @@ size_t seq_chunks(int64_t S) { return (size_t)((S + kSeqChunk - 1) / kSeqChunk);
 
 // topk_stats of layers, nb blocks each (partials [layer][block][E]).
 void launch_topk_stats(const Layers& layers, int nl, int dtype, const float* token_weights,
-                       int64_t T, int E, int K, int nb, float* pc, float* ps, double* pm,
+                       int64_t T, int E, int K, int nb, double* pc, double* ps, double* pm,
                        hipStream_t st) {
   int G, V;
   group_shape(E, K, G, V);
@@ -917,7 +922,7 @@ void launch_topk_stats(const Layers& layers, int nl, int dtype, const float* tok
 // seq_stats of nl layers, nc chunks of `chunk` tokens per sequence (partials
 // [layer][sequence][chunk][E]).
 void launch_seq_stats(const Layers& layers, int nl, int dtype, int64_t S, int B, int nc, int chunk,
-                      int E, int K, float* pc, float* ps, hipStream_t st) {
+                      int E, int K, double* pc, double* ps, hipStream_t st) {
   int G, V;
   group_shape(E, K, G, V);
   const dim3 grid(nc, B, nl);
@@ -969,10 +974,12 @@ void launch_seq_bwd(const Layers& layers, int nl, bool vec, int dtype, const dou
 int seq_loss_chunk(int L, int64_t S, int B) {
   return (S + 255) / 256 * B * L >= 1024 ? 256 : kSeqChunk;
 }
-// Blocks per layer of the whole-model top-k statistics.
+// Blocks per layer of the whole-model top-k statistics: what fills the chip,
+// and at most 16 tokens per lane group (16 groups or more per block).
 int switch_blocks(int L, int64_t T) {
-  const int nb = stats_blocks(T), most = 2048 / L > 16 ? 2048 / L : 16;
-  return nb < most ? nb : most;
+  const int64_t nb = stats_blocks(T), few = (T + 255) / 256;
+  const int64_t most = 2048 / L > few ? 2048 / L : few;
+  return (int)(nb < most ? nb : most);
 }
 
 }  // namespace
@@ -983,7 +990,7 @@ using namespace moe;
 extern "C" size_t moe_amd_topk_stats_workspace_size(int64_t T, int E) {
   if (T < 0 || E < 1) return 0;
   const size_t nb = (size_t)stats_blocks(T);
-  return align_up(nb * (size_t)E * 2 * sizeof(float), 16) + nb * 2 * sizeof(double);
+  return align_up(nb * (size_t)E * 2 * sizeof(double), 16) + nb * 2 * sizeof(double);
 }
 
 extern "C" int moe_amd_topk_stats(const void* probs, int probs_dtype, const float* token_weights,
@@ -1001,9 +1008,9 @@ extern "C" int moe_amd_topk_stats(const void* probs, int probs_dtype, const floa
   MOE_REQUIRE(((uintptr_t)workspace & 15) == 0, MOE_ERR_ALIGN, "%s: workspace alignment", who);
   hipStream_t st = (hipStream_t)stream;
   const int nb = stats_blocks(T);
-  float* pc = (float*)workspace;
-  float* ps = pc + (size_t)nb * E;
-  double* pm = (double*)((char*)workspace + align_up((size_t)nb * E * 2 * sizeof(float), 16));
+  double* pc = (double*)workspace;
+  double* ps = pc + (size_t)nb * E;
+  double* pm = (double*)((char*)workspace + align_up((size_t)nb * E * 2 * sizeof(double), 16));
   if (T == 0) {
     topk_stats_finalize_kernel<<<E + 1, 64, 0, st>>>(pc, ps, pm, 0, E, counts, prob_sums, margin);
     return check_launch(who);
@@ -1017,7 +1024,7 @@ extern "C" int moe_amd_topk_stats(const void* probs, int probs_dtype, const floa
 
 extern "C" size_t moe_amd_seq_stats_workspace_size(int64_t T, int E, int B) {
   if (T < 0 || E < 1 || B < 1 || T % B) return 0;
-  return (size_t)B * seq_chunks(T / B) * (size_t)E * 2 * sizeof(float);
+  return (size_t)B * seq_chunks(T / B) * (size_t)E * 2 * sizeof(double);
 }
 
 extern "C" int moe_amd_seq_stats(const void* scores, int scores_dtype,
@@ -1039,8 +1046,8 @@ extern "C" int moe_amd_seq_stats(const void* scores, int scores_dtype,
   MOE_REQUIRE(nc < 65536 && B < 65536 && (int64_t)B * E < ((int64_t)1 << 31), MOE_ERR_UNSUPPORTED,
               "%s: grid too large", who);
   hipStream_t st = (hipStream_t)stream;
-  float* pc = (float*)workspace;
-  float* ps = pc + (size_t)B * nc * E;
+  double* pc = (double*)workspace;
+  double* ps = pc + (size_t)B * nc * E;
   Layers layers{};
   layers.in[0] = scores;
   layers.sel[0] = selected;
@@ -1088,7 +1095,7 @@ extern "C" size_t moe_amd_seq_aux_loss_workspace_size(int L, int64_t T, int E, i
   const int64_t S = T / B;
   const int chunk = seq_loss_chunk(L, S, B);
   const size_t parts = (size_t)L * B * (size_t)((S + chunk - 1) / chunk) * E;
-  return align_up(parts * 2 * sizeof(float), 16) + ((size_t)L * B + 1) * sizeof(double);
+  return align_up(parts * 2 * sizeof(double), 16) + ((size_t)L * B + 1) * sizeof(double);
 }
 
 extern "C" int moe_amd_seq_aux_loss(const void* const* scores, const int64_t* const* selected,
@@ -1116,9 +1123,9 @@ extern "C" int moe_amd_seq_aux_loss(const void* const* scores, const int64_t* co
   const int nc = (int)nc64;
   hipStream_t st = (hipStream_t)stream;
   const size_t per_layer = (size_t)B * nc * E;
-  float* pc = (float*)workspace;
-  float* ps = pc + (size_t)L * per_layer;
-  double* parts = (double*)((char*)workspace + align_up((size_t)L * per_layer * 2 * sizeof(float), 16));
+  double* pc = (double*)workspace;
+  double* ps = pc + (size_t)L * per_layer;
+  double* parts = (double*)((char*)workspace + align_up((size_t)L * per_layer * 2 * sizeof(double), 16));
   for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
     const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
     Layers layers{};
@@ -1163,7 +1170,7 @@ extern "C" int moe_amd_seq_aux_loss_backward(const void* const* scores, int L, i
 
 extern "C" size_t moe_amd_switch_aux_loss_workspace_size(int L, int64_t T, int E) {
   if (L < 1 || T < 1 || E < 1) return 0;
-  return align_up((size_t)L * switch_blocks(L, T) * E * 2 * sizeof(float), 16) +
+  return align_up((size_t)L * switch_blocks(L, T) * E * 2 * sizeof(double), 16) +
          (size_t)L * 2 * E * sizeof(double);
 }
 
@@ -1186,9 +1193,9 @@ extern "C" int moe_amd_switch_aux_loss(const void* const* probs, int L, int prob
   hipStream_t st = (hipStream_t)stream;
   const int nb = switch_blocks(L, T);
   const size_t per_layer = (size_t)nb * E;
-  float* pc = (float*)workspace;
-  float* ps = pc + L * per_layer;
-  double* sums = (double*)((char*)workspace + align_up(L * per_layer * 2 * sizeof(float), 16));
+  double* pc = (double*)workspace;
+  double* ps = pc + L * per_layer;
+  double* sums = (double*)((char*)workspace + align_up(L * per_layer * 2 * sizeof(double), 16));
   for (int l0 = 0; l0 < L; l0 += kMaxLayers) {
     const int nl = L - l0 < kMaxLayers ? L - l0 : kMaxLayers;
     Layers layers{};

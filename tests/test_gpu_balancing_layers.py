@@ -7,6 +7,7 @@ terms); bf16 gradients within their rounding, 2^-8."""
 import pytest
 import torch
 
+from moe_amd import _lib, ops
 from moe_amd import balancing as Bal
 from oracle import balancing_oracle as B
 
@@ -97,3 +98,39 @@ def test_layers_of_odd_alignment():
         gin.append(v.requires_grad_(True))
     loss = Bal.seq_load_balancing_loss_func(tuple(gin), E, K)
     _compare(loss, ref, gin, ref_in, torch.float32)
+
+
+def _seq_loss64(p, sel, L, E, K, B):
+    """The fp64 loss of moe_amd_seq_aux_loss on L layers that are all p, without
+    its scale factors: sum over layers, sequences and experts of counts * mean."""
+    T = p.shape[0]
+    n = int(_lib.load().moe_amd_seq_aux_loss_workspace_size(L, T, E, B))
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+    out = torch.empty(L * B * E + 1, device=DEV, dtype=torch.float64)
+    loss = torch.empty((), device=DEV)
+    ops._call("moe_amd_seq_aux_loss", Bal._ptr_array([p] * L), Bal._ptr_array([sel] * L), L, 0, T, E,
+              K, B, 1.0, 1.0, 1.0, ws.data_ptr(), n, out.data_ptr(), out[-1:].data_ptr(),
+              loss.data_ptr(), ops._stream(p))
+    return out[-1].item()
+
+
+@pytest.mark.parametrize("E", [64, 256, 320])  # 8 and 16 lanes per token, a wave per token
+@pytest.mark.parametrize("L", [1, 16, 128])
+def test_sums_are_fp64_beyond_16_tokens(E, L):
+    """Expert 0 gets 1 from every 256th token and 2^-29 from the others, which
+    an fp32 sum that holds a 1 loses.  At most the 15 other tokens of such a
+    token's lane group may be added to it in fp32."""
+    print(f"sums E={E} L={L}", flush=True)
+    T, tiny = 16384, 2.0 ** -29
+    p = torch.zeros(T, E, device=DEV)
+    p[:, 0] = tiny
+    p[::256, 0] = 1.0
+    ones = T // 256
+    want, limit = ones + (T - ones) * tiny, 15 * ones * tiny
+    _, loss = Bal._switch_loss(E, 1, None, None, *[p] * L)  # = E * sums[0] / (L T)
+    assert abs(loss.item() * T / E - want) <= limit
+    assert abs(Bal.topk_stats(p, 1)[1][0].item() - want) <= limit
+    p[:, 1] = 1.0  # row sums of 1 (in fp32)
+    p[::256, 1] = 0.0
+    sel = torch.zeros(T, 1, device=DEV, dtype=torch.int64)
+    assert abs(_seq_loss64(p, sel, L, E, 1, 1) / L - want) <= limit  # counts T times mean
