@@ -647,11 +647,27 @@ __global__ __launch_bounds__(1024) void switch_loss_kernel(
   if (threadIdx.x == 0) *loss = acc * num_experts;
 }
 
+// Sum of one fp64 value per lane over groups of G lanes.
+template <int G>
+__device__ __forceinline__ double group_sum_f64(double v) {
+  group_steps<G>([&](auto c) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const uint32_t lo = dpp_u32<decltype(c)::value>((uint32_t)b);
+    const uint32_t hi = dpp_u32<decltype(c)::value>((uint32_t)(b >> 32));
+    v += __builtin_bit_cast(double, (uint64_t)hi << 32 | lo);
+  });
+  return v;
+}
+
 // Gradient of the sequence-wise loss with G lanes per token (E == G*V), all
 // layers in one launch: block (c, b, l) holds its lanes' coefficients of
 // sequence b in registers and streams tokens [c*chunk, ...) through 16-byte
-// vectors.  The arithmetic of seq_aux_bwd_kernel, sums over the G lanes in
-// the group's butterfly order.
+// vectors.  seq_aux_bwd_kernel's formula, with the inner product <g, s'> and
+// its difference from g in fp64: balanced routing cancels most of g there, and
+// in fp32 the roundings of the products (each on its own, where a lane of the
+// wave-per-row kernel fuses all but its first) were most of the error: 2-norm
+// 4.9e-7 -> 3.4e-7 from 64 bits at E = 128, 9.5e-7 -> 6.1e-7 at 64, in the same
+// time (49 us for 16 layers of 16384 x 128).
 template <int G, int V>
 __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_group_kernel(
     Layers layers, int dtype, const double* __restrict__ coef, const float* __restrict__ grad,
@@ -663,10 +679,10 @@ __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_group_kernel(
   const void* const __restrict__ scores = layers.in[blockIdx.z];
   void* const __restrict__ out = layers.out[blockIdx.z];
   const double up = grad ? (double)*grad : 1.0;
-  float gc[V];
+  double gc[V];
 #pragma unroll
   for (int j = 0; j < V; ++j)
-    gc[j] = (float)(coef[((size_t)blockIdx.z * gridDim.y + b) * E + expert_of<G>(g, j)] * up);
+    gc[j] = coef[((size_t)blockIdx.z * gridDim.y + b) * E + expert_of<G>(g, j)] * up;
   const int64_t s0 = (int64_t)blockIdx.x * chunk;
   const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
   for (int64_t sb = s0 + (int64_t)wid * TPW; sb < s1; sb += kWaves * TPW) {
@@ -676,16 +692,16 @@ __global__ __launch_bounds__(64 * kWaves) void seq_aux_bwd_group_kernel(
     float v[V];
     load_row<G, V>(scores, dtype, t, g, v);
     const float rs = group_sum<G>(tree_sum<V>(v)) + 1e-20f;
-    float pr[V];
+    double dot = 0.0;
 #pragma unroll
-    for (int j = 0; j < V; ++j) pr[j] = gc[j] * (v[j] / rs);
-    const float dot = group_sum<G>(tree_sum<V>(pr));
+    for (int j = 0; j < V; ++j) dot = fma(gc[j], (double)(v[j] / rs), dot);
+    dot = group_sum_f64<G>(dot);
     if (!tok) continue;
 #pragma unroll
     for (int q = 0; q < V / 4; ++q) {
       float d[4];
 #pragma unroll
-      for (int h = 0; h < 4; ++h) d[h] = (gc[4 * q + h] - dot) / rs;
+      for (int h = 0; h < 4; ++h) d[h] = (float)(gc[4 * q + h] - dot) / rs;
       const int64_t at = t * E + (q * G + g) * 4;
       if (dtype == MOE_DTYPE_F32) *(f32x4*)((float*)out + at) = f32x4{d[0], d[1], d[2], d[3]};
       else *(u32x2*)((bf16*)out + at) = u32x2{pack_bf2(d[0], d[1]), pack_bf2(d[2], d[3])};

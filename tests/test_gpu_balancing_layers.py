@@ -134,3 +134,31 @@ def test_sums_are_fp64_beyond_16_tokens(E, L):
     p[::256, 1] = 0.0
     sel = torch.zeros(T, 1, device=DEV, dtype=torch.int64)
     assert abs(_seq_loss64(p, sel, L, E, 1, 1) / L - want) <= limit  # counts T times mean
+
+
+@pytest.mark.parametrize("E,K", [(32, 2), (64, 6), (128, 4), (256, 8)])
+def test_seq_gradient_inner_product_in_fp64(E, K):
+    """2-norm distance of the gradient from 64 bits: that of the formula with
+    fp32 row sums (as a tree) and quotients but an fp64 inner product, within
+    5% for another order of the row sums.  An fp32 inner product is 40% off."""
+    print(f"seq gradient E={E}", flush=True)
+    B_, S, L = 8, 1024, 2
+    g = torch.Generator(device=DEV).manual_seed(E)
+    layers = [torch.sigmoid(torch.randn(B_ * S, E, generator=g, device=DEV)).requires_grad_(True)
+              for _ in range(L)]
+    sel = [p.detach().topk(K, dim=-1).indices for p in layers]
+    Bal.seq_load_balancing_loss_func(tuple(layers), E, K, B_, tuple(sel)).backward()
+    got = emulated = 0.0
+    for p, s in zip(layers, sel):
+        p32, p64 = p.detach(), p.detach().double()
+        f = torch.zeros_like(p64).scatter_(1, s, 1.0).reshape(B_, S, E).sum(1) * (E / (K * S))
+        c = (f / (L * B_ * S)).repeat_interleave(S, dim=0)
+        n64 = p64.sum(-1, keepdim=True) + 1e-20
+        want = (c - (c * p64 / n64).sum(-1, keepdim=True)) / n64
+        n32 = p32
+        while n32.shape[1] > 1:
+            n32 = n32[:, 0::2] + n32[:, 1::2]
+        em = (c - (c * (p32 / n32).double()).sum(-1, keepdim=True)).float() / n32
+        got += float((p.grad.double() - want).square().sum())
+        emulated += float((em.double() - want).square().sum())
+    assert got <= 1.05 ** 2 * emulated
