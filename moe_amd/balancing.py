@@ -109,6 +109,8 @@ class SwitchAuxLoss(torch.autograd.Function):
     @on_tensor_device
     def backward(ctx, g):
         w, coef = ctx.token_weights, ctx.coef
+        if g.dtype == torch.float64:  # fp64 layers: the kernels take an fp32 factor
+            coef, g = _contig(coef * g), torch.ones((), device=coef.device)
         g = _contig(g.to(torch.float32))
         grads: list = [None] * len(ctx.meta)
         for meta in dict.fromkeys(ctx.meta):

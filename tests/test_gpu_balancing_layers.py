@@ -162,3 +162,17 @@ def test_seq_gradient_inner_product_in_fp64(E, K):
         got += float((p.grad.double() - want).square().sum())
         emulated += float((em.double() - want).square().sum())
     assert got <= 1.05 ** 2 * emulated
+
+
+def test_switch_gradient_of_fp64_layers_keeps_fp64_upstream():
+    """An upstream gradient past fp32's range, on layers whose loss is fp64."""
+    layers, _ = _layers((64, 64), 32, torch.float32, 3, softmax=True)
+    grads = []
+    for up in (1.0, 2.0 ** 130):
+        gin = [x.to(DEV, torch.float64).requires_grad_(True) for x in layers]
+        loss = Bal.load_balancing_loss_func(tuple(gin), 32, 4)
+        assert loss.dtype == torch.float64
+        loss.backward(torch.tensor(up, dtype=torch.float64, device=DEV))
+        grads.append([x.grad for x in gin])
+    for a, b in zip(*grads):
+        assert a.abs().max() > 0 and torch.equal(a * 2.0 ** 130, b)
