@@ -164,7 +164,8 @@ int moe_amd_router_softmax_topk_backward(const float* probs, const int64_t* topk
  * num_groups > 0: groups scored by the sum of their top K/group_topk,
  * group_topk groups kept); weights = gathered unbiased scores, divided by
  * (sum + 1e-20) when renormalize, times scaling_factor when > 0, stored in
- * weights_dtype.  Replaces DeepSeekRouter.forward lines 111-152 of
+ * weights_dtype.  scores may be the logits' own buffer.  Replaces
+ * DeepSeekRouter.forward lines 111-152 of
  * src/models/router.py (group_limited_topk: lines 22-70).
  * tokens_per_expert (may be NULL) accumulates the bincount of line 145. */
 int moe_amd_router_sigmoid_topk(const float* logits, const float* expert_bias, int64_t T, int E,

@@ -104,16 +104,26 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void softmax_topk_kernel(
 // scores = sigmoid(logits) stored, then the selection core shared with the
 // fused gating linear (router_group.h: group scores and kept groups when
 // ngroups > 0, each group on one lane; rank keys of the biased scores, the
-// winner's unbiased score taken from its owner lane, weights renormalised by
-// their sum in rank order (+1e-20), scaled), cast.  VEC: E == G*V, fp32 rows
+// winner's unbiased score recomputed from its logit (score_at), weights
+// renormalised by their sum in rank order (+1e-20), scaled), cast.  VEC: E == G*V, fp32 rows
 // moved as 16-byte vectors.  Eight waves per block: every block adds its
 // counts to the same E addresses, about 18 ns each, and four-wave blocks spent
 // 9 to 19 us of 36 to 41 on that (T = 32768, E = 128 and T = 65536, E = 64).
 constexpr int kSigmoidWaves = 8;
+
+// The unbiased score of an entry whose score is already stored: from its
+// logit again, or the stored score itself where scores is the logits' own
+// buffer.  (No __restrict__ on the two in these kernels: the read stays behind
+// the stores, and a wave's vector memory accesses are performed in order.)
+__device__ __forceinline__ float score_at(const float* logits, const float* scores, int64_t i,
+                                          int scores_in) {
+  return dsk_score(logits[i], scores_in || scores == logits);
+}
+
 template <int G, int V, bool VEC>
 __global__ __launch_bounds__(64 * kSigmoidWaves) void sigmoid_topk_group_kernel(
-    const float* __restrict__ logits, const float* __restrict__ bias, int64_t T, int E, int K,
-    int renorm, float scaling, int ngroups, int gtopk, float* __restrict__ scores,
+    const float* logits, const float* __restrict__ bias, int64_t T, int E, int K,
+    int renorm, float scaling, int ngroups, int gtopk, float* scores,
     void* __restrict__ topk_w, int w_dtype, int64_t* __restrict__ topk_idx,
     float* __restrict__ tpe, int scores_in) {
   extern __shared__ int hist[];  // [E] when tpe != nullptr
@@ -170,7 +180,7 @@ __global__ __launch_bounds__(64 * kSigmoidWaves) void sigmoid_topk_group_kernel(
     float my_w;
     int my_e;
     group_sigmoid_topk<G, V>(
-        [&](int e) { return dsk_score(logits[tt * E + e], scores_in); }, key, grp, g, K, ngroups,
+        [&](int e) { return score_at(logits, scores, tt * E + e, scores_in); }, key, grp, g, K, ngroups,
         eg, gtopk, renorm, scaling, scores_in, false, cnt, my_w, my_e);
     if (tok && g < K) {
       if (w_dtype == MOE_DTYPE_BF16)
@@ -325,8 +335,8 @@ int grid_sigmoid(int64_t T, int G) {
 
 template <int NV, bool GROUPS>
 __global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_kernel(
-    const float* __restrict__ logits, const float* __restrict__ bias, int64_t T, int E, int K,
-    int renorm, float scaling, int num_groups, int group_topk, float* __restrict__ scores,
+    const float* logits, const float* __restrict__ bias, int64_t T, int E, int K,
+    int renorm, float scaling, int num_groups, int group_topk, float* scores,
     void* __restrict__ topk_w, int w_dtype, int64_t* __restrict__ topk_idx,
     float* __restrict__ tpe, int scores_in) {
   extern __shared__ int hist[];
@@ -413,7 +423,7 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_kernel(
       }
       ek = wave_topk<NV>(b, taken, lane, K);
     }
-    float wk = lane < K ? dsk_score(logits[t * E + ek], scores_in) : 0.f;
+    float wk = lane < K ? score_at(logits, scores, t * E + ek, scores_in) : 0.f;
     float ssum = 0.f;
     if (renorm)
       for (int k = 0; k < K; ++k)
@@ -448,8 +458,8 @@ __global__ __launch_bounds__(64 * kWavesPerBlock) void sigmoid_topk_kernel(
 // sum in rank order (+1e-20), scaled, cast.  K <= 16.
 template <int SL>
 __global__ __launch_bounds__(256) void sigmoid_topk_split_kernel(
-    const float* __restrict__ logits, const float* __restrict__ bias, int64_t T, int E, int K,
-    int renorm, float scaling, float* __restrict__ scores, void* __restrict__ topk_w,
+    const float* logits, const float* __restrict__ bias, int64_t T, int E, int K,
+    int renorm, float scaling, float* scores, void* __restrict__ topk_w,
     int w_dtype, int64_t* __restrict__ topk_idx, float* __restrict__ tpe, int scores_in) {
   __shared__ uint64_t cand[4 * 16];
   extern __shared__ int hist[];  // [E] when tpe != nullptr
@@ -481,7 +491,7 @@ __global__ __launch_bounds__(256) void sigmoid_topk_split_kernel(
       uint64_t c[1] = {lane < 4 * K ? cand[lane] : 0ull};
       uint64_t kk;
       const int ek = wave_topk_keys<1>(c, lane, K, kk);
-      float wk = lane < K ? dsk_score(lrow[ek], scores_in) : 0.f;
+      float wk = lane < K ? score_at(logits, scores, t * E + ek, scores_in) : 0.f;
       float ssum = 0.f;
       if (renorm)
         for (int k = 0; k < K; ++k)

@@ -53,3 +53,25 @@ def test_grouped_routing(T, E, K, groups, kept):
     v = scores.cpu().double().gather(1, want)
     ref = v / v.sum(-1, keepdim=True) * 2.5
     assert float(((w.cpu().double() - ref).abs() / ref).max()) <= (K + 3) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("T,E,K,groups,kept", [
+    (300, 128, 8, 8, 4), (300, 64, 6, 0, 0), (300, 256, 8, 0, 0),  # lanes per token, vectors
+    (300, 100, 8, 0, 0), (300, 96, 6, 6, 3),                       # ... without vectors
+    (300, 64, 20, 0, 0), (300, 512, 8, 8, 4),                      # a wave per token
+    (300, 320, 8, 0, 0), (300, 1792, 8, 0, 0),                     # a workgroup per token
+])
+def test_scores_in_the_logits_buffer(T, E, K, groups, kept):
+    """scores written over the logits: the same scores, weights and indices."""
+    print(f"scores in place T={T} E={E} K={K} groups={groups}/{kept}", flush=True)
+    g = torch.Generator().manual_seed(T + E + K)
+    logits = torch.randn(T, E, generator=g).to(DEV)
+    bias = ((torch.rand(E, generator=g) * 2 - 1) * 0.05).to(DEV)
+    want = ops.router_sigmoid_topk(logits, bias, K, True, 2.5, groups or None, kept or None)
+    buf, w = logits.clone(), torch.empty(T, K, device=DEV)
+    idx = torch.empty(T, K, device=DEV, dtype=torch.int64)
+    ops._call("moe_amd_router_sigmoid_topk", buf.data_ptr(), bias.data_ptr(), T, E, K, 1, 2.5, groups,
+              kept, buf.data_ptr(), w.data_ptr(), 0, idx.data_ptr(), None, ops._stream(buf))
+    torch.cuda.synchronize()
+    for a, b in zip((buf, w, idx), want):
+        assert torch.equal(a, b)
