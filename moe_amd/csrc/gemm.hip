@@ -1007,7 +1007,7 @@ __device__ __forceinline__ void grouped_gemm(const GemmArgs& p) {
       // the descriptors' extents: loads return 0, stores are dropped.
       constexpr int NIT = 8;  // iterations of 4 rows per row sub-tile
       const int fw = c.ct * BC + ewc * 128;
-      const int nr = c.row_end - c.row0;  // >= 1
+      const int nr = min(c.row_end - c.row0, BR);  // >= 1; the tile's own rows, as in setup()
       const int c8 = (ln & 15) * 8, rq = ln >> 4;
       const bool fok = fw + c8 < I;
       const auto rgu = make_rsrc(p.a1 + (int64_t)c.row0 * I2, (uint32_t)nr * (uint32_t)I2 * 2);

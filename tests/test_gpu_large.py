@@ -85,3 +85,29 @@ def test_dw_expert_rows_beyond_4gib(gemm):
     print(f"  max rel err {err:.2e}", flush=True)
     assert err < 1e-2
     assert not dw[1].any()
+
+
+def test_fused_down_backward_expert_rows_beyond_4gib():
+    """One expert owns 1.4 M rows, 4.3 GB of d_gate_up: the tile whose rows to
+    the expert's end take 2^32 bytes and a few more (rows 1792..2047) must give
+    what those rows give by themselves."""
+    from moe_amd import ops
+    Ts, Hs, Is = 1_400_000, 64, 768
+    r0, r1 = 1792, 2048
+    assert 0 < (Ts - r0) * 2 * Is * 2 - (1 << 32) < (r1 - r0) * 2 * Is * 2
+    print(f"fused down backward past 4 GiB: T={Ts} H={Hs} I={Is}", flush=True)
+    g = torch.Generator(device=DEV).manual_seed(6)
+
+    def rand(*s):
+        return torch.empty(*s, device=DEV, dtype=torch.bfloat16).normal_(generator=g)
+
+    dout, w2, gu = rand(Ts, Hs), rand(1, Hs, Is), rand(Ts, 2 * Is)
+    w = torch.rand(Ts, 1, device=DEV, generator=g)
+    parts = []
+    for a, b in ((0, Ts), (r0, r1)):
+        plan = ops.permute(torch.zeros(b - a, 1, dtype=torch.int64, device=DEV), 1)
+        res = ops.gemm_down_backward_fused(dout[a:b], plan, w2, gu[a:b], w[a:b])
+        parts.append([t[r0 - a:r1 - a].clone() for t in res])
+    torch.cuda.synchronize()
+    for full, own in zip(*parts):
+        assert own.abs().max() > 0 and torch.equal(full, own)
