@@ -98,13 +98,24 @@ def test_compile_fullgraph_matches_eager(layer):
         assert torch.equal(a, b)
 
 
-def test_layer_backward_overlap_matches_in_order():
+def _side_stream_uses(monkeypatch):
+    """Lets every gather backward use the second stream; the list grows by one
+    entry per use."""
+    from moe_amd import library
+    uses, get = [], library._side_stream
+    monkeypatch.setattr(library, "_BESIDE_BYTES", -1)
+    monkeypatch.setattr(library, "_side_stream", lambda device: uses.append(device) or get(device))
+    return uses
+
+
+def test_layer_backward_overlap_matches_in_order(monkeypatch):
     """The softmax layer's backward with the gather backward on a second
     stream (beside the weight-gradient GEMMs) gives the same bits as with
     every kernel in order on one stream (the per-launch timing mode), on
     three steps in a row."""
     from moe_amd import ops
     print("backward overlap vs in order", flush=True)
+    uses = _side_stream_uses(monkeypatch)
     x, wr, w1, w2, _, _, dout = _inputs(T=4096, H=512, E=32, K=4, I=256, seed=7)
     grads = []
     for timed in (True, False, False, False):
@@ -118,15 +129,17 @@ def test_layer_backward_overlap_matches_in_order():
             ops.record_kernel_times(None)
         torch.cuda.synchronize()
         grads.append([t.grad.clone() for t in leaves])
+        assert len(uses) == len(grads) - 1  # the timed run stays in order
     for g in grads[1:]:
         for a, b in zip(grads[0], g):
             assert torch.equal(a, b)
 
 
-def test_experts_backward_overlap_matches_in_order():
+def test_experts_backward_overlap_matches_in_order(monkeypatch):
     """The same for the expert-layer op (the ExpertsInterface path)."""
     from moe_amd import ops
     print("experts backward overlap vs in order", flush=True)
+    uses = _side_stream_uses(monkeypatch)
     x, _, w1, w2, w, idx, dout = _inputs(T=4096, H=512, E=32, K=4, I=256, seed=8)
     grads = []
     for timed in (True, False, False):
@@ -140,6 +153,22 @@ def test_experts_backward_overlap_matches_in_order():
             ops.record_kernel_times(None)
         torch.cuda.synchronize()
         grads.append([t.grad.clone() for t in leaves])
+        assert len(uses) == len(grads) - 1  # the timed run stays in order
     for g in grads[1:]:
         for a, b in zip(grads[0], g):
             assert torch.equal(a, b)
+
+
+def test_gather_backward_stream_by_size(monkeypatch):
+    """Up to _BESIDE_BYTES of row gradients the gather stays in order, past
+    them it takes the second stream."""
+    from moe_amd import library
+    x, _, w1, w2, w, idx, dout = _inputs(T=512, H=512, E=32, K=4, I=256, seed=9)
+    uses = _side_stream_uses(monkeypatch)
+    nbytes = 512 * 4 * 512 * 2
+    for limit, used in ((nbytes, 0), (nbytes - 1, 1)):
+        monkeypatch.setattr(library, "_BESIDE_BYTES", limit)
+        xg = x.detach().clone().requires_grad_(True)
+        experts_forward(xg, idx, w, w1, w2).backward(dout)
+        assert len(uses) == used
+    torch.cuda.synchronize()
