@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from moe_amd import ops
+from moe_amd import _lib, ops
 from oracle import moe_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -101,20 +101,39 @@ FORMS = [(1, 1, 1), (4, 128, 8), (63, 7, 1), (65, 16, 4), (1024, 33, 1), (1025, 
          (16384, 1, 1), (300, 2076, 8), (300, 2077, 8), (5000, 2288, 8), (70000, 3, 1)]
 
 
+def _permute_into(idx, E, fill):
+    """moe_amd_permute into buffers whose bytes are all `fill`."""
+    S, lib = idx.numel(), _lib.load()
+
+    def buf(nbytes, dtype=torch.uint8):
+        return torch.full((max(int(nbytes), 16),), fill, device=DEV, dtype=torch.uint8)[:nbytes].view(dtype)
+
+    ws = buf(lib.moe_amd_permute_workspace_size(S, E))
+    outs = [buf(4 * E, torch.int32), buf(4 * (E + 1), torch.int32), buf(4 * S, torch.int32),
+            buf(4 * S, torch.int32), buf(lib.moe_amd_tile_plan_size(S, E))]
+    ops._call("moe_amd_permute", idx.data_ptr(), S, E, ws.data_ptr(), ws.numel(),
+              *[t.data_ptr() for t in outs], outs[-1].numel(), ops._stream(idx))
+    return outs
+
+
 @pytest.mark.parametrize("T,E,K", FORMS)
 def test_permute_forms(T, E, K):
     print(f"permute form T={T} E={E} K={K}", flush=True)
     idx = _routing(T, E, K, 11 * T + E, skew=1.0, sentinel_every=5 if E > 1 else 0)
     S = T * K
     plan = ops.permute(idx.to(DEV), E)
-    again = ops.permute(idx.to(DEV), E)
+    poisoned = [_permute_into(idx.to(DEV), E, fill) for fill in (0xAA, 0x55)]
     torch.cuda.synchronize()
     ref = O.permute(idx, E)
     for got, want in ((plan.counts, ref.counts), (plan.offsets, ref.offsets),
                       (plan.row_src, ref.row_src), (plan.slot, ref.slot),
                       (plan.tile_starts, ref.tile_starts)):
         assert np.array_equal(got.cpu().numpy(), want)
-    assert torch.equal(plan.tile_plan, again.tile_plan)  # every byte is written
+    # every byte is written, whatever the buffers held
+    for mine in poisoned:
+        for got, want in zip(mine, (plan.counts, plan.offsets, plan.row_src, plan.slot,
+                                    plan.tile_plan)):
+            assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
     raw = plan.tile_plan.cpu().numpy()
     base = (3 * (E + 1) * 4 + 4 + 15) // 16 * 16
     for b, bm in enumerate(O.TILE_SIZES):
