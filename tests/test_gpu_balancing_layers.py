@@ -176,3 +176,49 @@ def test_switch_gradient_of_fp64_layers_keeps_fp64_upstream():
         grads.append([x.grad for x in gin])
     for a, b in zip(*grads):
         assert a.abs().max() > 0 and torch.equal(a * 2.0 ** 130, b)
+
+
+@pytest.mark.parametrize("T,Bz,E,K,given,dtype", [
+    (520, 2, 128, 8, True, torch.float32), (300, 1, 64, 6, False, torch.float32),
+    (260, 4, 256, 8, True, torch.bfloat16), (130, 2, 100, 4, False, torch.float32),
+    (96, 2, 1792, 8, True, torch.float32),
+])
+def test_one_layer_entry_points_match_whole_model_ones(T, Bz, E, K, given, dtype):
+    """moe_amd_seq_stats, moe_amd_seq_aux_backward and moe_amd_switch_aux_backward
+    against the whole-model entry points with one layer: the coefficients (sums
+    of whole numbers) and the gradients bit for bit, the loss to fp64 rounding."""
+    print(f"one layer T={T} B={Bz} E={E} {dtype}", flush=True)
+    (p,), g = _layers((T,), E, dtype, T + E)
+    p, code, lib = p.to(DEV), ops._dtype_code(dtype), _lib.load()
+    sel = torch.rand(T, E, generator=g).topk(K, dim=-1).indices.to(DEV) if given else None
+    st, f64 = ops._stream(p), dict(device=DEV, dtype=torch.float64)
+    sel_ptr = sel.data_ptr() if given else None
+    n = int(lib.moe_amd_seq_stats_workspace_size(T, E, Bz))
+    ws, counts, mean = torch.empty(n, device=DEV, dtype=torch.uint8), torch.empty(Bz, E, **f64), \
+        torch.empty(Bz, E, **f64)
+    ops._call("moe_amd_seq_stats", p.data_ptr(), code, sel_ptr, T, E, K, Bz, ws.data_ptr(), n,
+              counts.data_ptr(), mean.data_ptr(), st)
+    n = int(lib.moe_amd_seq_aux_loss_workspace_size(1, T, E, Bz))
+    ws = torch.empty(n, device=DEV, dtype=torch.uint8)
+    coef, loss64 = torch.empty(Bz, E, **f64), torch.empty((), **f64)
+    loss, up = torch.empty((), device=DEV), torch.ones((), device=DEV)
+    ops._call("moe_amd_seq_aux_loss", Bal._ptr_array([p]), Bal._ptr_array([sel]), 1, code, T, E, K, Bz,
+              0.5, 0.25, 2.0, ws.data_ptr(), n, coef.data_ptr(), loss64.data_ptr(), loss.data_ptr(), st)
+    assert torch.equal(coef, counts * 0.5 * 0.25)
+    want = float((counts * 0.5 * mean).sum() * 2.0)
+    assert abs(loss64.item() - want) <= 1e-13 * want
+    one, all_ = torch.empty_like(p), torch.empty_like(p)
+    ops._call("moe_amd_seq_aux_backward", p.data_ptr(), code, coef.data_ptr(), T, E, Bz, one.data_ptr(),
+              st)
+    ops._call("moe_amd_seq_aux_loss_backward", Bal._ptr_array([p]), 1, code, coef.data_ptr(),
+              up.data_ptr(), T, E, Bz, Bal._ptr_array([all_]), st)
+    assert torch.equal(one, all_) and bool(one.any())
+    w = torch.rand(T, generator=g).to(DEV)
+    for tok_w in (None, w):
+        ptr = tok_w.data_ptr() if tok_w is not None else None
+        ops._call("moe_amd_switch_aux_backward", coef.data_ptr(), ptr, T, E, code, one.data_ptr(), st)
+        ops._call("moe_amd_switch_aux_loss_backward", coef.data_ptr(), up.data_ptr(), ptr, 1, T, E, code,
+                  Bal._ptr_array([all_]), st)
+        assert torch.equal(one, all_)
+        want = coef[0].float()[None] * (tok_w[:, None] if tok_w is not None else 1.0)
+        assert torch.equal(one, want.expand(T, E).to(dtype))
