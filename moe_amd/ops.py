@@ -88,11 +88,17 @@ def _ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# torch's own accessor of a stream's handle, where this torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(t: torch.Tensor) -> int:
     """The current stream's handle on t's device.  A launch costs the host
     about as much as the arguments it is given: torch.cuda.current_stream
-    builds a Stream object for 4 us, this reads the handle."""
-    return torch._C._cuda_getCurrentRawStream(t.device.index)
+    builds a Stream object for 4 us, the accessor only reads the handle."""
+    if _raw_stream is None:
+        return torch.cuda.current_stream(t.device).cuda_stream
+    return _raw_stream(t.device.index)
 
 
 def _dtype_code(dt: torch.dtype) -> int:

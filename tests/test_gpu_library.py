@@ -172,3 +172,14 @@ def test_gather_backward_stream_by_size(monkeypatch):
         experts_forward(xg, idx, w, w1, w2).backward(dout)
         assert len(uses) == used
     torch.cuda.synchronize()
+
+def test_stream_handle(monkeypatch):
+    """The handle of the current stream, with and without torch's accessor."""
+    from moe_amd import ops
+    t = torch.empty(1, device=DEV)
+    side = torch.cuda.Stream()
+    for raw in (ops._raw_stream, None):
+        monkeypatch.setattr(ops, "_raw_stream", raw)
+        assert ops._stream(t) == torch.cuda.current_stream().cuda_stream
+        with torch.cuda.stream(side):
+            assert ops._stream(t) == side.cuda_stream
