@@ -302,15 +302,19 @@ int grid_tokens(int64_t ntok) {
 }
 
 // Combine and gather backward: one wave per token walks the row in pieces of
-// 1 KB, a memory round trip each; while the tokens leave the chip short of
-// waves (256 CUs x 4 SIMDs x 8 = 8192 at once) the pieces go to waves of
-// their own (blockIdx.y).
+// 1 KB, a memory round trip each.  While the tokens leave the chip short of
+// waves the pieces go to waves of their own (blockIdx.y): all of them up to
+// 1024 tokens, two halves of the row up to 8192 where a half is more than one
+// piece.  More than two there, or halves of one piece, read more rows at once
+// for no more bytes and lose: combine of 8 rows, us by waves per token 1 / 2 /
+// 4 (or all), bf16 H = 2048: T = 512 8.9 / 7.8 / 7.7, 1536 12.3 / 9.7 / 10.2,
+// 4096 32.9 / 30.9 / 33.5, 8192 60.3 / 55.7 / 67.5; fp32 H = 2048, T = 4096
+// 70 / 63 / 75; fp32 H = 512 (2 pieces), T = 8192 26.9 / 27.3.
 template <typename T>
 dim3 grid_rows(int64_t ntok, int H) {
   const int pieces = (H + 64 * Vec<T>::N - 1) / (64 * Vec<T>::N);
-  const int64_t ny = ntok > 0 ? 16384 / ntok : 1;
-  return dim3((unsigned)grid_tokens(ntok),
-              (unsigned)(ny < 1 ? 1 : (ny < pieces ? ny : pieces)));
+  const int ny = ntok <= 1024 ? pieces : (ntok <= 8192 && pieces > 2 ? 2 : 1);
+  return dim3((unsigned)grid_tokens(ntok), (unsigned)ny);
 }
 
 int check_rows(int64_t T, int K, int E, int H, int dtype, const char* who) {
