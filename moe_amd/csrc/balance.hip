@@ -57,20 +57,24 @@ int stats_blocks(int64_t T) {
 }
 
 // Combines the four waves' per-lane accumulators of one [E] vector in wave
-// order and writes the block's partial.  `buf` holds kWaves * 64 values.
-template <int NV, typename T>
-__device__ void block_combine(const T (&acc)[NV], int E, double* buf, double* out) {
+// order, in fp64, and writes the block's partial: kWaves entries per lane at a
+// time, one by each wave.
+constexpr int kCombineBuf = kWaves * kWaves * 64;  // floats of `buf`
+template <int NV>
+__device__ void block_combine(const float (&acc)[NV], int E, float* buf, double* out) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
+  for (int j0 = 0; j0 < NV; j0 += kWaves) {
     __syncthreads();
-    buf[wid * 64 + lane] = (double)acc[j];
+#pragma unroll
+    for (int q = 0; q < kWaves && j0 + q < NV; ++q) buf[(q * kWaves + wid) * 64 + lane] = acc[j0 + q];
     __syncthreads();
-    if (wid == 0) {
-      double s = buf[lane];
-      for (int w = 1; w < kWaves; ++w) s += buf[w * 64 + lane];
-      const int e = j * 64 + lane;
-      if (e < E) out[e] = s;
+    const int e = (j0 + wid) * 64 + lane;
+    if (e < E && j0 + wid < NV) {
+      double s = 0.0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) s += (double)buf[(wid * kWaves + w) * 64 + lane];
+      out[e] = s;
     }
   }
 }
@@ -206,13 +210,13 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
     double* __restrict__ part_margin) {
   const void* const __restrict__ probs = layers.in[blockIdx.y];
   const size_t part = (size_t)blockIdx.y * gridDim.x + blockIdx.x;  // this block's partials
-  __shared__ double buf[kWaves * 64];
+  __shared__ float buf[kCombineBuf];
   __shared__ double mbuf[kWaves * 2];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  double cnt[NV], psum[NV];
+  float cnt[NV], psum[NV];
 #pragma unroll
-  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.0;
+  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.f;
   double msum = 0.0;
   float mmin = INFINITY;
   const int64_t nwaves = (int64_t)gridDim.x * kWaves;
@@ -225,7 +229,7 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
       const int e = j * 64 + lane;
       if (e < E) {
         v[j] = load_val(probs, dtype, t * E + e);
-        psum[j] += (double)w * (double)v[j];
+        psum[j] += w * v[j];
       } else {
         v[j] = -INFINITY;
         taken |= 1ull << j;
@@ -243,7 +247,7 @@ __global__ __launch_bounds__(64 * kWaves) void topk_stats_kernel(
     }
 #pragma unroll
     for (int j = 0; j < NV; ++j)
-      if (((taken & ~pad) >> j) & 1ull) cnt[j] += (double)w;
+      if (((taken & ~pad) >> j) & 1ull) cnt[j] += w;
     if (K < E) {  // margin between the k-th and (k+1)-th largest value
       float bv;
       int be;
@@ -454,17 +458,13 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
     double* __restrict__ part_sum) {
   const void* const __restrict__ scores = layers.in[blockIdx.z];
   const int64_t* const __restrict__ selected = layers.sel[blockIdx.z];
-  __shared__ double buf[kWaves * 64];
+  __shared__ float buf[kCombineBuf];
   const int lane = threadIdx.x & 63;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.y, c = blockIdx.x;
-  float cnt[NV];  // whole numbers up to chunk
-  double psum[NV];
+  float cnt[NV], psum[NV];
 #pragma unroll
-  for (int j = 0; j < NV; ++j) {
-    cnt[j] = 0.f;
-    psum[j] = 0.0;
-  }
+  for (int j = 0; j < NV; ++j) cnt[j] = psum[j] = 0.f;
   const int64_t s0 = (int64_t)c * chunk;
   const int64_t s1 = s0 + chunk < S ? s0 + chunk : S;
   for (int64_t st = s0 + wid; st < s1; st += kWaves) {
@@ -483,7 +483,7 @@ __global__ __launch_bounds__(64 * kWaves) void seq_stats_kernel(
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       v[j] = v[j] / rs;
-      psum[j] += (double)v[j];
+      psum[j] += v[j];
     }
     if (selected) {
       for (int k = 0; k < K; ++k) {
@@ -594,33 +594,30 @@ __global__ __launch_bounds__(256) void loss_sum_kernel(const double* __restrict_
   }
 }
 
-// Switch loss, one block per layer: the layer's counts and sums from its
-// blocks' partials (sums64: [L][2][E]); 64 experts at a time, the 16 waves
-// take the partials in turn and are added in wave order.
+// Switch loss, block (l, i): layer l's counts and sums of 64 experts from its
+// blocks' partials (sums64: [L][2][E]); the 16 waves take the partials in turn
+// and are added in wave order.
 __global__ __launch_bounds__(1024) void switch_layer_sums_kernel(
     const double* __restrict__ part_cnt, const double* __restrict__ part_sum, int nblk, int E,
     double* __restrict__ sums64) {
   __shared__ double red[2][16][64];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const size_t base = (size_t)blockIdx.x * nblk * E;
-  for (int e0 = 0; e0 < E; e0 += 64) {
-    const int e = e0 + lane;
-    double c = 0.0, s = 0.0;
-    if (e < E)
+  const int e = blockIdx.y * 64 + lane;
+  double c = 0.0, s = 0.0;
+  if (e < E)
 #pragma unroll 4
-      for (int k = wid; k < nblk; k += 16) {
-        c += part_cnt[base + (size_t)k * E + e];
-        s += part_sum[base + (size_t)k * E + e];
-      }
-    __syncthreads();
-    red[0][wid][lane] = c;
-    red[1][wid][lane] = s;
-    __syncthreads();
-    if (wid < 2 && e < E) {
-      double v = 0.0;
-      for (int w = 0; w < 16; ++w) v += red[wid][w][lane];
-      sums64[((size_t)blockIdx.x * 2 + wid) * E + e] = v;
+    for (int k = wid; k < nblk; k += 16) {
+      c += part_cnt[base + (size_t)k * E + e];
+      s += part_sum[base + (size_t)k * E + e];
     }
+  red[0][wid][lane] = c;
+  red[1][wid][lane] = s;
+  __syncthreads();
+  if (wid < 2 && e < E) {
+    double v = 0.0;
+    for (int w = 0; w < 16; ++w) v += red[wid][w][lane];
+    sums64[((size_t)blockIdx.x * 2 + wid) * E + e] = v;
   }
 }
 
@@ -984,15 +981,22 @@ void launch_seq_bwd(const Layers& layers, int nl, bool vec, int dtype, const dou
 #undef MOE_SEQ_BWD
 }
 
+bool group_lanes(int E, int K) {  // the kernels with G lanes per token
+  int G, V;
+  group_shape(E, K, G, V);
+  return G != 0;
+}
+
 // Tokens per block of the whole-model sequence statistics: 256 (a block's
 // combine costs as much as 100 tokens), 64 while that leaves the chip short of
-// blocks.
-int seq_loss_chunk(int L, int64_t S, int B) {
-  return (S + 255) / 256 * B * L >= 1024 ? 256 : kSeqChunk;
+// blocks, and with a wave per token, which adds its 16 tokens of them in fp32.
+int seq_loss_chunk(int L, int64_t S, int B, int E, int K) {
+  return group_lanes(E, K) && (S + 255) / 256 * B * L >= 1024 ? 256 : kSeqChunk;
 }
 // Blocks per layer of the whole-model top-k statistics: what fills the chip,
 // and at most 16 tokens per lane group (16 groups or more per block).
-int switch_blocks(int L, int64_t T) {
+int switch_blocks(int L, int64_t T, int E, int K) {
+  if (!group_lanes(E, K)) return stats_blocks(T);
   const int64_t nb = stats_blocks(T), few = (T + 255) / 256;
   const int64_t most = 2048 / L > few ? 2048 / L : few;
   return (int)(nb < most ? nb : most);
@@ -1108,9 +1112,7 @@ extern "C" int moe_amd_switch_aux_backward(const double* coef, const float* toke
 
 extern "C" size_t moe_amd_seq_aux_loss_workspace_size(int L, int64_t T, int E, int B) {
   if (L < 1 || T < 1 || E < 1 || B < 1 || T % B) return 0;
-  const int64_t S = T / B;
-  const int chunk = seq_loss_chunk(L, S, B);
-  const size_t parts = (size_t)L * B * (size_t)((S + chunk - 1) / chunk) * E;
+  const size_t parts = (size_t)L * B * seq_chunks(T / B) * E;  // the most, whatever K
   return align_up(parts * 2 * sizeof(double), 16) + ((size_t)L * B + 1) * sizeof(double);
 }
 
@@ -1132,7 +1134,7 @@ extern "C" int moe_amd_seq_aux_loss(const void* const* scores, const int64_t* co
               "%s: workspace of %zu bytes needed", who, need);
   MOE_REQUIRE(((uintptr_t)workspace & 15) == 0, MOE_ERR_ALIGN, "%s: workspace alignment", who);
   const int64_t S = T / B;
-  const int chunk = seq_loss_chunk(L, S, B);
+  const int chunk = seq_loss_chunk(L, S, B, E, K);
   const int64_t nc64 = (S + chunk - 1) / chunk;
   MOE_REQUIRE(nc64 < 65536 && B < 65536 && L < 65536, MOE_ERR_UNSUPPORTED, "%s: grid too large",
               who);
@@ -1186,7 +1188,8 @@ extern "C" int moe_amd_seq_aux_loss_backward(const void* const* scores, int L, i
 
 extern "C" size_t moe_amd_switch_aux_loss_workspace_size(int L, int64_t T, int E) {
   if (L < 1 || T < 1 || E < 1) return 0;
-  return align_up((size_t)L * switch_blocks(L, T) * E * 2 * sizeof(double), 16) +
+  // the most blocks, whatever K
+  return align_up((size_t)L * stats_blocks(T) * E * 2 * sizeof(double), 16) +
          (size_t)L * 2 * E * sizeof(double);
 }
 
@@ -1207,7 +1210,7 @@ extern "C" int moe_amd_switch_aux_loss(const void* const* probs, int L, int prob
               "%s: workspace of %zu bytes needed", who, need);
   MOE_REQUIRE(((uintptr_t)workspace & 15) == 0, MOE_ERR_ALIGN, "%s: workspace alignment", who);
   hipStream_t st = (hipStream_t)stream;
-  const int nb = switch_blocks(L, T);
+  const int nb = switch_blocks(L, T, E, K);
   const size_t per_layer = (size_t)nb * E;
   double* pc = (double*)workspace;
   double* ps = pc + L * per_layer;
@@ -1219,7 +1222,7 @@ extern "C" int moe_amd_switch_aux_loss(const void* const* probs, int L, int prob
     launch_topk_stats(layers, nl, probs_dtype, token_weights, T, E, K, nb, pc + l0 * per_layer,
                       ps + l0 * per_layer, nullptr, st);
   }
-  switch_layer_sums_kernel<<<L, 1024, 0, st>>>(pc, ps, nb, E, sums);
+  switch_layer_sums_kernel<<<dim3(L, (E + 63) / 64), 1024, 0, st>>>(pc, ps, nb, E, sums);
   switch_loss_kernel<<<1, 1024, 0, st>>>(sums, L, E, num_experts, denom, denom_dev, coef, loss);
   return check_launch(who);
 }
