@@ -40,12 +40,12 @@
 // subnormal then lies at the smallest bf16 one, so that no term underflows
 // (without it a value below 2^-110 lost its third term, then its second: 2.2e-6
 // at 2^-116, 5.6e-4 at 2^-124; now 9e-8 down to 2^-128, as at 1).
-// A value that is not finite, or overflows (from 2^112 on, sums from 2^96 on), makes every element it
-// touches non-finite here; a workgroup that finds such an element in its tile
-// computes the tile again with the fp32 MFMA (v_mfma_f32_32x32x2_f32), whose
-// infinities and NaNs are the plain fp32 ones, and takes those elements from
-// it.  The others keep their bits: an element depends on its own row and
-// column only, whatever else is in the tile.
+// A value that is not finite, or overflows (from 2^112 on, sums from 2^96 on),
+// makes every element it touches non-finite here; a workgroup that finds such
+// an element in its tile computes the tile again with the fp32 MFMA
+// (v_mfma_f32_32x32x2_f32), whose infinities and NaNs are the plain fp32 ones,
+// and takes those elements from it.  The others keep their bits: an element
+// depends on its own row and column only, whatever else is in the tile.
 //
 // Workgroup: 256 threads = 4 waves as 2 x 2, a 128 x 128 tile of C, each wave
 // a 64 x 64 block of 2 x 2 MFMA sub-tiles (64 fp32 accumulators per lane for
@@ -374,9 +374,9 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
     load_src(0);
     load_rows(0);
     load_cols(0);
-    // One stage, with the last NP of the eight products (small ones first).
-    auto stage = [&](int s, auto np) {
-      constexpr int NP = decltype(np)::value;
+    // dW of an expert with few rows: eight products (see the head of the file)
+    const bool few = ROW_KM && nk == 1;
+    for (int s = 0; s < nk; ++s) {
       constexpr int TA[8] = {2, 1, 2, 0, 1, 1, 0, 0}, TB[8] = {1, 2, 0, 2, 1, 0, 1, 0};
       // An operand's next loads go out as soon as its registers are free, so
       // they have a barrier, the MFMAs and the other operand's split to land.
@@ -405,8 +405,7 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
             a[t][i] = *(const bf16x8*)(planes + t * kPlane + (fa[i] ^ (kk * 32)));
             b[t][i] = *(const bf16x8*)(planes + t * kPlane + (fb[i] ^ (kk * 32)));
           }
-#pragma unroll
-        for (int t = 8 - NP; t < 8; ++t)
+        auto product = [&](int t) {  // small ones first
 #pragma unroll
           for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -414,14 +413,15 @@ __global__ __launch_bounds__(FNT, 2) void f32_gemm_kernel(FArgs p) {
               f32x16& c = t < 7 ? low[i][j] : acc[i][j];
               c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[TA[t]][i], b[TB[t]][j], c, 0, 0, 0);
             }
+        };
+        if (few) {
+          product(0);
+          product(1);
+        }
+#pragma unroll
+        for (int t = 2; t < 8; ++t) product(t);
       }
       sync_lds();  // the stage is read: the next one may be written
-    };
-    // dW of an expert with few rows: see the head of the file
-    if (ROW_KM && nk == 1) {
-      stage(0, std::integral_constant<int, 8>{});
-    } else {
-      for (int s = 0; s < nk; ++s) stage(s, std::integral_constant<int, 6>{});
     }
     // Non-finite elements: the tile again on the fp32 MFMA (into `low`, which is
     // free by now), from which only they are taken.
