@@ -77,7 +77,7 @@ def hbm_bytes(name: str, cfg, touched: int | None = None) -> float:
         "moe_amd_gemm_down": S * I * b + w2 + S * H * b,
         # d_out rows, down_proj, gate_up, weights in; d_gate_up, act_w, partials out
         "moe_amd_gemm_down_backward_dx_fused": S * H * b + w2 + 2 * S * 2 * I * b + S * I * b
-        + S * 3 * 4,
+        + S * 2 * ((I + 255) // 256) * 4,
         "moe_amd_gemm_down_backward_dw_gathered": S * H * b + S * I * b + w2,
         "moe_amd_gemm_gate_up_backward_dx": S * 2 * I * b + w1 + S * H * b,
         "moe_amd_gemm_gate_up_backward_dw": S * 2 * I * b + S * H * b + w1,
@@ -287,59 +287,59 @@ def copy_calibration(nbytes: int) -> None:
 # in profiles/gemm_hbm_traffic_L.md and profiles/hbm_traffic_retrofit_XS_global_M.md.
 RECORDED_TRAFFIC = {
     "L": {
-        "gemm_gate_up_swiglu": 11724022260,
-        "gemm_down": 4744795525,
-        "gemm_down_backward_dx_fused": 8253627728,
-        "gemm_down_backward_dw_gathered": 4596779959,
-        "gemm_gate_up_backward_dx": 8668277529,
-        "gemm_gate_up_backward_dw": 7097372741,
-        "torch_gating_linear": 289691204,
-        "router_linear_backward_dx": 290595429,
-        "router_linear_backward_dw": 318972910,
-        "combine": 2420153756,
-        "gather_backward": 2686437232,
+        "gemm_gate_up_swiglu": 11293472704,
+        "gemm_down": 4709806688,
+        "gemm_down_backward_dx_fused": 9065983520,
+        "gemm_down_backward_dw_gathered": 4634555456,
+        "gemm_gate_up_backward_dx": 10491491552,
+        "gemm_gate_up_backward_dw": 6967112832,
+        "torch_gating_linear": 289704469,
+        "router_linear_backward_dx": 290575264,
+        "router_linear_backward_dw": 318979904,
+        "combine": 2420268512,
+        "gather_backward": 2686567168,
     },
     "Retrofit": {
-        "gemm_gate_up_swiglu": 4259894233,
-        "gemm_down": 2187627238,
-        "gemm_down_backward_dx_fused": 2953221848,
-        "gemm_down_backward_dw_gathered": 6584539798,
-        "gemm_gate_up_backward_dx": 4160436454,
-        "gemm_gate_up_backward_dw": 12601085429,
-        "gemm_down_backward_dw_gathered_accumulate": 3221565168,
-        "gemm_gate_up_backward_dw_accumulate": 5932094247,
-        "combine": 605117922,
-        "gather_backward": 604582303,
-        "router_sigmoid_topk": 236798958,
-        "router_sigmoid_topk_backward": 236630583,
+        "gemm_gate_up_swiglu": 4802389152,
+        "gemm_down": 2246650016,
+        "gemm_down_backward_dx_fused": 3888917376,
+        "gemm_down_backward_dw_gathered": 6582089992,
+        "gemm_gate_up_backward_dx": 4919799520,
+        "gemm_gate_up_backward_dw": 12603711784,
+        "gemm_down_backward_dw_gathered_accumulate": 3221776576,
+        "gemm_gate_up_backward_dw_accumulate": 5929264680,
+        "combine": 605151904,
+        "gather_backward": 604600128,
+        "router_sigmoid_topk": 236800448,
+        "router_sigmoid_topk_backward": 236651456,
     },
     "XS global": {
-        "gemm_gate_up_swiglu": 988172263,
-        "gemm_down": 485318597,
-        "gemm_down_backward_dx_fused": 915755323,
-        "gemm_down_backward_dw_gathered": 460877930,
-        "gemm_gate_up_backward_dx": 841622096,
-        "gemm_gate_up_backward_dw": 765743919,
-        "gemm_down_backward_dw_gathered_accumulate": 667508511,
-        "gemm_gate_up_backward_dw_accumulate": 1205827387,
-        "torch_gating_linear": 40041486,
-        "router_linear_backward_dx": 40104928,
-        "router_linear_backward_dw": 71518478,
-        "combine": 168878452,
-        "gather_backward": 201893637,
+        "gemm_gate_up_swiglu": 1040439584,
+        "gemm_down": 490224864,
+        "gemm_down_backward_dx_fused": 1047681984,
+        "gemm_down_backward_dw_gathered": 460724224,
+        "gemm_gate_up_backward_dx": 897604800,
+        "gemm_gate_up_backward_dw": 766615392,
+        "gemm_down_backward_dw_gathered_accumulate": 667535008,
+        "gemm_gate_up_backward_dw_accumulate": 1205840864,
+        "torch_gating_linear": 40043861,
+        "router_linear_backward_dx": 40080800,
+        "router_linear_backward_dw": 71515904,
+        "combine": 168881984,
+        "gather_backward": 201899968,
     },
     "M standard": {
-        "gemm_gate_up_swiglu": 5058396448,
-        "gemm_down": 2587789420,
-        "gemm_down_backward_dx_fused": 3937119063,
-        "gemm_down_backward_dw_gathered": 2680022403,
-        "gemm_gate_up_backward_dx": 4894430789,
-        "gemm_gate_up_backward_dw": 4329990543,
-        "torch_gating_linear": 147097438,
-        "router_linear_backward_dx": 147560983,
-        "router_linear_backward_dw": 176374337,
-        "combine": 1210121163,
-        "gather_backward": 1343266837,
+        "gemm_gate_up_swiglu": 6173746880,
+        "gemm_down": 2571860816,
+        "gemm_down_backward_dx_fused": 4971609528,
+        "gemm_down_backward_dw_gathered": 2649972040,
+        "gemm_gate_up_backward_dx": 5749901088,
+        "gemm_gate_up_backward_dw": 4346097536,
+        "torch_gating_linear": 147008362,
+        "router_linear_backward_dx": 147558112,
+        "router_linear_backward_dw": 176373440,
+        "combine": 1210173216,
+        "gather_backward": 1343312416,
     },
 }
 

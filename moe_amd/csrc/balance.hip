@@ -596,7 +596,8 @@ __global__ __launch_bounds__(256) void loss_sum_kernel(const double* __restrict_
 
 // Switch loss, block (l, i): layer l's counts and sums of 64 experts from its
 // blocks' partials (sums64: [L][2][E]); the 16 waves take the partials in turn
-// and are added in wave order.
+// and are added in wave order.  (One block per layer read a wide layer's
+// partials alone: 16384 x 1792 with gradients 672 us, now 446.)
 __global__ __launch_bounds__(1024) void switch_layer_sums_kernel(
     const double* __restrict__ part_cnt, const double* __restrict__ part_sum, int nblk, int E,
     double* __restrict__ sums64) {

@@ -1781,7 +1781,11 @@ __global__ __launch_bounds__(kWaves<BR> * 64, 1) void grouped_gemm_kernel(GemmAr
 
 // A token-grouped GEMM whose row-tile height the permutation chose: one
 // launch holds all three (a launch per height, of which two return at once,
-// cost 2-5 us for each of those two).
+// cost 2-5 us for each of those two).  The 256-row body is as fast in it as in
+// a kernel of its own, though the three bodies' scalar spills share one
+// register plan: 511 rows in each of 128 experts here and 512 there, H = 2048,
+// G1F 407 / 400, G2F 213 / 218, G1DX 371 / 374, G2DXF 276 / 270 us; reading the
+// arguments anew in each branch (fewer spills) measured the same.
 template <int MODE>
 __global__ __launch_bounds__(kWaves<256> * 64, 1) void token_gemm_kernel(GemmArgs p) {
   const int b = __builtin_amdgcn_readfirstlane(*p.row_tile);

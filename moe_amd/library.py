@@ -133,8 +133,10 @@ def _side_stream(device: torch.device) -> torch.cuda.Stream:
 
 # d_xs bytes up to which the gather backward stays on the current stream.  It
 # then takes less than the events and the stream switch cost: expert layer
-# forward + backward beside / in order 298 / 184 us at 9 MB of d_xs, 530 / 513
-# at 17, 640 / 619 at 34, 897 / 886 at 67, 1526 / 1524 at 134, 2255 / 2278 at 268.
+# forward + backward beside / in order 460 / 320 us at 9 MB of d_xs, 440 / 322 at
+# 17, 427 / 319 at 34 (host-bound: the host's share varies by a third from box to
+# box), 858 / 843 at 67, 1237 / 1226 at 134 (64 experts), 1520 / 1516 (128), 2032 /
+# 2032 and 2283 / 2287 at 268.
 _BESIDE_BYTES = 128 << 20
 
 
@@ -142,7 +144,7 @@ def _gather_backward_beside(d_xs: Tensor, plan, addend: Optional[Tensor]):
     """d_x = gather_backward(d_xs, plan, addend) launched on a second stream,
     after the current stream's work so far, so that it (HBM-bound, no LDS)
     runs beside the weight-gradient GEMMs the caller launches next (MFMA-
-    bound, one workgroup per CU holding all of its LDS and 376-380 of each
+    bound, one workgroup per CU holding all of its LDS and 408-420 of each
     SIMD's 512 VGPRs per lane; the gather needs no LDS and at most 62 VGPRs, so
     its waves share those CUs).  Returns (d_x, join): join() makes the current
     stream wait for it.  With per-launch timing on, or for a small d_xs, it runs
