@@ -24,8 +24,9 @@
 //                   one launch (train.py:79-139)
 //
 // Every sum is deterministic: a lane accumulates the experts it owns in
-// registers, the waves of a block are combined in wave order, and the block
-// partials are reduced in block order (in fp64).  No float atomics.
+// registers (fp32, at most 16 tokens while the grid may grow), the lane groups
+// and waves of a block are combined in order and the block partials in block
+// order, both in fp64.  No float atomics.
 #include "common.h"
 #include "wave_topk.h"
 

@@ -217,7 +217,7 @@ def test_f32_gemms_nonfinite(bad):
     assert torch.equal(y[torch.isinf(y)] > 0, want[torch.isinf(y)] > 0)
     mags = act.double().abs() @ w2[0].double().abs().T
     err = (y.double() - want).abs()[fin]
-    # the fp32 MFMA that recomputes these tiles: one rounding per two products
+    # elements taken from the fp32 MFMA: one rounding per two products
     assert bool((err <= max(_bound(I), I * 2.0 ** -24) * mags[fin]).all())
 
 
